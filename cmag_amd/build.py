@@ -30,6 +30,7 @@ SOURCES = [
     "system.cpp",
     "grid.hip",
     "sort.hip",
+    "cellsort.hip",
     "sph.hip",
     "integrate.hip",
     "batch.hip",

@@ -6,14 +6,13 @@
 // share one arena: instance k owns particles [part0, part1) and cell keys
 // [cell0, cell0 + its cell count).  One step of all instances is
 //
-//   prologue   per-instance time state on the device (PeristalsisSystem.cpp:
+//   hash       global key = cell0 + local cell hash, counted per cell; the
+//              boundary configuration of Peristalsis walls is fused in front of it
+//   offsets    compact offsets and cell ranges over all cells, and the
+//              per-instance time state one step on (PeristalsisSystem.cpp:
 //              330-343 for the moving walls), so the step needs no host input
-//   hash       global key = cell0 + local cell hash; the boundary
-//              configuration of Peristalsis walls is fused in front of it
-//   sort       one stable radix sort of every instance's keys: instance k's
-//              particles stay in [part0, part1), ordered as its own sort orders
-//              them
-//   reorder    one gather + cell ranges + compact offsets over all cells
+//   place,     every instance's particles into cell order: instance k's stay in
+//   reorder    [part0, part1), ordered as its own sort orders them
 //   density, force, integrate
 //              persistent kernels over a table of (instance, first particle)
 //              tiles; a workgroup runs one contiguous chunk of tiles and reads
@@ -31,6 +30,7 @@
 #include <new>
 #include <vector>
 
+#include "cellsort_device.hpp"
 #include "common.hpp"
 #include "integrate_device.hpp"
 #include "kernels.hpp"
@@ -52,40 +52,41 @@ __device__ __forceinline__ void tile_chunk(uint32_t num_tiles, uint32_t& t0, uin
     t1 = min(num_tiles, t0 + per);
 }
 
-// PeristalsisSystem::Update's state machine (PeristalsisSystem.cpp:330-343),
-// one thread per instance; other systems only advance their clock
-__global__ __launch_bounds__(64) void batch_prologue_kernel(const cmag_params* __restrict__ params,
-                                                            StepState* __restrict__ state, uint32_t m) {
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= m) return;
-    StepState s = state[k];
-    advance_step_state(params[k], s);
-    state[k] = s;
-}
-
+// keys and counts, as hash_count_kernel makes them for one system; each
+// instance's time record is advanced by the offset kernel that follows, so
+// this one works from an advanced copy
 __global__ __launch_bounds__(256) void batch_hash_kernel(const cmag_params* __restrict__ params,
                                                          const BatchInst* __restrict__ inst,
                                                          const StepState* __restrict__ state,
                                                          const uint2* __restrict__ tiles, uint32_t num_tiles,
-                                                         float4* __restrict__ pos, uint32_t* __restrict__ hash,
-                                                         uint32_t* __restrict__ index) {
+                                                         float4* __restrict__ pos, uint32_t* __restrict__ key,
+                                                         uint32_t* __restrict__ place,
+                                                         uint32_t* __restrict__ cell_count) {
     uint32_t t0, t1;
     tile_chunk(num_tiles, t0, t1);
     for (uint32_t t = t0; t < t1; ++t) {
         const uint2 tile = tiles[t];
         const BatchInst I = inst[tile.x];
         const uint32_t i = tile.y + threadIdx.x;
-        if (i >= I.part1) continue;
-        const cmag_params& P = params[tile.x];
-        float4 p = pos[i];
-        if (P.system == CMAG_SYS_PERISTALSIS && state[tile.x].configure_now && (p.w > 0.0f || p.w < 0.0f)) {
-            // configureBoundaryD, PeristalsisKernel.cu:144-171
-            p = make_float4(p.x, wall_y(P, p.x, p.w, state[tile.x].configure_height, 0.0f), p.z, p.w);
-            pos[i] = p;
+        const bool valid = i < I.part1;
+        uint32_t k = 0;
+        if (valid) {
+            const cmag_params& P = params[tile.x];
+            float4 p = pos[i];
+            if (P.system == CMAG_SYS_PERISTALSIS && (p.w > 0.0f || p.w < 0.0f)) {
+                // configureBoundaryD, PeristalsisKernel.cu:144-171
+                StepState st = state[tile.x];
+                advance_step_state(P, st);
+                if (st.configure_now) {
+                    p = make_float4(p.x, wall_y(P, p.x, p.w, st.configure_height, 0.0f), p.z, p.w);
+                    pos[i] = p;
+                }
+            }
+            const Cell c = grid_pos(P, p.x, p.y, p.z);
+            k = I.cell0 + grid_hash(P, c.x, c.y, c.z);
+            key[i] = k;
         }
-        const Cell c = grid_pos(P, p.x, p.y, p.z);
-        hash[i] = I.cell0 + grid_hash(P, c.x, c.y, c.z);
-        index[i] = i;
+        count_particle(cell_count, place, i, k, 0u, valid);
     }
 }
 
@@ -182,7 +183,7 @@ struct cmag_batch {
     std::vector<cmag_params> P;
     std::vector<BatchInst> I;
     uint32_t m = 0, n = 0, totalCells = 0;
-    int key_bits = 0, dim = 2, hash_order = CMAG_HASH_LINEAR;
+    int dim = 2, hash_order = CMAG_HASH_LINEAR;
     int num_cus = 256;
     cmag_batch_tuning tune{256u, (uint32_t)NB_CAP, 0u, 10u};
     hipStream_t stream = nullptr;
@@ -195,10 +196,9 @@ struct cmag_batch {
 
     float *pos = nullptr, *vel = nullptr, *velLF = nullptr, *acc = nullptr, *presF = nullptr;
     float *measures = nullptr, *sortedPos = nullptr, *sortedVel = nullptr;
-    uint32_t *hash = nullptr, *index = nullptr, *hashAlt = nullptr, *indexAlt = nullptr;
-    uint32_t *cellStart = nullptr, *cellEnd = nullptr, *cellFirst = nullptr, *scanWs = nullptr;
-    void* sortWs = nullptr;
-    size_t sortWsBytes = 0;
+    uint32_t *hash = nullptr, *index = nullptr;
+    uint32_t *cellStart = nullptr, *cellEnd = nullptr, *cellFirst = nullptr;
+    CellSort sort;
 
     hipGraphExec_t graph = nullptr;
     uint32_t graph_steps = 0;
@@ -214,9 +214,10 @@ struct cmag_batch {
         for (hipEvent_t e : ev)
             if (e) (void)hipEventDestroy(e);
         void* bufs[] = {dP, dI, dS, dTiles, pos, vel, velLF, acc, presF, measures, sortedPos, sortedVel,
-                        hash, index, hashAlt, indexAlt, cellStart, cellEnd, cellFirst, scanWs, sortWs};
+                        hash, index, cellStart, cellEnd, cellFirst};
         for (void* b : bufs)
             if (b) (void)hipFree(b);
+        sort.release();
         if (stream) (void)hipStreamDestroy(stream);
     }
 
@@ -232,7 +233,7 @@ struct cmag_batch {
             CMAG_HIP_TRY(hipMalloc((void**)b, f4));
             CMAG_HIP_TRY(hipMemsetAsync(*b, 0, f4, stream));
         }
-        uint32_t** ub[] = {&hash, &index, &hashAlt, &indexAlt};
+        uint32_t** ub[] = {&hash, &index};
         for (uint32_t** b : ub) {
             CMAG_HIP_TRY(hipMalloc((void**)b, u));
             CMAG_HIP_TRY(hipMemsetAsync(*b, 0, u, stream));
@@ -240,9 +241,7 @@ struct cmag_batch {
         CMAG_HIP_TRY(hipMalloc((void**)&cellStart, sizeof(uint32_t) * (size_t)totalCells));
         CMAG_HIP_TRY(hipMalloc((void**)&cellEnd, sizeof(uint32_t) * (size_t)totalCells));
         CMAG_HIP_TRY(hipMalloc((void**)&cellFirst, sizeof(uint32_t) * ((size_t)totalCells + 1)));
-        CMAG_HIP_TRY(hipMalloc((void**)&scanWs, sizeof(uint32_t) * (scan_levels_words(totalCells) + 1)));
-        sortWsBytes = radix_sort_workspace_bytes(n);
-        CMAG_HIP_TRY(hipMalloc(&sortWs, sortWsBytes));
+        CMAG_TRY(sort.alloc(totalCells, n, stream));
         CMAG_HIP_TRY(hipMalloc((void**)&dP, sizeof(cmag_params) * m));
         CMAG_HIP_TRY(hipMalloc((void**)&dI, sizeof(BatchInst) * m));
         CMAG_HIP_TRY(hipMalloc((void**)&dS, sizeof(StepState) * m));
@@ -331,30 +330,15 @@ struct cmag_batch {
     int enqueue_step() {
         if (n == 0) return CMAG_OK;
         const dim3 g(grid_blocks()), b(tune.block);
-        const int passes = (key_bits + 7) / 8;
-        const bool odd = passes % 2 == 1;
-        uint32_t* hk = odd ? hashAlt : hash;
-        uint32_t* hv = odd ? indexAlt : index;
         CMAG_TRY(mark(CMAG_STAGE_HASH));
-        hipLaunchKernelGGL(batch_prologue_kernel, dim3(div_up(m, 64)), dim3(64), 0, stream, dP, dS, m);
-        CMAG_TRY(check_launch("batch_prologue_kernel"));
+        CMAG_TRY(sort.begin(stream));
         hipLaunchKernelGGL(batch_hash_kernel, g, b, 0, stream, dP, dI, dS, dTiles, numTiles,
-                           reinterpret_cast<float4*>(pos), hk, hv);
+                           reinterpret_cast<float4*>(pos), sort.key, sort.place, sort.cell_count);
         CMAG_TRY(check_launch("batch_hash_kernel"));
         CMAG_TRY(mark(CMAG_STAGE_SORT));
-        bool in_alt = false;
-        CMAG_TRY(radix_sort_pairs(hk, hv, odd ? hash : hashAlt, odd ? index : indexAlt, n, key_bits, sortWs,
-                                  sortWsBytes, &in_alt, stream));
-        const bool moved = n >= 2 && key_bits > 0;
-        if (moved && in_alt != odd) return fail(CMAG_E_STATE, "radix sort ended in an unexpected buffer");
-        if (!moved && odd) {
-            CMAG_TRY(launch_copy_u32(hash, hk, n, stream));
-            CMAG_TRY(launch_copy_u32(index, hv, n, stream));
-        }
+        CMAG_TRY(sort.offsets(cellFirst, cellStart, false, dP, P[0], dS, m, stream));
         CMAG_TRY(mark(CMAG_STAGE_REORDER));
-        CMAG_TRY(launch_reorder(cellStart, cellEnd, sortedPos, sortedVel, hash, index, pos, velLF, n, totalCells,
-                                stream));
-        CMAG_TRY(launch_cell_offsets(cellStart, cellEnd, cellFirst, totalCells, n, scanWs, stream));
+        CMAG_TRY(sort.reorder(pos, velLF, cellFirst, hash, index, cellEnd, sortedPos, sortedVel, nullptr, stream));
         CMAG_TRY(mark(CMAG_STAGE_DENSITY));
         if (dim == 3) {
             if (hash_order == CMAG_HASH_MORTON) CMAG_TRY((launch_passes<3, 1>(g, b)));
@@ -416,6 +400,7 @@ struct cmag_batch {
         const uint32_t S = std::max(1u, tune.steps_per_graph);
         if (steps >= S) {
             if (graph_steps != S) CMAG_TRY(build_graph(S));
+            CMAG_TRY(sort.ready(stream));
             for (uint32_t k = 0; k + S <= steps; k += S) CMAG_HIP_TRY(hipGraphLaunch(graph, stream));
         }
         for (uint32_t k = 0; k < steps % S; ++k) CMAG_TRY(update());
@@ -538,9 +523,6 @@ int cmag_batch_create(const cmag_params* params, const uint32_t* counts, uint32_
         p0 += counts[k];
         c0 += c;
     }
-    int bits = 0;
-    while (bits < 32 && ((uint64_t)1 << bits) < cells) ++bits;
-    b->key_bits = bits;
     int rc = b->alloc();
     if (rc != CMAG_OK) {
         delete b;

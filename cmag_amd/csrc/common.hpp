@@ -42,6 +42,17 @@ struct Cell {
     int x, y, z;
 };
 
+// Workgroups are dispatched round-robin over the 8 XCDs (each with its own
+// L2).  Renumbering them so XCD k runs one contiguous block range keeps the
+// neighbour particles a workgroup reads in the L2 of the XCD that reads them.
+__device__ __forceinline__ uint32_t xcd_block() {
+    constexpr uint32_t XCDS = 8;
+    const uint32_t nb = gridDim.x, b = blockIdx.x;
+    const uint32_t k = b % XCDS, slot = b / XCDS;
+    const uint32_t base = nb / XCDS, extra = nb % XCDS;
+    return k * base + min(k, extra) + slot;
+}
+
 // calcGridPos (fluid_kernel.cu:19-25, poiseuilleFlowKernel.cu:18-24): the hash is
 // bit-exact only with IEEE division and no contraction, which this function keeps.
 __device__ __forceinline__ Cell grid_pos(const cmag_params& P, float x, float y, float z) {

@@ -5,7 +5,9 @@
 //                     its launcher, fluidSystem.cu:164)
 // The reference staged the previous hash through shared memory; on CDNA4 the
 // previous key is a plain coalesced load that hits the same cache line, and
-// the gather of pos/velLeapFrog is a float4 (16 B) load per particle.
+// the gather of pos/velLeapFrog is a float4 (16 B) load per particle.  These
+// serve callers of the stage launchers; a System or batch sorts by counting
+// (cellsort.hip).
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -63,9 +65,6 @@ int launch_calc_hash(const cmag_params& P, const float* pos4, uint32_t* hash, ui
 // Run heads of the sorted keys mark cellStart; the element before a head ends
 // the previous cell; the last element ends its cell.  Gathers pos and the
 // leapfrog velocity into sorted order.
-// BUCKET: also the sub-cell bucket of every sorted row (DamBreak: fluid
-// eighth 0..7 of the cell along x, walls 8), one byte per row
-template <bool BUCKET>
 __global__ __launch_bounds__(256) void reorder_kernel(uint32_t* __restrict__ cellStart,
                                                        uint32_t* __restrict__ cellEnd,
                                                        float4* __restrict__ sortedPos,
@@ -74,8 +73,7 @@ __global__ __launch_bounds__(256) void reorder_kernel(uint32_t* __restrict__ cel
                                                        const uint32_t* __restrict__ index,
                                                        const float4* __restrict__ oldPos,
                                                        const float4* __restrict__ oldVel,
-                                                       uint32_t n, uint32_t numCells, const cmag_params P,
-                                                       uint8_t* __restrict__ bucket) {
+                                                       uint32_t n, uint32_t numCells) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     uint32_t h = hash[i];
@@ -93,44 +91,21 @@ __global__ __launch_bounds__(256) void reorder_kernel(uint32_t* __restrict__ cel
     if (i == n - 1 && h < numCells) cellEnd[h] = n;
     const uint32_t k = index[i];
     if (k < n) {  // a valid permutation always passes; anything else is skipped
-        const float4 p = oldPos[k];
-        sortedPos[i] = p;
+        sortedPos[i] = oldPos[k];
         sortedVel[i] = oldVel[k];
-        if (BUCKET) bucket[i] = (uint8_t)(p.w != CMAG_DB_FLUID ? X_SUBS : x_sub(P, p.x));
     }
 }
 
 int launch_reorder(uint32_t* cellStart, uint32_t* cellEnd, float* sortedPos, float* sortedVel,
                    const uint32_t* hash, const uint32_t* index, const float* oldPos,
-                   const float* oldVel, uint32_t n, uint32_t numCells, hipStream_t s, const cmag_params* P,
-                   uint8_t* bucket) {
+                   const float* oldVel, uint32_t n, uint32_t numCells, hipStream_t s) {
     CMAG_TRY(launch_fill_u32(cellStart, CMAG_CELL_EMPTY, numCells, s));
     if (n == 0) return CMAG_OK;
     auto f4 = [](float* q) { return reinterpret_cast<float4*>(q); };
     auto c4 = [](const float* q) { return reinterpret_cast<const float4*>(q); };
-    if (bucket) {
-        if (!P) return fail(CMAG_E_INVALID, "reorder: the buckets need the parameter block");
-        hipLaunchKernelGGL(reorder_kernel<true>, dim3(div_up(n, 256)), dim3(256), 0, s, cellStart, cellEnd,
-                           f4(sortedPos), f4(sortedVel), hash, index, c4(oldPos), c4(oldVel), n, numCells, *P,
-                           bucket);
-    } else {
-        hipLaunchKernelGGL(reorder_kernel<false>, dim3(div_up(n, 256)), dim3(256), 0, s, cellStart, cellEnd,
-                           f4(sortedPos), f4(sortedVel), hash, index, c4(oldPos), c4(oldVel), n, numCells,
-                           cmag_params{}, nullptr);
-    }
+    hipLaunchKernelGGL(reorder_kernel, dim3(div_up(n, 256)), dim3(256), 0, s, cellStart, cellEnd, f4(sortedPos),
+                       f4(sortedVel), hash, index, c4(oldPos), c4(oldVel), n, numCells);
     return check_launch("reorder_kernel");
-}
-
-__global__ void set_word_kernel(uint32_t* p, uint32_t v) { *p = v; }
-
-// compact cell offsets for the neighbour walkers: a run of cells with
-// consecutive keys is then one range [first[k0], first[k1 + 1]) without
-// any empty-cell test
-int launch_cell_offsets(const uint32_t* cellStart, const uint32_t* cellEnd, uint32_t* first,
-                        uint32_t numCells, uint32_t n, uint32_t* ws, hipStream_t s) {
-    CMAG_TRY(exclusive_scan_cell_counts(cellStart, cellEnd, first, numCells, ws, s));
-    hipLaunchKernelGGL(set_word_kernel, dim3(1), dim3(1), 0, s, first + numCells, n);
-    return check_launch("set_word_kernel");
 }
 
 }  // namespace cmag

@@ -60,38 +60,6 @@ int launch_configure_boundary(const cmag_params& P, float* pos, float wave_heigh
     return check_launch("configure_boundary_kernel");
 }
 
-__global__ __launch_bounds__(64) void step_prologue_kernel(const cmag_params P, StepState* __restrict__ state) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    StepState st = *state;
-    advance_step_state(P, st);
-    *state = st;
-}
-
-int launch_step_prologue(const cmag_params& P, StepState* state, hipStream_t s) {
-    hipLaunchKernelGGL(step_prologue_kernel, dim3(1), dim3(64), 0, s, P, state);
-    return check_launch("step_prologue_kernel");
-}
-
-// configureBoundaryD (PeristalsisKernel.cu:144-171) when this step's state
-// record asks for it; a no-op step otherwise
-__global__ __launch_bounds__(256) void configure_boundary_state_kernel(const cmag_params P, float4* __restrict__ pos,
-                                                                        const StepState* __restrict__ st,
-                                                                        uint32_t n) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || !st->configure_now) return;
-    const float4 p = pos[i];
-    if (p.w > 0.0f || p.w < 0.0f)
-        pos[i] = make_float4(p.x, wall_y(P, p.x, p.w, st->configure_height, 0.0f), p.z, p.w);
-}
-
-int launch_configure_boundary_from_state(const cmag_params& P, float* pos, const StepState* state, uint32_t n,
-                                         hipStream_t s) {
-    if (n == 0) return CMAG_OK;
-    hipLaunchKernelGGL(configure_boundary_state_kernel, dim3(div_up(n, 256)), dim3(256), 0, s, P,
-                       reinterpret_cast<float4*>(pos), state, n);
-    return check_launch("configure_boundary_state_kernel");
-}
-
 template <bool REMOVE>
 __global__ __launch_bounds__(256) void right_boundary_kernel(const cmag_params P, float4* __restrict__ pos,
                                                               uint32_t n) {

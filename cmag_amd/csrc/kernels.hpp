@@ -7,7 +7,7 @@
 #include <cstddef>
 #include <cstdint>
 
-#include "cmag_params.h"
+#include "cmag_hip.h"
 
 namespace cmag {
 
@@ -19,24 +19,54 @@ int launch_fill_colors(const cmag_params& P, const float* pos4, float* color4, u
 int launch_copy_u32(uint32_t* dst, const uint32_t* src, size_t n, hipStream_t s);
 int launch_calc_hash(const cmag_params& P, const float* pos4, uint32_t* hash, uint32_t* index,
                      uint32_t n, hipStream_t s);
-// with bucket (and P): also the sub-cell bucket byte of every sorted row
 int launch_reorder(uint32_t* cellStart, uint32_t* cellEnd, float* sortedPos, float* sortedVel,
                    const uint32_t* hash, const uint32_t* index, const float* oldPos,
-                   const float* oldVel, uint32_t n, uint32_t numCells, hipStream_t s,
-                   const cmag_params* P = nullptr, uint8_t* bucket = nullptr);
+                   const float* oldVel, uint32_t n, uint32_t numCells, hipStream_t s);
 
 // out = exclusive_scan(in) (in place allowed); ws holds scan_levels_words(len) words
 size_t scan_levels_words(size_t len);
 int exclusive_scan_u32(const uint32_t* in, uint32_t* out, size_t len, uint32_t* ws, hipStream_t s);
-// out = exclusive_scan of the cell counts (cellEnd - cellStart, 0 for an
-// empty cell) without materialising them; ws as above
-int exclusive_scan_cell_counts(const uint32_t* cellStart, const uint32_t* cellEnd, uint32_t* first,
-                               size_t numCells, uint32_t* ws, hipStream_t s);
+// particles of a system in sub-cell walk order: an entry of its sort holds the particle number in 27 bits
+constexpr uint32_t WALK_MAX_PARTICLES = 1u << 27;
 
-// first[c] = number of particles in cells < c, first[C] = n (from the cell
-// ranges); ws holds scan_levels_words(C) words
-int launch_cell_offsets(const uint32_t* cellStart, const uint32_t* cellEnd, uint32_t* first,
-                        uint32_t numCells, uint32_t n, uint32_t* ws, hipStream_t s);
+// the sub-cell walk order's copy of the sorted rows (DamBreak): pos, vel and
+// particle number of every row, and its row in the reference order
+struct WalkRows {
+    float *pos, *vel;
+    uint32_t *index, *to_ref;
+};
+
+// A step's particles into cell order by counting (cellsort.hip): hash(), then
+// offsets(), then reorder(), on one stream.  The counters are zero between
+// sorts.  first[c] = number of particles in cells < c, first[C] = n, is what the
+// neighbour walkers read: a run of cells with consecutive keys is one range
+// [first[k0], first[k1 + 1]) without any empty-cell test.
+struct CellSort {
+    size_t cells = 0;
+    uint32_t n = 0;
+    void* arena = nullptr;
+    uint32_t *key = nullptr, *place = nullptr, *perm = nullptr;  // per particle; perm: per row
+    uint32_t *cell_count = nullptr, *total = nullptr, *carry = nullptr, *scan_ws = nullptr;
+    uint16_t* occ = nullptr;  // cells that hold sub-cell counts, one bit each
+    uint32_t* pre = nullptr;  // the sub-cell walk's running counts, 16 B a cell
+    bool counts_clean = false;
+
+    int alloc(size_t cells, uint32_t n, hipStream_t s);
+    int alloc_walk(hipStream_t s);
+    void release();
+    int clear(hipStream_t s);
+    // zero counters: they are left so by every sort, one that ended early leaves them to be cleared
+    int ready(hipStream_t s) { return counts_clean ? CMAG_OK : clear(s); }
+    // call in front of a kernel that counts
+    int begin(hipStream_t s);
+    // keys and counts; state: the Peristalsis time record (walls are configured from it)
+    int hash(const cmag_params& P, float* pos, const StepState* state, bool walk, hipStream_t s);
+    // also advances the m records of state by one step (params: a block per record, or P0)
+    int offsets(uint32_t* first, uint32_t* cellStart, bool walk, const cmag_params* params, const cmag_params& P0,
+                StepState* state, uint32_t m, hipStream_t s);
+    int reorder(const float* pos, const float* vel, const uint32_t* first, uint32_t* hash, uint32_t* index,
+                uint32_t* cellEnd, float* sortedPos, float* sortedVel, const WalkRows* walk, hipStream_t s);
+};
 
 // stable LSD radix sort.  Sorts (keys, vals) using (alt_keys, alt_vals) as the
 // ping-pong buffers; *result_in_alt tells where the sorted pair ended up.
@@ -45,20 +75,14 @@ int radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* alt_keys, uint32_
                      uint32_t n, int key_bits, void* workspace, size_t workspace_bytes,
                      bool* result_in_alt, hipStream_t s);
 
-// neighbour passes.  cellFirst (optional, from launch_cell_offsets) selects the
+// neighbour passes.  cellFirst (optional, from CellSort) selects the
 // compact-offset walker; without it the reference cellStart/cellEnd are walked.
 int launch_density(const cmag_params& P, float* measures, const float* sortedPos,
                    const uint32_t* cellStart, const uint32_t* cellEnd, uint32_t n, hipStream_t s,
                    const uint32_t* cellFirst = nullptr);
-// sub-cell walk order (DamBreak): build the internal order from the reference
-// one (pre: 4 uint32 per cell, cleared here; bucket: the rows' buckets from
-// launch_reorder, padded to whole 16-byte words + 16), then density and force
-// over it; density writes the reference-order measures through w2r and leaves
-// -rho (fluid rows) in posW.w and p / rho^2 in velW.w for the force pass
-int launch_subcell_build(const cmag_params& P, const uint32_t* hash, const uint32_t* index, const float* sortedPos,
-                         const float* sortedVel, const uint32_t* cellFirst, uint32_t n, uint32_t numCells,
-                         uint32_t* pre, const uint8_t* bucket, float* posW, float* velW, uint32_t* indexW,
-                         uint32_t* w2r, hipStream_t s);
+// sub-cell walk order (DamBreak; the copies and pre from CellSort): density and
+// force over it; density writes the reference-order measures through w2r and
+// leaves -rho (fluid rows) in posW.w and p / rho^2 in velW.w for the force pass
 // masks (optional, 2 * MASK_ROWS words per particle): density leaves the
 // in-range masks of staged blocks there and force reads them
 int launch_density_sub(const cmag_params& P, float* measures, const uint32_t* w2r, float* posW, float* velW,
@@ -89,11 +113,6 @@ int launch_integrate(const cmag_params& P, float* pos, float* vel, float* velLF,
                      const StepState* state = nullptr);
 int launch_configure_boundary(const cmag_params& P, float* pos, float wave_height, uint32_t n,
                               hipStream_t s);
-// advance one system's state record by one step (one thread), then move the
-// walls to the record's configure_height when it says so
-int launch_step_prologue(const cmag_params& P, StepState* state, hipStream_t s);
-int launch_configure_boundary_from_state(const cmag_params& P, float* pos, const StepState* state, uint32_t n,
-                                         hipStream_t s);
 int launch_shift_right_boundary(const cmag_params& P, float* pos, uint32_t n, hipStream_t s);
 int launch_remove_right_boundary(const cmag_params& P, float* pos, uint32_t n, hipStream_t s);
 

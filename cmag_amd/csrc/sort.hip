@@ -14,6 +14,7 @@
 // No inter-workgroup waiting anywhere, so no launch order assumptions.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "scan_device.hpp"
 
 #include <mutex>
 #include <string>
@@ -32,36 +33,6 @@ constexpr int SCAN_NT = 256;
 constexpr int SCAN_ITEMS = 16;
 constexpr int SCAN_TILE = SCAN_NT * SCAN_ITEMS;
 
-__device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {
-    const int lane = __lane_id();
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        uint32_t t = __shfl_up(v, d, 64);
-        if (lane >= d) v += t;
-    }
-    return v;
-}
-
-// exclusive prefix of v over the workgroup; lds needs NT/64 words
-template <int NT>
-__device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* lds, uint32_t* total) {
-    constexpr int NW = NT / 64;
-    const int lane = __lane_id(), w = threadIdx.x / 64;
-    uint32_t inc = wave_inclusive_scan(v);
-    if (lane == 63) lds[w] = inc;
-    __syncthreads();
-    uint32_t pre = 0, tot = 0;
-#pragma unroll
-    for (int k = 0; k < NW; ++k) {
-        uint32_t x = lds[k];
-        pre += (k < w) ? x : 0u;
-        tot += x;
-    }
-    __syncthreads();
-    *total = tot;
-    return pre + inc - v;
-}
-
 // lanes of this wave whose 8-bit digit equals mine (among valid lanes)
 __device__ __forceinline__ uint64_t match_digit(uint32_t d, bool valid) {
     uint64_t m = __ballot(valid);
@@ -75,36 +46,9 @@ __device__ __forceinline__ uint64_t match_digit(uint32_t d, bool valid) {
 }
 
 // ---- exclusive scan of a uint32 array -------------------------------------
-// The input is a plain array (ScanArray) or the cell counts end - start (0 for
-// an empty cell, whose end is not read for its value) computed from the
-// reorder's cell ranges as they are read (ScanCellCounts).
-struct ScanArray {
-    const uint32_t* in;
-    __device__ __forceinline__ uint32_t at(size_t i) const { return in[i]; }
-    __device__ __forceinline__ uint4 at4(size_t i) const { return *reinterpret_cast<const uint4*>(in + i); }
-    bool aligned16() const { return (reinterpret_cast<uintptr_t>(in) & 15u) == 0; }
-};
-
-struct ScanCellCounts {
-    const uint32_t* start;
-    const uint32_t* end;
-    __device__ static __forceinline__ uint32_t count(uint32_t st, uint32_t en) {
-        return st == CMAG_CELL_EMPTY ? 0u : en - st;
-    }
-    __device__ __forceinline__ uint32_t at(size_t i) const { return count(start[i], end[i]); }
-    __device__ __forceinline__ uint4 at4(size_t i) const {
-        const uint4 a = *reinterpret_cast<const uint4*>(start + i), b = *reinterpret_cast<const uint4*>(end + i);
-        return make_uint4(count(a.x, b.x), count(a.y, b.y), count(a.z, b.z), count(a.w, b.w));
-    }
-    bool aligned16() const {
-        return ((reinterpret_cast<uintptr_t>(start) | reinterpret_cast<uintptr_t>(end)) & 15u) == 0;
-    }
-};
-
 // the block total of one tile; each thread sums SCAN_ITEMS consecutive
 // elements, as 16-byte words when vec and they lie inside len
-template <typename Src>
-__global__ __launch_bounds__(SCAN_NT) void scan_reduce_kernel(const Src src, size_t len,
+__global__ __launch_bounds__(SCAN_NT) void scan_reduce_kernel(const uint32_t* __restrict__ in, size_t len,
                                                                uint32_t* __restrict__ partial, bool vec) {
     __shared__ uint32_t lds[SCAN_NT / 64];
     const size_t base = (size_t)blockIdx.x * SCAN_TILE + (size_t)threadIdx.x * SCAN_ITEMS;
@@ -112,12 +56,12 @@ __global__ __launch_bounds__(SCAN_NT) void scan_reduce_kernel(const Src src, siz
     if (vec && base + SCAN_ITEMS <= len) {
 #pragma unroll
         for (int q = 0; q < SCAN_ITEMS / 4; ++q) {
-            const uint4 x = src.at4(base + 4 * q);
+            const uint4 x = *reinterpret_cast<const uint4*>(in + base + 4 * q);
             sum += (x.x + x.y) + (x.z + x.w);
         }
     } else {
 #pragma unroll
-        for (int k = 0; k < SCAN_ITEMS; ++k) sum += (base + k < len) ? src.at(base + k) : 0u;
+        for (int k = 0; k < SCAN_ITEMS; ++k) sum += (base + k < len) ? in[base + k] : 0u;
     }
     uint32_t tot;
     block_exclusive_scan<SCAN_NT>(sum, lds, &tot);
@@ -129,8 +73,7 @@ __global__ __launch_bounds__(SCAN_NT) void scan_reduce_kernel(const Src src, siz
 // elements lie inside len; `carry` (may be null) holds the exclusive base of
 // every block.  An in-place scan of a plain array is allowed: every thread
 // reads its own elements before the block barrier and writes them after it.
-template <typename Src>
-__global__ __launch_bounds__(SCAN_NT) void scan_down_kernel(const Src src, uint32_t* out, size_t len,
+__global__ __launch_bounds__(SCAN_NT) void scan_down_kernel(const uint32_t* in, uint32_t* out, size_t len,
                                                              const uint32_t* __restrict__ carry, bool vec) {
     static_assert(SCAN_ITEMS % 4 == 0, "16-byte words per thread");
     __shared__ uint32_t lds[SCAN_NT / 64];
@@ -140,12 +83,12 @@ __global__ __launch_bounds__(SCAN_NT) void scan_down_kernel(const Src src, uint3
     if (whole) {
 #pragma unroll
         for (int q = 0; q < SCAN_ITEMS / 4; ++q) {
-            const uint4 x = src.at4(base + 4 * q);
+            const uint4 x = *reinterpret_cast<const uint4*>(in + base + 4 * q);
             v[4 * q] = x.x; v[4 * q + 1] = x.y; v[4 * q + 2] = x.z; v[4 * q + 3] = x.w;
         }
     } else {
 #pragma unroll
-        for (int k = 0; k < SCAN_ITEMS; ++k) v[k] = (base + k < len) ? src.at(base + k) : 0u;
+        for (int k = 0; k < SCAN_ITEMS; ++k) v[k] = (base + k < len) ? in[base + k] : 0u;
     }
     uint32_t sum = 0;
 #pragma unroll
@@ -179,36 +122,24 @@ size_t scan_levels_words(size_t len) {
     return words;
 }
 
-template <typename Src>
-static int exclusive_scan(const Src& src, uint32_t* out, size_t len, uint32_t* ws, hipStream_t s) {
+// out = exclusive_scan(in) (in place allowed); workspace holds scan_levels_words(len) words
+int exclusive_scan_u32(const uint32_t* in, uint32_t* out, size_t len, uint32_t* ws, hipStream_t s) {
     if (len == 0) return CMAG_OK;
-    const bool vec = src.aligned16() && (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
+    const bool vec = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
     if (len <= (size_t)SCAN_TILE) {
-        hipLaunchKernelGGL(scan_down_kernel<Src>, dim3(1), dim3(SCAN_NT), 0, s, src, out, len,
-                           (const uint32_t*)nullptr, vec);
+        hipLaunchKernelGGL(scan_down_kernel, dim3(1), dim3(SCAN_NT), 0, s, in, out, len, (const uint32_t*)nullptr,
+                           vec);
         return check_launch("scan_down_kernel");
     }
     size_t blocks = (len + SCAN_TILE - 1) / SCAN_TILE;
     uint32_t* partial = ws;
-    hipLaunchKernelGGL(scan_reduce_kernel<Src>, dim3((uint32_t)blocks), dim3(SCAN_NT), 0, s, src, len, partial,
-                       vec);
+    hipLaunchKernelGGL(scan_reduce_kernel, dim3((uint32_t)blocks), dim3(SCAN_NT), 0, s, in, len, partial, vec);
     CMAG_TRY(check_launch("scan_reduce_kernel"));
     // scan the partials in place (recursively for very long inputs)
-    CMAG_TRY(exclusive_scan(ScanArray{partial}, partial, blocks, ws + blocks, s));
-    hipLaunchKernelGGL(scan_down_kernel<Src>, dim3((uint32_t)blocks), dim3(SCAN_NT), 0, s, src, out, len,
+    CMAG_TRY(exclusive_scan_u32(partial, partial, blocks, ws + blocks, s));
+    hipLaunchKernelGGL(scan_down_kernel, dim3((uint32_t)blocks), dim3(SCAN_NT), 0, s, in, out, len,
                        (const uint32_t*)partial, vec);
     return check_launch("scan_down_kernel");
-}
-
-// out = exclusive_scan(in); workspace holds scan_levels_words(len) words
-int exclusive_scan_u32(const uint32_t* in, uint32_t* out, size_t len, uint32_t* ws, hipStream_t s) {
-    return exclusive_scan(ScanArray{in}, out, len, ws, s);
-}
-
-// first[c] = exclusive scan of the cell counts; workspace as above
-int exclusive_scan_cell_counts(const uint32_t* cellStart, const uint32_t* cellEnd, uint32_t* first,
-                               size_t numCells, uint32_t* ws, hipStream_t s) {
-    return exclusive_scan(ScanCellCounts{cellStart, cellEnd}, first, numCells, ws, s);
 }
 
 // ---- radix passes ----------------------------------------------------------

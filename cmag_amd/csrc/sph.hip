@@ -147,83 +147,6 @@ int launch_force(const cmag_params& P, float* acc, const float* measures, const 
 }
 
 // ---- sub-cell walk order (DamBreak) ---------------------------------------------
-// The bucket of every sorted row (a byte: fluid eighth 0..7 of the cell
-// along x, walls 8) comes from the reorder.  subcell_move_kernel: row i of
-// the reference order (cell c = hash[i]) moves to row first[c] + below of the
-// sub-cell order, below = the rows of the cell in a lower bucket or in the
-// same bucket and earlier in reference order; the cell's first row also
-// writes the running bucket counts pre[c] (eight 16-bit counts; cells without
-// particles keep the zeros they were cleared to).  O(cell size) work per row (~18 at the
-// measured sizes) over 16-byte loads of the buckets.
-__global__ __launch_bounds__(256) void subcell_move_kernel(const uint32_t* __restrict__ hash,
-                                                           const uint32_t* __restrict__ index,
-                                                           const float4* __restrict__ sortedPos,
-                                                           const float4* __restrict__ sortedVel,
-                                                           const uint32_t* __restrict__ first,
-                                                           const uint8_t* __restrict__ bucket, uint32_t n,
-                                                           uint4* __restrict__ pre, float4* __restrict__ posW,
-                                                           float4* __restrict__ velW, uint32_t* __restrict__ indexW,
-                                                           uint32_t* __restrict__ w2r) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t c = hash[i];
-    const uint32_t a = first[c], b = min(first[c + 1], n);
-    const uint32_t bi = bucket[i];
-    uint32_t below = 0;
-    uint32_t cnt[X_SUBS] = {};  // fluid rows of eighths <= t
-    // the cell's bucket bytes, 16 per load from a 16-byte boundary (the array
-    // is padded so a load never reads past its end)
-    for (uint32_t k16 = a & ~15u; k16 < b; k16 += 16u) {
-        const uint4 v = *reinterpret_cast<const uint4*>(bucket + k16);
-        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-        // byte t of acc counts this chunk's rows of eighths <= t (at most 16)
-        uint64_t acc = 0;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const uint32_t k = k16 + (uint32_t)j;
-            if (k < a || k >= b) continue;
-            const uint32_t bk = (w[j >> 2] >> (8 * (j & 3))) & 0xffu;
-            below += (bk < bi || (bk == bi && k < i)) ? 1u : 0u;
-            acc += bk < (uint32_t)X_SUBS ? 0x0101010101010101ull << (8u * bk) : 0ull;
-        }
-#pragma unroll
-        for (int t = 0; t < X_SUBS; ++t) cnt[t] += (uint32_t)(acc >> (8 * t)) & 0xffu;
-    }
-    const uint32_t w = a + below;
-    if (w >= n) return;  // inconsistent cell arrays only
-    // the walk tells walls from fluid by the sign bit of w (the density pass
-    // stores -rho in fluid rows): every non-fluid row, whatever its type code
-    // (-0.0 and negative codes included), gets the non-negative tag +0
-    float4 p = sortedPos[i];
-    if (p.w != CMAG_DB_FLUID) p.w = 0.0f;
-    posW[w] = p;
-    velW[w] = sortedVel[i];
-    indexW[w] = index[i];
-    w2r[w] = i;
-    // 16-bit counts, capped: a cell of more than 65,535 rows (no physical
-    // state has one) keeps its runs inside the cell
-    if (i == a) {
-        uint32_t h[X_SUBS];
-#pragma unroll
-        for (int t = 0; t < X_SUBS; ++t) h[t] = min(cnt[t], 0xffffu);
-        pre[c] = make_uint4(h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16);
-    }
-}
-
-int launch_subcell_build(const cmag_params& P, const uint32_t* hash, const uint32_t* index, const float* sortedPos,
-                         const float* sortedVel, const uint32_t* cellFirst, uint32_t n, uint32_t numCells,
-                         uint32_t* pre, const uint8_t* bucket, float* posW, float* velW, uint32_t* indexW,
-                         uint32_t* w2r, hipStream_t s) {
-    (void)P;
-    if (n == 0) return CMAG_OK;
-    CMAG_TRY(launch_fill_u32(pre, 0u, 4 * (size_t)numCells, s));
-    hipLaunchKernelGGL(subcell_move_kernel, dim3(div_up(n, 256)), dim3(256), 0, s, hash, index,
-                       reinterpret_cast<const float4*>(sortedPos), reinterpret_cast<const float4*>(sortedVel),
-                       cellFirst, bucket, n, reinterpret_cast<uint4*>(pre), reinterpret_cast<float4*>(posW),
-                       reinterpret_cast<float4*>(velW), indexW, w2r);
-    return check_launch("subcell_move_kernel");
-}
-
 // Density in sub-cell order (cell lookups staged in LDS as in force_sub_kernel,
 // and the candidate positions of four stencil rows as well).
 // The result goes to the reference-order row

@@ -37,17 +37,6 @@ __device__ __forceinline__ float frcp(float x) { return __builtin_amdgcn_rcpf(x)
 __device__ __forceinline__ float frsq(float x) { return __builtin_amdgcn_rsqf(x); }
 __device__ __forceinline__ float fsqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 
-// Workgroups are dispatched round-robin over the 8 XCDs (each with its own
-// L2).  Renumbering them so XCD k runs one contiguous block range keeps the
-// neighbour particles a workgroup reads in the L2 of the XCD that reads them.
-__device__ __forceinline__ uint32_t xcd_block() {
-    constexpr uint32_t XCDS = 8;
-    const uint32_t nb = gridDim.x, b = blockIdx.x;
-    const uint32_t k = b % XCDS, slot = b / XCDS;
-    const uint32_t base = nb / XCDS, extra = nb % XCDS;
-    return k * base + min(k, extra) + slot;
-}
-
 // integer power by squaring (gamma is an integer in [1,15])
 __device__ __forceinline__ float pow_int(float x, int e) {
     float r = 1.0f, b = x;

@@ -23,17 +23,15 @@ struct cmag_system {
     cmag_params P{};
     int ref_kind = REF_NONE;  // system kind when built by a reference constructor
     uint32_t n = 0, numCells = 0;
-    int key_bits = 0;
     hipStream_t stream = nullptr;
     hipStream_t own_stream = nullptr;
 
     float *pos = nullptr, *vel = nullptr, *velLF = nullptr, *acc = nullptr, *presF = nullptr;
     float *measures = nullptr, *sortedPos = nullptr, *sortedVel = nullptr, *predicted = nullptr;
-    uint32_t *hash = nullptr, *index = nullptr, *hashAlt = nullptr, *indexAlt = nullptr;
+    uint32_t *hash = nullptr, *index = nullptr;
     uint32_t *cellStart = nullptr, *cellEnd = nullptr;
-    uint32_t *cellFirst = nullptr, *scanWs = nullptr;  // compact cell offsets for the walkers
-    void* sortWs = nullptr;
-    size_t sortWsBytes = 0;
+    uint32_t* cellFirst = nullptr;  // compact cell offsets for the walkers
+    CellSort sort;
     // adjoint scratch (sorted order), allocated by the first vjp_step
     float *gaccU = nullptr, *gaccS = nullptr, *gposS = nullptr, *gvelS = nullptr, *grho = nullptr;
     // sub-cell walk order (DamBreak): the neighbour passes run over copies of
@@ -42,8 +40,7 @@ struct cmag_system {
     // meaning, and -rho / p into the copies' w for the force pass
     bool subwalk = false;
     float *posW = nullptr, *velW = nullptr;
-    uint32_t *indexW = nullptr, *w2r = nullptr, *preW = nullptr;
-    uint8_t* bucketR = nullptr;
+    uint32_t *indexW = nullptr, *w2r = nullptr;
     // in-range masks the density pass leaves for the force pass (staged blocks
     // of the sub-cell walk): 9 rows x 64 bits per particle
     static constexpr size_t MASK_WORDS = 18;
@@ -95,11 +92,11 @@ struct cmag_system {
         for (hipEvent_t e : ev)
             if (e) (void)hipEventDestroy(e);
         void* bufs[] = {pos, vel, velLF, acc, presF, measures, sortedPos, sortedVel, predicted,
-                        hash, index, hashAlt, indexAlt, cellStart, cellEnd, cellFirst, scanWs, sortWs,
-                        gaccU, gaccS, gposS, gvelS, grho, dState, posW, velW, indexW, w2r, preW, bucketR,
-                        masks, color};
+                        hash, index, cellStart, cellEnd, cellFirst,
+                        gaccU, gaccS, gposS, gvelS, grho, dState, posW, velW, indexW, w2r, masks, color};
         for (void* b : bufs)
             if (b) (void)hipFree(b);
+        sort.release();
         if (own_stream) (void)hipStreamDestroy(own_stream);
     }
 
@@ -115,25 +112,21 @@ struct cmag_system {
             CMAG_HIP_TRY(hipMalloc((void**)&predicted, f4));
             CMAG_HIP_TRY(hipMalloc((void**)&dState, sizeof(StepState)));
         }
-        uint32_t** ub[] = {&hash, &index, &hashAlt, &indexAlt};
+        uint32_t** ub[] = {&hash, &index};
         for (uint32_t** b : ub) CMAG_HIP_TRY(hipMalloc((void**)b, u));
         CMAG_HIP_TRY(hipMalloc((void**)&cellStart, sizeof(uint32_t) * (size_t)numCells));
         CMAG_HIP_TRY(hipMalloc((void**)&cellEnd, sizeof(uint32_t) * (size_t)numCells));
         CMAG_HIP_TRY(hipMalloc((void**)&cellFirst, sizeof(uint32_t) * ((size_t)numCells + 1)));
-        CMAG_HIP_TRY(hipMalloc((void**)&scanWs, sizeof(uint32_t) * (scan_levels_words(numCells) + 1)));
-        sortWsBytes = radix_sort_workspace_bytes(n);
-        CMAG_HIP_TRY(hipMalloc(&sortWs, sortWsBytes));
+        CMAG_TRY(sort.alloc(numCells, n, stream));
         float* zb[] = {pos, vel, velLF, acc, measures, sortedPos, sortedVel, presF, predicted};
         for (float* b : zb)
             if (b) CMAG_HIP_TRY(hipMemsetAsync(b, 0, f4, stream));
-        for (uint32_t* b : {hash, index, hashAlt, indexAlt}) CMAG_HIP_TRY(hipMemsetAsync(b, 0, u, stream));
+        for (uint32_t* b : {hash, index}) CMAG_HIP_TRY(hipMemsetAsync(b, 0, u, stream));
         CMAG_HIP_TRY(hipMemsetAsync(cellStart, 0xff, sizeof(uint32_t) * (size_t)numCells, stream));
         CMAG_HIP_TRY(hipMemsetAsync(cellEnd, 0, sizeof(uint32_t) * (size_t)numCells, stream));
         CMAG_HIP_TRY(hipStreamSynchronize(stream));
         return CMAG_OK;
     }
-
-    int passes() const { return (key_bits + 7) / 8; }
 
     // the sub-cell walk needs DamBreak's DIV_CELL cells, no periodic images,
     // rows whose first and last cells are distinct, and a stencil that reaches
@@ -155,9 +148,7 @@ struct cmag_system {
             // padding rows: the walk reads up to two rows past a run
             for (float** b : {&posW, &velW}) CMAG_HIP_TRY(hipMalloc((void**)b, f4 + 64));
             for (uint32_t** b : {&indexW, &w2r}) CMAG_HIP_TRY(hipMalloc((void**)b, u));
-            // padded to whole 16-byte words: the move kernel reads buckets 16 at a time
-            CMAG_HIP_TRY(hipMalloc((void**)&bucketR, ((size_t)n + 31) & ~(size_t)15));
-            CMAG_HIP_TRY(hipMalloc((void**)&preW, sizeof(uint32_t) * 4 * (size_t)numCells));
+            CMAG_TRY(sort.alloc_walk(stream));
             CMAG_HIP_TRY(hipMalloc((void**)&masks, sizeof(uint32_t) * MASK_WORDS * (size_t)(n ? n : 1)));
         }
         if (on != subwalk) invalidate_graph();
@@ -166,36 +157,24 @@ struct cmag_system {
     }
 
     // hash -> sort -> reorder/cellStart -> density: the neighbour structure
-    // and densities of the current state
+    // and densities of the current state.  For Peristalsis the state record
+    // advances on the device on the way (PeristalsisSystem::Update,
+    // PeristalsisSystem.cpp:330-343) and the walls are configured when it says so
     int enqueue_front() {
-        // the hash goes to whichever buffer makes the sort end in (hash, index)
-        const bool odd = passes() % 2 == 1;
-        uint32_t* hk = odd ? hashAlt : hash;
-        uint32_t* hv = odd ? indexAlt : index;
+        // the walk order's entries carry a particle's bucket above its number
+        if (subwalk && n >= WALK_MAX_PARTICLES) return fail(CMAG_E_INVALID, "force passes take at most 2^27 particles");
+        StepState* st = P.system == CMAG_SYS_PERISTALSIS ? dState : nullptr;
         CMAG_TRY(mark(CMAG_STAGE_HASH));
-        CMAG_TRY(launch_calc_hash(P, pos, hk, hv, n, stream));
+        CMAG_TRY(sort.hash(P, pos, st, subwalk, stream));
         CMAG_TRY(mark(CMAG_STAGE_SORT));
-        bool in_alt = false;
-        CMAG_TRY(radix_sort_pairs(hk, hv, odd ? hash : hashAlt, odd ? index : indexAlt, n, key_bits,
-                                  sortWs, sortWsBytes, &in_alt, stream));
-        const bool sorted_moved = n >= 2 && key_bits > 0;
-        if (sorted_moved && in_alt != odd)
-            return fail(CMAG_E_STATE, "radix sort ended in an unexpected buffer");
-        if (!sorted_moved && odd) {
-            // no pass ran: move the keys from where the hash put them
-            CMAG_TRY(launch_copy_u32(hash, hk, n, stream));
-            CMAG_TRY(launch_copy_u32(index, hv, n, stream));
-        }
+        CMAG_TRY(sort.offsets(cellFirst, cellStart, subwalk, nullptr, P, st, st ? 1u : 0u, stream));
         CMAG_TRY(mark(CMAG_STAGE_REORDER));
-        CMAG_TRY(launch_reorder(cellStart, cellEnd, sortedPos, sortedVel, hash, index, pos, velLF, n,
-                                numCells, stream, &P, subwalk ? bucketR : nullptr));
-        CMAG_TRY(launch_cell_offsets(cellStart, cellEnd, cellFirst, numCells, n, scanWs, stream));
-        if (subwalk)
-            CMAG_TRY(launch_subcell_build(P, hash, index, sortedPos, sortedVel, cellFirst, n, numCells, preW, bucketR,
-                                          posW, velW, indexW, w2r, stream));
+        const WalkRows rows{posW, velW, indexW, w2r};
+        CMAG_TRY(sort.reorder(pos, velLF, cellFirst, hash, index, cellEnd, sortedPos, sortedVel,
+                              subwalk ? &rows : nullptr, stream));
         CMAG_TRY(mark(CMAG_STAGE_DENSITY));
         if (subwalk)
-            CMAG_TRY(launch_density_sub(P, measures, w2r, posW, velW, cellFirst, preW, n, stream,
+            CMAG_TRY(launch_density_sub(P, measures, w2r, posW, velW, cellFirst, sort.pre, n, stream,
                                         use_masks ? masks : nullptr));
         else
             CMAG_TRY(launch_density(P, measures, sortedPos, cellStart, cellEnd, n, stream, cellFirst));
@@ -210,7 +189,7 @@ struct cmag_system {
             CMAG_TRY(launch_peristalsis_forces(P, acc, presF, measures, sortedPos, sortedVel, index,
                                                cellStart, cellEnd, n, stream, cellFirst));
         } else if (subwalk) {
-            CMAG_TRY(launch_force_sub(P, acc, posW, velW, indexW, cellFirst, preW, n, stream,
+            CMAG_TRY(launch_force_sub(P, acc, posW, velW, indexW, cellFirst, sort.pre, n, stream,
                                       use_masks ? masks : nullptr));
         } else {
             CMAG_TRY(launch_force(P, acc, measures, sortedPos, sortedVel, index, cellStart, cellEnd, n,
@@ -221,17 +200,6 @@ struct cmag_system {
         CMAG_TRY(mark(CMAG_NUM_STAGES));
         if (timing) pending = true;
         return CMAG_OK;
-    }
-
-    // one update() on the stream: for Peristalsis the state record advances on
-    // the device (PeristalsisSystem::Update, PeristalsisSystem.cpp:330-343) and
-    // the walls are configured when it says so, in front of the step
-    int enqueue_update() {
-        if (P.system == CMAG_SYS_PERISTALSIS) {
-            CMAG_TRY(launch_step_prologue(P, dState, stream));
-            CMAG_TRY(launch_configure_boundary_from_state(P, pos, dState, n, stream));
-        }
-        return enqueue_step();
     }
 
     // send the host's state record to the device if the host changed it
@@ -260,7 +228,7 @@ struct cmag_system {
     int update() {
         CMAG_TRY(collect());
         CMAG_TRY(upload_state());
-        CMAG_TRY(enqueue_update());
+        CMAG_TRY(enqueue_step());
         advance_clock();
         return CMAG_OK;
     }
@@ -278,7 +246,7 @@ struct cmag_system {
         const bool was_timing = timing;
         timing = false;  // no event nodes inside the graph
         CMAG_HIP_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-        int rc = enqueue_update();
+        int rc = enqueue_step();
         timing = was_timing;
         hipError_t e = hipStreamEndCapture(stream, &g);
         if (rc != CMAG_OK) {
@@ -301,6 +269,7 @@ struct cmag_system {
         CMAG_TRY(collect());
         CMAG_TRY(upload_state());
         if (!graph_valid) CMAG_TRY(build_graph());
+        CMAG_TRY(sort.ready(stream));
         for (uint32_t k = 0; k < steps; ++k) {
             CMAG_HIP_TRY(hipGraphLaunch(graph, stream));
             advance_clock();
@@ -421,7 +390,6 @@ static int make_system(const cmag_params& P, uint32_t n, int ref_kind, cmag_syst
     s->ref_kind = ref_kind;
     s->n = n;
     s->numCells = cmag_params_num_cells(&P);
-    s->key_bits = cmag_params_key_bits(&P);
     s->hstate = initial_step_state(P, 0.0f);
     int rc = s->alloc();
     if (rc == CMAG_OK && s->subwalk_eligible()) rc = s->set_subwalk(true);
@@ -606,7 +574,6 @@ int cmag_system_set_params(cmag_system* s, const cmag_params* p) {
         if (p->grid_size[a] != s->P.grid_size[a]) return fail(CMAG_E_INVALID, "set_params may not change the grid");
     if (p->system != s->P.system) return fail(CMAG_E_INVALID, "set_params may not change the system kind");
     s->P = *p;
-    s->key_bits = cmag_params_key_bits(p);
     s->state_dirty = true;
     s->invalidate_graph();
     if (s->subwalk && !s->subwalk_eligible()) s->subwalk = false;
