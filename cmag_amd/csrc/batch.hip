@@ -96,7 +96,9 @@ __global__ __launch_bounds__(256) void batch_density_kernel(const cmag_params* _
                                                             const uint2* __restrict__ tiles, uint32_t num_tiles,
                                                             float4* __restrict__ measures,
                                                             const float4* __restrict__ sortedPos,
-                                                            const uint32_t* __restrict__ cellFirst) {
+                                                            const uint32_t* __restrict__ cellFirst,
+                                                            float2* __restrict__ pairs, uint32_t* __restrict__ masks,
+                                                            uint32_t n) {
     uint32_t t0, t1;
     tile_chunk(num_tiles, t0, t1);
     for (uint32_t t = t0; t < t1; ++t) {
@@ -106,12 +108,13 @@ __global__ __launch_bounds__(256) void batch_density_kernel(const cmag_params* _
         if (i >= I.part1) continue;
         const cmag_params& P = params[tile.x];
         const FirstCells cells{cellFirst + I.cell0};
+        uint32_t* const mk = masks && row_masks_apply(P) ? masks : nullptr;
         if (P.system == CMAG_SYS_DAMBREAK)
             density_body<CMAG_SYS_DAMBREAK, DIM, HASH>(P, i, measures, sortedPos, cells);
         else if (P.system == CMAG_SYS_POISEUILLE)
-            density_body<CMAG_SYS_POISEUILLE, DIM, HASH>(P, i, measures, sortedPos, cells);
+            density_body<CMAG_SYS_POISEUILLE, DIM, HASH>(P, i, measures, sortedPos, cells, pairs, mk, n);
         else
-            density_body<CMAG_SYS_PERISTALSIS, DIM, HASH>(P, i, measures, sortedPos, cells);
+            density_body<CMAG_SYS_PERISTALSIS, DIM, HASH>(P, i, measures, sortedPos, cells, pairs, mk, n);
     }
 }
 
@@ -124,7 +127,9 @@ __global__ __launch_bounds__(256) void batch_force_kernel(const cmag_params* __r
                                                           const float4* __restrict__ sortedPos,
                                                           const float4* __restrict__ sortedVel,
                                                           const uint32_t* __restrict__ index,
-                                                          const uint32_t* __restrict__ cellFirst, uint32_t n) {
+                                                          const uint32_t* __restrict__ cellFirst,
+                                                          const float2* __restrict__ pairs,
+                                                          const uint32_t* __restrict__ masks, uint32_t n) {
     __shared__ uint32_t nbl[256 / 64][CAP][64];
     uint32_t(*mine)[64] = nbl[threadIdx.x >> 6];
     uint32_t t0, t1;
@@ -136,15 +141,18 @@ __global__ __launch_bounds__(256) void batch_force_kernel(const cmag_params* __r
         if (i >= I.part1) continue;
         const cmag_params& P = params[tile.x];
         const FirstCells cells{cellFirst + I.cell0};
+        const uint32_t* const mk = masks && row_masks_apply(P) ? masks : nullptr;
         if (P.system == CMAG_SYS_DAMBREAK)
             force_body<CMAG_SYS_DAMBREAK, DIM, HASH, FirstCells, CAP>(P, i, acc, measures, sortedPos, sortedVel,
                                                                       index, cells, n, mine);
         else if (P.system == CMAG_SYS_POISEUILLE)
-            force_body<CMAG_SYS_POISEUILLE, DIM, HASH, FirstCells, CAP>(P, i, acc, measures, sortedPos,
-                                                                        sortedVel, index, cells, n, mine);
+            force_body<CMAG_SYS_POISEUILLE, DIM, HASH, FirstCells, CAP>(P, i, acc, measures, sortedPos, sortedVel,
+                                                                        index, cells, n, mine, nullptr, nullptr,
+                                                                        nullptr, n, pairs, mk);
         else
             peristalsis_force_body<DIM, HASH, true, true, FirstCells, CAP>(P, i, acc, presF, measures, sortedPos,
-                                                                           sortedVel, index, cells, n, mine);
+                                                                           sortedVel, index, cells, n, mine, pairs, mk,
+                                                                           n);
     }
 }
 
@@ -196,6 +204,8 @@ struct cmag_batch {
 
     float *pos = nullptr, *vel = nullptr, *velLF = nullptr, *acc = nullptr, *presF = nullptr;
     float *measures = nullptr, *sortedPos = nullptr, *sortedVel = nullptr;
+    float* pairs = nullptr;         // the density pass's pair values and in-range masks
+    uint32_t* rowMasks = nullptr;   // for the force pass (sph_device.hpp)
     uint32_t *hash = nullptr, *index = nullptr;
     uint32_t *cellStart = nullptr, *cellEnd = nullptr, *cellFirst = nullptr;
     CellSort sort;
@@ -214,7 +224,7 @@ struct cmag_batch {
         for (hipEvent_t e : ev)
             if (e) (void)hipEventDestroy(e);
         void* bufs[] = {dP, dI, dS, dTiles, pos, vel, velLF, acc, presF, measures, sortedPos, sortedVel,
-                        hash, index, cellStart, cellEnd, cellFirst};
+                        hash, index, cellStart, cellEnd, cellFirst, pairs, rowMasks};
         for (void* b : bufs)
             if (b) (void)hipFree(b);
         sort.release();
@@ -230,9 +240,14 @@ struct cmag_batch {
         const size_t u = sizeof(uint32_t) * (size_t)n;
         float** fb[] = {&pos, &vel, &velLF, &acc, &presF, &measures, &sortedPos, &sortedVel};
         for (float** b : fb) {
-            CMAG_HIP_TRY(hipMalloc((void**)b, f4));
+            // padding rows: the neighbour walks read up to two rows past a run
+            CMAG_HIP_TRY(hipMalloc((void**)b, f4 + (b == &sortedPos ? 64 : 0)));
             CMAG_HIP_TRY(hipMemsetAsync(*b, 0, f4, stream));
         }
+        CMAG_HIP_TRY(hipMalloc((void**)&pairs, f4 / 2));
+        bool any_masks = false;
+        for (const cmag_params& q : P) any_masks = any_masks || row_masks_apply(q);
+        if (any_masks) CMAG_HIP_TRY(hipMalloc((void**)&rowMasks, u * ROW_MASK_ROWS));
         uint32_t** ub[] = {&hash, &index};
         for (uint32_t** b : ub) {
             CMAG_HIP_TRY(hipMalloc((void**)b, u));
@@ -308,7 +323,8 @@ struct cmag_batch {
         auto c4 = [](const float* q) { return reinterpret_cast<const float4*>(q); };
 #define CMAG_BATCH_FORCE(CAP)                                                                              \
     hipLaunchKernelGGL((batch_force_kernel<DIM, HASH, CAP>), g, b, 0, stream, dP, dI, dTiles, numTiles,     \
-                       f4(acc), f4(presF), c4(measures), c4(sortedPos), c4(sortedVel), index, cellFirst, n)
+                       f4(acc), f4(presF), c4(measures), c4(sortedPos), c4(sortedVel), index, cellFirst,      \
+                       reinterpret_cast<const float2*>(pairs), rowMasks, n)
         if (tune.nb_cap == 8) CMAG_BATCH_FORCE(8);
         else if (tune.nb_cap == 32) CMAG_BATCH_FORCE(32);
         else CMAG_BATCH_FORCE(16);
@@ -320,7 +336,7 @@ struct cmag_batch {
     int launch_passes(dim3 g, dim3 b) {
         hipLaunchKernelGGL((batch_density_kernel<DIM, HASH>), g, b, 0, stream, dP, dI, dTiles, numTiles,
                            reinterpret_cast<float4*>(measures), reinterpret_cast<const float4*>(sortedPos),
-                           cellFirst);
+                           cellFirst, reinterpret_cast<float2*>(pairs), rowMasks, n);
         CMAG_TRY(check_launch("batch_density_kernel"));
         CMAG_TRY(mark(CMAG_STAGE_FORCE));
         return launch_force_cap<DIM, HASH>(g, b);

@@ -140,7 +140,7 @@ __global__ __launch_bounds__(NT) void cell_offsets_kernel(const uint32_t* __rest
             // whole tiles in front: whole 16-byte words
             const uint4* w = reinterpret_cast<const uint4*>(cell_count);
             const size_t words = (size_t)tile * off_tile(NT) / 4;
-#pragma unroll 4
+#pragma unroll 14
             for (size_t q = threadIdx.x; q < words; q += NT) sum += sum4(w[q]);
         }
         (void)block_exclusive_scan<NT>(sum, lds, &base);

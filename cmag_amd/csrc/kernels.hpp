@@ -77,9 +77,17 @@ int radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* alt_keys, uint32_
 
 // neighbour passes.  cellFirst (optional, from CellSort) selects the
 // compact-offset walker; without it the reference cellStart/cellEnd are walked.
+// With cellFirst the rows of sortedPos are followed by two of padding, and the
+// channels' density pass leaves pair values (2 floats a row) and, with
+// row_masks, in-range masks (ROW_MASK_ROWS words a row) for the force pass.
+constexpr int ROW_MASK_ROWS = 7;  // stencils of up to 3 cells a side
+__host__ __device__ inline bool row_masks_apply(const cmag_params& P) {
+    return P.dim == 2 && P.system != CMAG_SYS_DAMBREAK && P.hash_order == CMAG_HASH_LINEAR &&
+           2 * P.cellcount + 1 <= ROW_MASK_ROWS;
+}
 int launch_density(const cmag_params& P, float* measures, const float* sortedPos,
                    const uint32_t* cellStart, const uint32_t* cellEnd, uint32_t n, hipStream_t s,
-                   const uint32_t* cellFirst = nullptr);
+                   const uint32_t* cellFirst = nullptr, float* pairs = nullptr, uint32_t* row_masks = nullptr);
 // sub-cell walk order (DamBreak; the copies and pre from CellSort): density and
 // force over it; density writes the reference-order measures through w2r and
 // leaves -rho (fluid rows) in posW.w and p / rho^2 in velW.w for the force pass
@@ -94,11 +102,13 @@ int launch_force_sub(const cmag_params& P, float* acc, const float* posW, const 
 int launch_force(const cmag_params& P, float* acc, const float* measures, const float* sortedPos,
                  const float* sortedVel, const uint32_t* index, const uint32_t* cellStart,
                  const uint32_t* cellEnd, uint32_t n, hipStream_t s,
-                 const uint32_t* cellFirst = nullptr);
+                 const uint32_t* cellFirst = nullptr, const float* pairs = nullptr,
+                 const uint32_t* row_masks = nullptr);
 int launch_peristalsis_forces(const cmag_params& P, float* viscF, float* presF, const float* measures,
                               const float* sortedPos, const float* sortedVel, const uint32_t* index,
                               const uint32_t* cellStart, const uint32_t* cellEnd, uint32_t n,
-                              hipStream_t s, const uint32_t* cellFirst = nullptr);
+                              hipStream_t s, const uint32_t* cellFirst = nullptr, const float* pairs = nullptr,
+                              const uint32_t* row_masks = nullptr);
 int launch_pressure_force(const cmag_params& P, float* presF, const float* measures,
                           const float* sortedPos, const uint32_t* index, const uint32_t* cellStart,
                           const uint32_t* cellEnd, uint32_t n, hipStream_t s);

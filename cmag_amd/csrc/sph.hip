@@ -10,10 +10,11 @@ namespace cmag {
 template <int SYS, int DIM, int HASH, typename Cells>
 __global__ __launch_bounds__(256) void density_kernel(const cmag_params P, float4* __restrict__ measures,
                                                        const float4* __restrict__ sortedPos, const Cells cells,
-                                                       uint32_t n) {
+                                                       uint32_t n, float2* __restrict__ pairs,
+                                                       uint32_t* __restrict__ row_masks) {
     const uint32_t i = xcd_block() * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    density_body<SYS, DIM, HASH>(P, i, measures, sortedPos, cells);
+    density_body<SYS, DIM, HASH>(P, i, measures, sortedPos, cells, pairs, row_masks, n);
 }
 
 template <int SYS, int DIM, int HASH, typename Cells>
@@ -22,11 +23,13 @@ __global__ __launch_bounds__(256) void force_kernel(const cmag_params P, float4*
                                                      const float4* __restrict__ sortedPos,
                                                      const float4* __restrict__ sortedVel,
                                                      const uint32_t* __restrict__ index, const Cells cells,
-                                                     uint32_t n) {
+                                                     uint32_t n, const float2* __restrict__ pairs,
+                                                     const uint32_t* __restrict__ row_masks) {
     __shared__ uint32_t nbl[256 / 64][NB_CAP][64];
     const uint32_t i = xcd_block() * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    force_body<SYS, DIM, HASH>(P, i, acc, measures, sortedPos, sortedVel, index, cells, n, nbl[threadIdx.x >> 6]);
+    force_body<SYS, DIM, HASH>(P, i, acc, measures, sortedPos, sortedVel, index, cells, n, nbl[threadIdx.x >> 6],
+                               nullptr, nullptr, nullptr, n, pairs, row_masks);
 }
 
 // Peristalsis: pressure and viscous passes; the fused variant produces both
@@ -36,12 +39,13 @@ __global__ __launch_bounds__(256) void peristalsis_force_kernel(
     const cmag_params P, float4* __restrict__ viscF, float4* __restrict__ presF,
     const float4* __restrict__ measures, const float4* __restrict__ sortedPos,
     const float4* __restrict__ sortedVel, const uint32_t* __restrict__ index, const Cells cells,
-    uint32_t n) {
+    uint32_t n, const float2* __restrict__ pairs, const uint32_t* __restrict__ row_masks) {
     __shared__ uint32_t nbl[256 / 64][NB_CAP][64];
     const uint32_t i = xcd_block() * blockDim.x + threadIdx.x;
     if (i >= n) return;
     peristalsis_force_body<DIM, HASH, WANT_VISC, WANT_PRES>(P, i, viscF, presF, measures, sortedPos, sortedVel,
-                                                            index, cells, n, nbl[threadIdx.x >> 6]);
+                                                            index, cells, n, nbl[threadIdx.x >> 6], pairs, row_masks,
+                                                            n);
 }
 
 // in-range neighbours (j != i, r^2 < 4h^2) of each sorted particle: the pair
@@ -86,23 +90,25 @@ template <int SYS, int DIM, int H>
 struct DensityGo {
     template <typename Cells>
     static void run(const cmag_params& P, float* measures, const float* sortedPos, const Cells& cells,
-                    uint32_t n, hipStream_t s) {
+                    uint32_t n, float* pairs, uint32_t* row_masks, hipStream_t s) {
         hipLaunchKernelGGL((density_kernel<SYS, DIM, H, Cells>), dim3(div_up(n, 256)), dim3(256), 0, s, P,
                            reinterpret_cast<float4*>(measures), reinterpret_cast<const float4*>(sortedPos),
-                           cells, n);
+                           cells, n, reinterpret_cast<float2*>(pairs), row_masks);
     }
     static void go(const cmag_params& P, float* measures, const float* sortedPos, const uint32_t* cellStart,
-                   const uint32_t* cellEnd, const uint32_t* cellFirst, uint32_t n, hipStream_t s) {
-        if (cellFirst) run(P, measures, sortedPos, FirstCells{cellFirst}, n, s);
-        else run(P, measures, sortedPos, RefCells{cellStart, cellEnd, n}, n, s);
+                   const uint32_t* cellEnd, const uint32_t* cellFirst, uint32_t n, float* pairs, uint32_t* row_masks,
+                   hipStream_t s) {
+        if (cellFirst) run(P, measures, sortedPos, FirstCells{cellFirst}, n, pairs, row_masks, s);
+        else run(P, measures, sortedPos, RefCells{cellStart, cellEnd, n}, n, nullptr, nullptr, s);
     }
 };
 
 int launch_density(const cmag_params& P, float* measures, const float* sortedPos,
                    const uint32_t* cellStart, const uint32_t* cellEnd, uint32_t n, hipStream_t s,
-                   const uint32_t* cellFirst) {
+                   const uint32_t* cellFirst, float* pairs, uint32_t* row_masks) {
     if (n == 0) return CMAG_OK;
-    dispatch3<DensityGo>(P, P, measures, sortedPos, cellStart, cellEnd, cellFirst, n, s);
+    dispatch3<DensityGo>(P, P, measures, sortedPos, cellStart, cellEnd, cellFirst, n, pairs,
+                         row_masks && row_masks_apply(P) ? row_masks : nullptr, s);
     return check_launch("density_kernel");
 }
 
@@ -120,29 +126,38 @@ struct ForceGo {
     template <typename Cells>
     static void run(const cmag_params& P, float* acc, const float* measures, const float* sortedPos,
                     const float* sortedVel, const uint32_t* index, const Cells& cells, uint32_t n,
-                    hipStream_t s) {
+                    const float* pairs, const uint32_t* row_masks, hipStream_t s) {
         if constexpr (SYS != CMAG_SYS_PERISTALSIS)
             hipLaunchKernelGGL((force_kernel<SYS, DIM, H, Cells>), dim3(div_up(n, 256)), dim3(256), 0, s, P,
                                reinterpret_cast<float4*>(acc), reinterpret_cast<const float4*>(measures),
                                reinterpret_cast<const float4*>(sortedPos),
-                               reinterpret_cast<const float4*>(sortedVel), index, cells, n);
+                               reinterpret_cast<const float4*>(sortedVel), index, cells, n,
+                               reinterpret_cast<const float2*>(pairs), row_masks);
     }
     static void go(const cmag_params& P, float* acc, const float* measures, const float* sortedPos,
                    const float* sortedVel, const uint32_t* index, const uint32_t* cellStart,
-                   const uint32_t* cellEnd, const uint32_t* cellFirst, uint32_t n, hipStream_t s) {
-        if (cellFirst) run(P, acc, measures, sortedPos, sortedVel, index, FirstCells{cellFirst}, n, s);
-        else run(P, acc, measures, sortedPos, sortedVel, index, RefCells{cellStart, cellEnd, n}, n, s);
+                   const uint32_t* cellEnd, const uint32_t* cellFirst, uint32_t n, const float* pairs,
+                   const uint32_t* row_masks, hipStream_t s) {
+        if (cellFirst)
+            run(P, acc, measures, sortedPos, sortedVel, index, FirstCells{cellFirst}, n, pairs, row_masks, s);
+        else
+            run(P, acc, measures, sortedPos, sortedVel, index, RefCells{cellStart, cellEnd, n}, n, nullptr, nullptr,
+                s);
     }
 };
 
 int launch_force(const cmag_params& P, float* acc, const float* measures, const float* sortedPos,
                  const float* sortedVel, const uint32_t* index, const uint32_t* cellStart,
-                 const uint32_t* cellEnd, uint32_t n, hipStream_t s, const uint32_t* cellFirst) {
+                 const uint32_t* cellEnd, uint32_t n, hipStream_t s, const uint32_t* cellFirst, const float* pairs,
+                 const uint32_t* row_masks) {
     if (n == 0) return CMAG_OK;
     if (n >= (1u << NB_SHIFT_BITS)) return fail(CMAG_E_INVALID, "force passes take at most 2^27 particles");
     if (P.system == CMAG_SYS_PERISTALSIS)
         return fail(CMAG_E_INVALID, "Peristalsis uses the split pressure/viscous passes");
-    dispatch3<ForceGo>(P, P, acc, measures, sortedPos, sortedVel, index, cellStart, cellEnd, cellFirst, n, s);
+    if (cellFirst && P.system != CMAG_SYS_DAMBREAK && !pairs)
+        return fail(CMAG_E_INVALID, "the force pass over compact offsets takes the density pass's pair values");
+    dispatch3<ForceGo>(P, P, acc, measures, sortedPos, sortedVel, index, cellStart, cellEnd, cellFirst, n, pairs,
+                       row_masks && row_masks_apply(P) ? row_masks : nullptr, s);
     return check_launch("force_kernel");
 }
 
@@ -260,13 +275,14 @@ int launch_force_sub(const cmag_params& P, float* acc, const float* posW, const 
 template <bool V, bool PR, typename Cells>
 static void go_peri_cells(const cmag_params& P, float* viscF, float* presF, const float* measures,
                           const float* sortedPos, const float* sortedVel, const uint32_t* index,
-                          const Cells& cells, uint32_t n, hipStream_t s) {
+                          const Cells& cells, uint32_t n, const float* pairs, const uint32_t* row_masks,
+                          hipStream_t s) {
     const bool m = P.hash_order == CMAG_HASH_MORTON;
     auto launch = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3(div_up(n, 256)), dim3(256), 0, s, P, reinterpret_cast<float4*>(viscF),
                            reinterpret_cast<float4*>(presF), reinterpret_cast<const float4*>(measures),
                            reinterpret_cast<const float4*>(sortedPos), reinterpret_cast<const float4*>(sortedVel),
-                           index, cells, n);
+                           index, cells, n, reinterpret_cast<const float2*>(pairs), row_masks);
     };
     if (P.dim == 3) {
         if (m) launch(peristalsis_force_kernel<3, 1, V, PR, Cells>);
@@ -280,14 +296,10 @@ static void go_peri_cells(const cmag_params& P, float* viscF, float* presF, cons
 template <bool V, bool PR>
 static void go_peri(const cmag_params& P, float* viscF, float* presF, const float* measures,
                     const float* sortedPos, const float* sortedVel, const uint32_t* index,
-                    const uint32_t* cellStart, const uint32_t* cellEnd, const uint32_t* cellFirst, uint32_t n,
-                    hipStream_t s) {
+                    const uint32_t* cellStart, const uint32_t* cellEnd, uint32_t n, hipStream_t s) {
     if (n >= (1u << NB_SHIFT_BITS)) return;  // rejected by the callers
-    if (cellFirst)
-        go_peri_cells<V, PR>(P, viscF, presF, measures, sortedPos, sortedVel, index, FirstCells{cellFirst}, n, s);
-    else
-        go_peri_cells<V, PR>(P, viscF, presF, measures, sortedPos, sortedVel, index,
-                             RefCells{cellStart, cellEnd, n}, n, s);
+    go_peri_cells<V, PR>(P, viscF, presF, measures, sortedPos, sortedVel, index, RefCells{cellStart, cellEnd, n}, n,
+                         nullptr, nullptr, s);
 }
 
 int launch_pressure_force(const cmag_params& P, float* presF, const float* measures,
@@ -295,7 +307,7 @@ int launch_pressure_force(const cmag_params& P, float* presF, const float* measu
                           const uint32_t* cellEnd, uint32_t n, hipStream_t s) {
     if (n == 0) return CMAG_OK;
     if (n >= (1u << NB_SHIFT_BITS)) return fail(CMAG_E_INVALID, "force passes take at most 2^27 particles");
-    go_peri<false, true>(P, nullptr, presF, measures, sortedPos, nullptr, index, cellStart, cellEnd, nullptr, n, s);
+    go_peri<false, true>(P, nullptr, presF, measures, sortedPos, nullptr, index, cellStart, cellEnd, n, s);
     return check_launch("peristalsis_force_kernel<pressure>");
 }
 
@@ -305,17 +317,24 @@ int launch_viscous_force(const cmag_params& P, float* viscF, const float* measur
                          hipStream_t s) {
     if (n == 0) return CMAG_OK;
     if (n >= (1u << NB_SHIFT_BITS)) return fail(CMAG_E_INVALID, "force passes take at most 2^27 particles");
-    go_peri<true, false>(P, viscF, nullptr, measures, sortedPos, sortedVel, index, cellStart, cellEnd, nullptr, n, s);
+    go_peri<true, false>(P, viscF, nullptr, measures, sortedPos, sortedVel, index, cellStart, cellEnd, n, s);
     return check_launch("peristalsis_force_kernel<viscous>");
 }
 
 int launch_peristalsis_forces(const cmag_params& P, float* viscF, float* presF, const float* measures,
                               const float* sortedPos, const float* sortedVel, const uint32_t* index,
                               const uint32_t* cellStart, const uint32_t* cellEnd, uint32_t n,
-                              hipStream_t s, const uint32_t* cellFirst) {
+                              hipStream_t s, const uint32_t* cellFirst, const float* pairs,
+                              const uint32_t* row_masks) {
     if (n == 0) return CMAG_OK;
     if (n >= (1u << NB_SHIFT_BITS)) return fail(CMAG_E_INVALID, "force passes take at most 2^27 particles");
-    go_peri<true, true>(P, viscF, presF, measures, sortedPos, sortedVel, index, cellStart, cellEnd, cellFirst, n, s);
+    if (!cellFirst) {
+        go_peri<true, true>(P, viscF, presF, measures, sortedPos, sortedVel, index, cellStart, cellEnd, n, s);
+        return check_launch("peristalsis_force_kernel<fused>");
+    }
+    if (!pairs) return fail(CMAG_E_INVALID, "the force pass over compact offsets takes the density pass's pair values");
+    go_peri_cells<true, true>(P, viscF, presF, measures, sortedPos, sortedVel, index, FirstCells{cellFirst}, n, pairs,
+                              row_masks && row_masks_apply(P) ? row_masks : nullptr, s);
     return check_launch("peristalsis_force_kernel<fused>");
 }
 

@@ -18,6 +18,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "kernels.hpp"
 
 // Every fused multiply-add below is written out (fmaf) and no other is formed:
 // the same sum then rounds the same way in every kernel that inlines it
@@ -61,6 +62,7 @@ __device__ __forceinline__ float eos(const cmag_params& P, float dens) {
 //   FirstCells compact offsets first[c] (cells before c), one pair of loads
 struct RefCells {
     static constexpr bool SUB = false;
+    static constexpr bool PADDED = false;  // a caller's rows: nothing is read past them
     const uint32_t* __restrict__ cellStart;
     const uint32_t* __restrict__ cellEnd;
     uint32_t n;
@@ -81,6 +83,7 @@ struct RefCells {
 
 struct FirstCells {
     static constexpr bool SUB = false;
+    static constexpr bool PADDED = true;  // rows of a System or batch: two may be read past the last
     const uint32_t* __restrict__ first;
     __device__ __forceinline__ bool range(uint32_t k0, uint32_t k1, uint32_t& s, uint32_t& e) const {
         s = first[k0];
@@ -106,6 +109,7 @@ struct FirstCells {
 // zeros
 struct SubCells {
     static constexpr bool SUB = true;
+    static constexpr bool PADDED = true;
     const uint32_t* __restrict__ first;
     const uint4* __restrict__ pre;
     // count t (0..7) of a cell's entry, read as one 16-bit value (the eighth
@@ -171,14 +175,22 @@ __device__ __forceinline__ int force_row(int dim, int k) {
 // different x would otherwise serialise the wave.
 // PERIODIC = false compiles the image shifts out (DamBreak has none).
 //
-// walk_rows does the walk and hands each row's runs to row(a, b, qy, qz);
+// In the linear order a target inside the grid along x has the same one or two
+// runs of cells (two where its stencil crosses the seam) relative to every row,
+// so they are found once: a wave all of whose targets are so takes each row
+// with two to four offset loads.  Stepping through a row's cells instead cost
+// more than half the instructions of the 2-D passes (7 x 7 cells of one
+// spacing, 4.1M particles in 256 channels: density 2,647 VALU instructions per
+// wave of 64 targets and 264 us, force 4,582 and 552 us).
+//
+// walk_rows does the walk and hands each row's runs to row(a, b, qy, qz, whole);
+// whole: the whole row comes in this one call (in every lane of the wave).
 // walk_stencil and walk_stencil_pf turn them into candidate calls.  With
 // FORCE_ORDER and one cell per stencil side, the rows come in force_row order.
 template <int DIM, int HASH, bool PERIODIC = true, bool FORCE_ORDER = false, typename Cells, typename R>
 __device__ __forceinline__ void walk_rows(const cmag_params& P, const float4& pi, const Cell& gp,
                                           const Cells& cells, R&& run_pair) {
     const int cc = P.cellcount;
-    const int zlo = DIM == 2 ? 0 : -cc, zhi = DIM == 2 ? 0 : cc;
     const int sub = Cells::SUB ? x_sub(P, pi.x) : 0;
     const uint32_t gxm = P.grid_size[0] - 1u, gym = P.grid_size[1] - 1u, gzm = P.grid_size[2] - 1u;
     const uint32_t Mx = P.morton_mask[0], My = P.morton_mask[1], Mz = P.morton_mask[2];
@@ -196,6 +208,27 @@ __device__ __forceinline__ void walk_rows(const cmag_params& P, const float4& pi
             if (DIM == 3) kz0 = dilated_dec(kz0, Mz);
         }
     }
+    // linear order: the same cells [a0, a1], then [b0, b1] (none: b0 > b1),
+    // relative to every row; any_b: some lane has both
+    bool rows_alike = false, any_b = false;
+    int a0 = 0, a1 = 0, b0 = 1, b1 = 0;
+    float apx = pi.x, bpx = pi.x;
+    int acx = 1, bcx = 1;
+    if (HASH == CMAG_HASH_LINEAR && Cells::PADDED) {
+        const int gx = (int)P.grid_size[0], lo = gp.x - cc, hi = gp.x + cc;
+        const bool inside = lo >= 0 && hi < gx;
+        rows_alike = __ballot(!(inside || (gp.x >= 0 && gp.x < gx && 2 * cc + 1 <= gx))) == 0ull;
+        any_b = __ballot(!inside) != 0ull;
+        if (lo < 0) {
+            a0 = lo + gx; a1 = gx - 1; b0 = 0; b1 = hi;
+            if (perx) { apx = pi.x + P.world_size[0]; acx = 0; }
+        } else if (hi >= gx) {
+            a0 = lo; a1 = gx - 1; b0 = 0; b1 = hi - gx;
+            if (perx) { bpx = pi.x - P.world_size[0]; bcx = 2; }
+        } else {
+            a0 = lo; a1 = hi;
+        }
+    }
     // one stencil row (dy, dz); ky, kz: its Morton key parts
     auto row_body = [&](int dy, int dz, uint32_t ky, uint32_t kz) {
         const int nz = gp.z + dz;
@@ -208,6 +241,56 @@ __device__ __forceinline__ void walk_rows(const cmag_params& P, const float4& pi
         const uint32_t row = (HASH == CMAG_HASH_LINEAR)
                                  ? (((uint32_t)nz & gzm) * P.grid_size[1] + ((uint32_t)ny & gym)) * P.grid_size[0]
                                  : (kz | ky);
+        if constexpr (HASH == CMAG_HASH_LINEAR && Cells::PADDED) {
+            // one call of run_pair in the code (it is large): a row that is not
+            // alike comes cell by cell, the sub-cell walk's last walls by themselves
+            auto run = [](uint32_t s, uint32_t e, float px, int code) { return Run{s, e > s ? e - s : 0u, px, code}; };
+            const Run none{0u, 0u, pi.x, 13};
+            const int parts = rows_alike ? (Cells::SUB && any_b ? 2 : 1) : 2 * cc + 1;
+            uint32_t ws = 0, we = 0;
+            for (int part = 0; part < parts; ++part) {
+                Run a = none, b = none;
+                uint32_t s, e;
+                if (!rows_alike) {
+                    const int nx = gp.x + part - cc;
+                    const int sx = perx ? image_shift(nx, P.grid_size[0]) : 0;
+                    const float px = perx ? pi.x - (float)sx * P.world_size[0] : pi.x;
+                    const uint32_t key = row + ((uint32_t)nx & gxm);
+                    const int code = (sx + 1) + code_yz;
+                    if constexpr (Cells::SUB) {
+                        cells.range_sub(key, key, part == 0, part == 2 * cc, sub, s, e, ws, we);
+                        b = run(ws, we, px, code);
+                    } else {
+                        (void)cells.range(key, key, s, e);
+                    }
+                    a = run(s, e, px, code);
+                } else if constexpr (Cells::SUB) {
+                    const bool both = any_b && b0 <= b1;
+                    if (part == 0) {
+                        cells.range_sub(row + (uint32_t)a0, row + (uint32_t)a1, true, !both, sub, s, e, ws, we);
+                        a = run(s, e, pi.x, code_yz + 1);
+                        if (both) {
+                            cells.range_sub(row + (uint32_t)b0, row + (uint32_t)b1, false, true, sub, s, e, ws, we);
+                            b = run(s, e, pi.x, code_yz + 1);
+                        } else {
+                            b = run(ws, we, pi.x, code_yz + 1);
+                            ws = we = 0u;
+                        }
+                    } else {
+                        a = run(ws, we, pi.x, code_yz + 1);
+                    }
+                } else {
+                    (void)cells.range(row + (uint32_t)a0, row + (uint32_t)a1, s, e);
+                    a = run(s, e, apx, acx + code_yz);
+                    if (any_b && b0 <= b1) {
+                        (void)cells.range(row + (uint32_t)b0, row + (uint32_t)b1, s, e);
+                        b = run(s, e, bpx, bcx + code_yz);
+                    }
+                }
+                run_pair(a, b, py, pz, !Cells::SUB && rows_alike);
+            }
+            return;
+        }
         Run a{0u, 0u, pi.x, 13}, b{0u, 0u, pi.x, 13};
         bool have_a = false;
         auto push = [&](uint32_t s, uint32_t e, float px, int code) {
@@ -218,7 +301,7 @@ __device__ __forceinline__ void walk_rows(const cmag_params& P, const float4& pi
             } else if (b.len == 0) {
                 b = r;
             } else {  // a third run in one row (periodic seam with plain Z order, or walls)
-                run_pair(a, b, py, pz);
+                run_pair(a, b, py, pz, false);
                 a = r;
                 b.len = 0;
             }
@@ -261,8 +344,9 @@ __device__ __forceinline__ void walk_rows(const cmag_params& P, const float4& pi
             if (HASH == CMAG_HASH_MORTON) kx = dilated_inc(kx, Mx);
         }
         emit(k0, k1, run_px, (run_sx + 1) + code_yz, run_lo, true);
-        run_pair(a, b, py, pz);
+        run_pair(a, b, py, pz, false);
     };
+    const int zlo = DIM == 2 ? 0 : -cc, zhi = DIM == 2 ? 0 : cc;
     if (FORCE_ORDER && cc == 1) {
         // the force pass's row order (force_row), as its staged blocks take it;
         // the Morton key parts are stepped from the stencil's first row each time
@@ -299,7 +383,7 @@ __device__ __forceinline__ float4 row4(const float4* __restrict__ base, uint32_t
 template <int DIM, int HASH, bool PERIODIC = true, typename Cells, typename C>
 __device__ __forceinline__ void walk_stencil(const cmag_params& P, const float4& pi, const Cell& gp,
                                              const Cells& cells, C&& cand) {
-    walk_rows<DIM, HASH, PERIODIC>(P, pi, gp, cells, [&](const Run& a, const Run& b, float py, float pz) {
+    walk_rows<DIM, HASH, PERIODIC>(P, pi, gp, cells, [&](const Run& a, const Run& b, float py, float pz, bool) {
         const uint32_t total = a.len + b.len;
         for (uint32_t t = 0; t < total; ++t) {
             const bool second = t >= a.len;
@@ -338,38 +422,73 @@ __device__ __forceinline__ void walk_run_sub(const float4* __restrict__ pos, uin
     } while (off < end);
 }
 
+// one row of walk_stencil_pf
+template <bool PADDED, typename C>
+__device__ __forceinline__ void walk_row_pf(const Run& a, const Run& b, float py, float pz,
+                                            const float4* __restrict__ pos, C&& cand) {
+    const uint32_t total = a.len + b.len;
+    if (total == 0) return;
+    const uint32_t off_b = b.s - a.len;
+    auto row = [&](uint32_t t) { return (t >= a.len ? off_b : a.s) + t; };
+    auto visit = [&](uint32_t t, uint32_t j, const float4& pj, bool valid) {
+        const bool second = t >= a.len;
+        cand(j, pj, valid, second ? b.px : a.px, py, pz, second ? b.code : a.code);
+    };
+    const uint32_t last = total - 1u;
+    // padded: up to two rows past the row's last run are read (and flagged)
+    auto next = [&](uint32_t t) { return PADDED ? t : min(t, last); };
+    uint32_t j0 = row(0);
+    float4 p0 = row4(pos, j0);
+    for (uint32_t t = 0; t < total; t += 2) {
+        const uint32_t t1 = next(t + 1u);
+        const uint32_t j1 = row(t1);
+        const float4 p1 = row4(pos, j1);
+        visit(t, j0, p0, true);
+        j0 = row(next(t + 2u));
+        p0 = row4(pos, j0);
+        visit(t1, j1, p1, t + 1u < total);
+    }
+}
+
+// one row's candidates two at a time, for a pass that needs only their
+// positions: f(p0, px0, p1, px1, valid1).  A wave none of whose targets has a
+// second run (no seam near) steps a byte offset; the others choose between
+// their two runs per candidate.  Rows of a System or batch: up to two rows past
+// the last run are read (and flagged).
+template <typename F>
+__device__ __forceinline__ void walk_row_two(const Run& a, const Run& b, const float4* __restrict__ pos, F&& f) {
+    if (__ballot(b.len != 0u) == 0ull) {
+        const char* base = reinterpret_cast<const char*>(pos);
+        const uint32_t end = (a.s + a.len) << 4, end1 = end - 16u;
+        for (uint32_t off = a.s << 4; off < end; off += 32u) {
+            const float4 p0 = *reinterpret_cast<const float4*>(base + off);
+            const float4 p1 = *reinterpret_cast<const float4*>(base + off + 16u);
+            f(p0, a.px, p1, a.px, off < end1);
+        }
+        return;
+    }
+    const uint32_t total = a.len + b.len, off_b = b.s - a.len;
+    for (uint32_t t = 0; t < total; t += 2) {
+        const bool s0 = t >= a.len, s1 = t + 1u >= a.len;
+        const float4 p0 = row4(pos, (s0 ? off_b : a.s) + t);
+        const float4 p1 = row4(pos, (s1 ? off_b : a.s) + t + 1u);
+        f(p0, s0 ? b.px : a.px, p1, s1 ? b.px : a.px, t + 1u < total);
+    }
+}
+
 template <int DIM, int HASH, bool PERIODIC = true, bool FORCE_ORDER = false, typename Cells, typename C>
 __device__ __forceinline__ void walk_stencil_pf(const cmag_params& P, const float4& pi, const Cell& gp,
                                                 const Cells& cells, const float4* __restrict__ pos, C&& cand) {
     if constexpr (Cells::SUB) {
         walk_rows<DIM, HASH, PERIODIC, FORCE_ORDER>(P, pi, gp, cells,
-                                                    [&](const Run& a, const Run& b, float py, float pz) {
+                                                    [&](const Run& a, const Run& b, float py, float pz, bool) {
             walk_run_sub(pos, a.s, a.s + a.len, a.px, py, pz, a.code, cand);
             walk_run_sub(pos, b.s, b.s + b.len, b.px, py, pz, b.code, cand);
         });
         return;
     }
-    walk_rows<DIM, HASH, PERIODIC>(P, pi, gp, cells, [&](const Run& a, const Run& b, float py, float pz) {
-        const uint32_t total = a.len + b.len;
-        if (total == 0) return;
-        const uint32_t last = total - 1u;
-        const uint32_t off_b = b.s - a.len;
-        auto row = [&](uint32_t t) { return (t >= a.len ? off_b : a.s) + t; };
-        auto visit = [&](uint32_t t, uint32_t j, const float4& pj, bool valid) {
-            const bool second = t >= a.len;
-            cand(j, pj, valid, second ? b.px : a.px, py, pz, second ? b.code : a.code);
-        };
-        uint32_t j0 = row(0);
-        float4 p0 = row4(pos, j0);
-        for (uint32_t t = 0; t < total; t += 2) {
-            const uint32_t t1 = min(t + 1u, last);
-            const uint32_t j1 = row(t1);
-            const float4 p1 = row4(pos, j1);
-            visit(t, j0, p0, true);
-            j0 = row(min(t + 2u, last));
-            p0 = row4(pos, j0);
-            visit(t1, j1, p1, t + 1u < total);
-        }
+    walk_rows<DIM, HASH, PERIODIC>(P, pi, gp, cells, [&](const Run& a, const Run& b, float py, float pz, bool) {
+        walk_row_pf<Cells::PADDED>(a, b, py, pz, pos, cand);
     });
 }
 
@@ -816,20 +935,97 @@ __device__ __forceinline__ float density_sum_lookup(const cmag_params& P, const 
     return sum * P.kernel_coeff * P.particle_mass;
 }
 
+// ---- in-range masks of the 2-D channel passes ---------------------------------
+// The density pass tests every candidate; for each target and stencil row that
+// walk_rows hands out whole it keeps a 32-bit mask, bit t set when candidate t of
+// the row lies within 2h (r^2 < 4h^2, the force pass's own test on the same
+// float operations).  The force pass then queues the set bits' candidates, in
+// the walk's order, without loading or testing the others: about 21 (h = 1.3
+// spacings) or 28 (h = 1.5) of 49 on cells of one spacing.  A row of more than
+// 32 candidates is walked.  Layout [row][target], 4 bytes, coalesced; both
+// passes map targets to lanes alike, so a wave that gets its rows whole in one
+// gets them whole in the other.
+constexpr int ROW_MASK_BITS = 32;
+
+// m shifted left, with the comparison's bit below: one compare and one add
+// with carry
+__device__ __forceinline__ uint32_t shift_in_less(uint32_t m, float a, float b) {
+    const uint64_t lt = __ballot(a < b);
+    uint64_t carry;
+    asm("v_addc_co_u32_e64 %0, %1, %0, %0, %2" : "+v"(m), "=s"(carry) : "s"(lt));
+    return m;
+}
+
+// density_sum over whole rows two candidates at a time; with masks, leaving
+// the rows' in-range masks at masks[row * stride + i]
+template <int SYS, int DIM, int HASH, bool MASKS, typename Cells>
+__device__ __forceinline__ float density_sum_rows(const cmag_params& P, const float4& pi,
+                                                  const float4* __restrict__ sortedPos, const Cells& cells,
+                                                  uint32_t* __restrict__ masks, uint32_t i, uint32_t stride) {
+    const Cell gp = grid_pos(P, pi.x, pi.y, pi.z);
+    const float half_inv_h = -0.5f / P.smoothing_radius;
+    const float r2max = 4.0f * P.smoothing_radius * P.smoothing_radius;
+    float sum = 0.0f;
+    uint32_t* out = MASKS ? masks + i : nullptr;
+    walk_rows<DIM, HASH, SYS != CMAG_SYS_DAMBREAK>(P, pi, gp, cells,
+                                                   [&](const Run& a, const Run& b, float py, float pz, bool whole) {
+        uint32_t m = 0;
+        walk_row_two(a, b, sortedPos, [&](const float4& p0, float px0, const float4& p1, float px1, bool valid1) {
+            auto term = [&](float r2) {
+                const float t = fminf(fmaxf(fmaf(half_inv_h, fsqrt(r2), 1.0f), 0.0f), 1.0f);
+                const float t2 = t * t;
+                sum = fmaf(t2 * t2, fmaf(-4.0f, t, 5.0f), sum);
+            };
+            const float ra = norm2(px0 - p0.x, py - p0.y, pz - p0.z);
+            const float rb = valid1 ? norm2(px1 - p1.x, py - p1.y, pz - p1.z) : 1e30f;
+            term(ra);
+            term(rb);
+            if (MASKS) {
+                m = shift_in_less(m, ra, r2max);
+                m = shift_in_less(m, rb, r2max);
+            }
+        });
+        if (MASKS && whole) {
+            // candidate t was shifted in K - 1 - t places from the right, K even
+            const uint32_t total = a.len + b.len, K = (total + 1u) & ~1u;
+            if (total != 0u && total <= (uint32_t)ROW_MASK_BITS) *out = __brev(m) >> (32u - K);
+            else *out = 0u;
+            out += stride;
+        }
+    });
+    return sum * P.kernel_coeff * P.particle_mass;
+}
+
+// pairs (optional): what a neighbour's pair terms need of the density pass,
+// (p / rho, 1 / rho) in the reciprocal the terms use; masks (optional): as above
 template <int SYS, int DIM, int HASH, typename Cells>
 __device__ __forceinline__ void density_body(const cmag_params& P, uint32_t i, float4* __restrict__ measures,
-                                             const float4* __restrict__ sortedPos, const Cells& cells) {
+                                             const float4* __restrict__ sortedPos, const Cells& cells,
+                                             float2* __restrict__ pairs = nullptr,
+                                             uint32_t* __restrict__ masks = nullptr, uint32_t stride = 0) {
     const float4 pi = sortedPos[i];
     float2* m2 = reinterpret_cast<float2*>(measures);
-    if (SYS == CMAG_SYS_POISEUILLE && pi.w == CMAG_PO_WALL) {
-        m2[2 * (size_t)i] = make_float2(P.rest_density, eos(P, P.rest_density));
-        return;
-    }
-    const float dens = density_sum<SYS, DIM, HASH>(P, pi, sortedPos, cells);
-    if (SYS == CMAG_SYS_PERISTALSIS) {
-        measures[i] = make_float4(dens, eos(P, dens), 0.0f, pi.w);
+    const bool rest = SYS == CMAG_SYS_POISEUILLE && pi.w == CMAG_PO_WALL;
+    float dens = 0.0f;
+    if constexpr (Cells::PADDED && !Cells::SUB) {
+        // with masks a wall walks too: the force pass takes it as a target
+        if (SYS != CMAG_SYS_DAMBREAK && DIM == 2 && HASH == CMAG_HASH_LINEAR && masks)
+            dens = density_sum_rows<SYS, DIM, HASH, true>(P, pi, sortedPos, cells, masks, i, stride);
+        else if (!rest)
+            dens = density_sum_rows<SYS, DIM, HASH, false>(P, pi, sortedPos, cells, nullptr, i, stride);
     } else {
-        m2[2 * (size_t)i] = make_float2(dens, eos(P, dens));
+        if (!rest) dens = density_sum<SYS, DIM, HASH>(P, pi, sortedPos, cells);
+    }
+    if (rest) dens = P.rest_density;
+    const float p = eos(P, dens);
+    if (SYS == CMAG_SYS_PERISTALSIS) {
+        measures[i] = make_float4(dens, p, 0.0f, pi.w);
+    } else {
+        m2[2 * (size_t)i] = make_float2(dens, p);
+    }
+    if (SYS != CMAG_SYS_DAMBREAK && pairs) {
+        const float inv = frcp(dens);
+        pairs[i] = make_float2(p * inv, inv);
     }
 }
 
@@ -853,6 +1049,8 @@ __device__ __forceinline__ float3 vel_diff_poiseuille(const cmag_params& P, cons
 template <bool PERIODIC = true>
 __device__ __forceinline__ float3 image_target(const cmag_params& P, const float4& pi, int code) {
     if (!PERIODIC) return make_float3(pi.x, pi.y, pi.z);
+    if ((P.periodic_mask & 6) == 0)  // images along x only: code = 13 + sx
+        return make_float3((P.periodic_mask & 1) ? pi.x - (float)(code - 13) * P.world_size[0] : pi.x, pi.y, pi.z);
     const int sx = code % 3 - 1, sy = (code / 3) % 3 - 1, sz = code / 9 - 1;
     float3 q;
     q.x = (P.periodic_mask & 1) ? pi.x - (float)sx * P.world_size[0] : pi.x;
@@ -927,9 +1125,9 @@ struct ForceSum {
     }
 
     // Poiseuille pressure + Morris viscosity of an in-range neighbour
-    // (poiseuilleFlowKernel.cu:184-270); one reciprocal square root and one
-    // reciprocal per pair; valid = false adds nothing
-    __device__ __forceinline__ void pair(const float3& q, const float4& pj, const float4& mj, const float4& vj,
+    // (poiseuilleFlowKernel.cu:184-270); mj = (p_j / rho_j, 1 / rho_j); one
+    // reciprocal square root per pair; valid = false adds nothing
+    __device__ __forceinline__ void pair(const float3& q, const float4& pj, const float2& mj, const float4& vj,
                                          bool valid = true) {
         const float rx = q.x - pj.x, ry = q.y - pj.y, rz = q.z - pj.z;
         const float r2 = norm2(rx, ry, rz);
@@ -939,8 +1137,8 @@ struct ForceSum {
         const float t = fmaf(-0.5f, qq, 1.0f);
         const float t2 = t * t;
         const float temp = gc * fmaf(t2, t2, -(t2 * t) * fmaf(2.0f, qq, 1.0f));
-        const float inv_dj = frcp(mj.x);
-        const float s = fmaf(mj.y * inv_dj, inv_dj, pterm_i);
+        const float inv_dj = mj.y;
+        const float s = fmaf(mj.x, inv_dj, pterm_i);
         const float3 V = vel_diff_poiseuille(P, vi, pi, vj, pj);
         const float kk = valid ? -m * s * inv_d * temp : 0.0f;
         const float kv = valid ? visc_k * inv_dens * inv_dj * inv_d * temp : 0.0f;
@@ -949,6 +1147,57 @@ struct ForceSum {
         fz += fmaf(kk, rz, kv * V.z);
     }
 };
+
+// the walk of a 2-D channel's force pass: rows that come whole give their
+// in-range candidates from the density pass's masks (the target itself left
+// out), the others are tested by cand
+template <int HASH, int CAP, typename Cells, typename C, typename Q>
+__device__ __forceinline__ void walk_row_masks(const cmag_params& P, uint32_t i, const float4& pi, const Cell& gp,
+                                               const Cells& cells, const float4* __restrict__ pos,
+                                               const uint32_t* __restrict__ masks, uint32_t stride, NbQueue<CAP>& nq,
+                                               C&& cand, Q&& pairs) {
+    const uint32_t* in = masks + i;
+    int left = P.cellcount;  // rows until the target's own
+    walk_rows<2, HASH>(P, pi, gp, cells, [&](const Run& a, const Run& b, float py, float pz, bool whole) {
+        const uint32_t total = a.len + b.len, off_b = b.s - a.len;
+        uint32_t m = 0;
+        if (whole) {
+            m = *in;
+            in += stride;
+            if (left-- == 0) {
+                const uint32_t da = i - a.s, t = da < a.len ? da : i - off_b;
+                m &= ~(t < 32u ? 1u << t : 0u);
+            }
+        }
+        if (!whole || __ballot(total > (uint32_t)ROW_MASK_BITS)) {
+            // no mask, or a long row in some lane: all of them test this one
+            for (uint32_t t = 0; t < total; ++t) {
+                const bool second = t >= a.len;
+                const uint32_t j = (second ? off_b : a.s) + t;
+                cand(j, row4(pos, j), true, second ? b.px : a.px, py, pz, second ? b.code : a.code);
+            }
+            return;
+        }
+        while (m != 0u) {
+            const uint32_t t = (uint32_t)__ffs((int)m) - 1u;
+            m &= m - 1u;
+            const bool second = t >= a.len;
+            nq.push(NbEntry::pack((second ? off_b : a.s) + t, second ? b.code : a.code));
+            if (__ballot(nq.full())) nq.drain(NB_DRAIN, pairs);
+        }
+    });
+}
+
+// (p / rho, 1 / rho) of sorted row j: as the density pass left it (STORED), or
+// from measures, with the same operations
+template <bool STORED>
+__device__ __forceinline__ float2 pair_values(const float2* __restrict__ pairs, const float4* __restrict__ measures,
+                                              uint32_t j) {
+    if (STORED) return *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(pairs) + (j << 3));
+    const float4 m = row4(measures, j);
+    const float inv = frcp(m.x);
+    return make_float2(m.y * inv, inv);
+}
 
 // ---- force passes: two phases per target ------------------------------------
 // Phase 1 walks the stencil and only tests candidates (r^2 < 4h^2), appending
@@ -979,7 +1228,9 @@ __device__ __forceinline__ void force_body(const cmag_params& P, uint32_t i, flo
                                            const uint32_t* __restrict__ index, const Cells& cells, uint32_t n,
                                            uint32_t (*nbl)[64], const LookupPlan* lp = nullptr,
                                            const LookupTables* lt = nullptr,
-                                           const uint2* __restrict__ masks = nullptr, uint32_t stride = 0) {
+                                           const uint2* __restrict__ masks = nullptr, uint32_t stride = 0,
+                                           const float2* __restrict__ pv = nullptr,
+                                           const uint32_t* __restrict__ row_masks = nullptr) {
     const int lane = threadIdx.x & 63;
     constexpr bool PACKED = SYS == CMAG_SYS_DAMBREAK && Cells::SUB;
     auto is_wall = [](float w) { return PACKED ? __float_as_int(w) >= 0 : w != CMAG_DB_FLUID; };
@@ -1015,7 +1266,7 @@ __device__ __forceinline__ void force_body(const cmag_params& P, uint32_t i, flo
                 F.pair_db(q, p1, v1, m1.x, m1.y * i1 * i1, second);
             }
         } else {
-            const float4 m0 = row4(measures, j0), m1 = row4(measures, j1);
+            const float2 m0 = pair_values<Cells::PADDED>(pv, measures, j0), m1 = pair_values<Cells::PADDED>(pv, measures, j1);
             F.pair(image_target(P, pi, NbEntry::code(e0)), p0, m0, v0);
             F.pair(image_target(P, pi, NbEntry::code(e1)), p1, m1, v1, second);
         }
@@ -1142,6 +1393,8 @@ __device__ __forceinline__ void force_body(const cmag_params& P, uint32_t i, flo
         } else {
             walk_stencil_pf<DIM, HASH, false, true>(P, pi, gp, cells, sortedPos, cand);
         }
+    } else if (SYS != CMAG_SYS_DAMBREAK && DIM == 2 && HASH == CMAG_HASH_LINEAR && Cells::PADDED && row_masks) {
+        walk_row_masks<HASH>(P, i, pi, gp, cells, sortedPos, row_masks, stride, nq, cand, pairs);
     } else {
         walk_stencil_pf<DIM, HASH, SYS != CMAG_SYS_DAMBREAK>(P, pi, gp, cells, sortedPos, cand);
     }
@@ -1169,8 +1422,8 @@ struct PeriSum {
         gc = P.grad_coeff;
         visc_k = m * (P.mu + P.mu);
     }
-    // valid = false adds nothing
-    __device__ __forceinline__ void pair(const float3& q, const float4& pj, const float4& mj, const float4& vj,
+    // mj = (p_j / rho_j, 1 / rho_j); valid = false adds nothing
+    __device__ __forceinline__ void pair(const float3& q, const float4& pj, const float2& mj, const float4& vj,
                                          bool valid = true) {
         const float rx = q.x - pj.x, ry = q.y - pj.y, rz = q.z - pj.z;
         const float r2 = norm2(rx, ry, rz);
@@ -1180,9 +1433,9 @@ struct PeriSum {
         const float t = fmaf(-0.5f, qq, 1.0f);
         const float t2 = t * t;
         const float temp = gc * fmaf(t2, t2, -(t2 * t) * fmaf(2.0f, qq, 1.0f));
-        const float inv_dj = frcp(mj.x);
+        const float inv_dj = mj.y;
         if (WANT_PRES) {
-            const float kk = valid ? -m * temp * fmaf(mj.y * inv_dj, inv_dj, pterm_i) * inv_d : 0.0f;
+            const float kk = valid ? -m * temp * fmaf(mj.x, inv_dj, pterm_i) * inv_d : 0.0f;
             px = fmaf(kk, rx, px); py = fmaf(kk, ry, py); pz = fmaf(kk, rz, pz);
         }
         if (WANT_VISC) {
@@ -1197,7 +1450,8 @@ __device__ __forceinline__ void peristalsis_force_body(
     const cmag_params& P, uint32_t i, float4* __restrict__ viscF, float4* __restrict__ presF,
     const float4* __restrict__ measures, const float4* __restrict__ sortedPos,
     const float4* __restrict__ sortedVel, const uint32_t* __restrict__ index, const Cells& cells, uint32_t n,
-    uint32_t (*nbl)[64]) {
+    uint32_t (*nbl)[64], const float2* __restrict__ pv = nullptr, const uint32_t* __restrict__ row_masks = nullptr,
+    uint32_t stride = 0) {
     const int lane = threadIdx.x & 63;
     const float4 pi = sortedPos[i];
     PeriSum<WANT_VISC, WANT_PRES> F(P, pi, WANT_VISC ? sortedVel[i] : make_float4(0.f, 0.f, 0.f, 0.f),
@@ -1208,21 +1462,24 @@ __device__ __forceinline__ void peristalsis_force_body(
     const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
     auto pairs = [&](uint32_t e0, uint32_t e1, bool second) {
         const uint32_t j0 = NbEntry::index(e0), j1 = NbEntry::index(e1);
-        const float4 p0 = row4(sortedPos, j0), m0 = row4(measures, j0);
+        const float2 m0 = pair_values<Cells::PADDED>(pv, measures, j0), m1 = pair_values<Cells::PADDED>(pv, measures, j1);
+        const float4 p0 = row4(sortedPos, j0), p1 = row4(sortedPos, j1);
         const float4 v0 = WANT_VISC ? row4(sortedVel, j0) : zero4;
-        const float4 p1 = row4(sortedPos, j1), m1 = row4(measures, j1);
         const float4 v1 = WANT_VISC ? row4(sortedVel, j1) : zero4;
         F.pair(image_target(P, pi, NbEntry::code(e0)), p0, m0, v0);
         F.pair(image_target(P, pi, NbEntry::code(e1)), p1, m1, v1, second);
     };
 
-    walk_stencil_pf<DIM, HASH>(P, pi, gp, cells, sortedPos,
-                               [&](uint32_t j, const float4& pj, bool valid, float qx, float qy, float qz, int code) {
+    auto cand = [&](uint32_t j, const float4& pj, bool valid, float qx, float qy, float qz, int code) {
         const float rx = qx - pj.x, ry = qy - pj.y, rz = qz - pj.z;
         const float r2 = norm2(rx, ry, rz);
         if (valid && j != i && r2 < r2max) nq.push(NbEntry::pack(j, code));
         if (__ballot(nq.full())) nq.drain(NB_DRAIN, pairs);
-    });
+    };
+    if (DIM == 2 && HASH == CMAG_HASH_LINEAR && Cells::PADDED && row_masks)
+        walk_row_masks<HASH>(P, i, pi, gp, cells, sortedPos, row_masks, stride, nq, cand, pairs);
+    else
+        walk_stencil_pf<DIM, HASH>(P, pi, gp, cells, sortedPos, cand);
     nq.drain(CAP, pairs);
     const uint32_t k = index[i];
     if (k >= n) return;

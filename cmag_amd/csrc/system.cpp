@@ -46,6 +46,10 @@ struct cmag_system {
     static constexpr size_t MASK_WORDS = 18;
     bool use_masks = true;
     uint32_t* masks = nullptr;
+    // channels: what the density pass leaves for the force pass, a neighbour's
+    // pair values and (2-D, linear cells) the in-range masks of every row
+    float* pairs = nullptr;
+    uint32_t* rowMasks = nullptr;
     // the demos' colour buffer (float4 RGBA per particle), made on first use
     float* color = nullptr;
 
@@ -93,7 +97,7 @@ struct cmag_system {
             if (e) (void)hipEventDestroy(e);
         void* bufs[] = {pos, vel, velLF, acc, presF, measures, sortedPos, sortedVel, predicted,
                         hash, index, cellStart, cellEnd, cellFirst,
-                        gaccU, gaccS, gposS, gvelS, grho, dState, posW, velW, indexW, w2r, masks, color};
+                        gaccU, gaccS, gposS, gvelS, grho, dState, posW, velW, indexW, w2r, masks, pairs, rowMasks, color};
         for (void* b : bufs)
             if (b) (void)hipFree(b);
         sort.release();
@@ -106,11 +110,16 @@ struct cmag_system {
         CMAG_HIP_TRY(hipStreamCreate(&own_stream));
         stream = own_stream;
         float** fb[] = {&pos, &vel, &velLF, &acc, &measures, &sortedPos, &sortedVel};
-        for (float** b : fb) CMAG_HIP_TRY(hipMalloc((void**)b, f4));
+        // padding rows: the neighbour walks read up to two rows past a run
+        for (float** b : fb) CMAG_HIP_TRY(hipMalloc((void**)b, f4 + (b == &sortedPos ? 64 : 0)));
         if (P.system == CMAG_SYS_PERISTALSIS) {
             CMAG_HIP_TRY(hipMalloc((void**)&presF, f4));
             CMAG_HIP_TRY(hipMalloc((void**)&predicted, f4));
             CMAG_HIP_TRY(hipMalloc((void**)&dState, sizeof(StepState)));
+        }
+        if (P.system != CMAG_SYS_DAMBREAK) {
+            CMAG_HIP_TRY(hipMalloc((void**)&pairs, f4 / 2));
+            if (row_masks_apply(P)) CMAG_HIP_TRY(hipMalloc((void**)&rowMasks, u * ROW_MASK_ROWS));
         }
         uint32_t** ub[] = {&hash, &index};
         for (uint32_t** b : ub) CMAG_HIP_TRY(hipMalloc((void**)b, u));
@@ -160,7 +169,7 @@ struct cmag_system {
     // and densities of the current state.  For Peristalsis the state record
     // advances on the device on the way (PeristalsisSystem::Update,
     // PeristalsisSystem.cpp:330-343) and the walls are configured when it says so
-    int enqueue_front() {
+    int enqueue_front(bool for_force) {
         // the walk order's entries carry a particle's bucket above its number
         if (subwalk && n >= WALK_MAX_PARTICLES) return fail(CMAG_E_INVALID, "force passes take at most 2^27 particles");
         StepState* st = P.system == CMAG_SYS_PERISTALSIS ? dState : nullptr;
@@ -177,23 +186,24 @@ struct cmag_system {
             CMAG_TRY(launch_density_sub(P, measures, w2r, posW, velW, cellFirst, sort.pre, n, stream,
                                         use_masks ? masks : nullptr));
         else
-            CMAG_TRY(launch_density(P, measures, sortedPos, cellStart, cellEnd, n, stream, cellFirst));
+            CMAG_TRY(launch_density(P, measures, sortedPos, cellStart, cellEnd, n, stream, cellFirst,
+                                    for_force ? pairs : nullptr, for_force ? rowMasks : nullptr));
         return CMAG_OK;
     }
 
     // one update(): hash -> sort -> reorder/cellStart -> density -> forces -> integrate
     int enqueue_step() {
-        CMAG_TRY(enqueue_front());
+        CMAG_TRY(enqueue_front(true));
         CMAG_TRY(mark(CMAG_STAGE_FORCE));
         if (P.system == CMAG_SYS_PERISTALSIS) {
             CMAG_TRY(launch_peristalsis_forces(P, acc, presF, measures, sortedPos, sortedVel, index,
-                                               cellStart, cellEnd, n, stream, cellFirst));
+                                               cellStart, cellEnd, n, stream, cellFirst, pairs, rowMasks));
         } else if (subwalk) {
             CMAG_TRY(launch_force_sub(P, acc, posW, velW, indexW, cellFirst, sort.pre, n, stream,
                                       use_masks ? masks : nullptr));
         } else {
             CMAG_TRY(launch_force(P, acc, measures, sortedPos, sortedVel, index, cellStart, cellEnd, n,
-                                  stream, cellFirst));
+                                  stream, cellFirst, pairs, rowMasks));
         }
         CMAG_TRY(mark(CMAG_STAGE_INTEGRATE));
         CMAG_TRY(launch_integrate(P, pos, vel, velLF, acc, presF, 0.0f, n, stream, dState));
@@ -294,7 +304,7 @@ struct cmag_system {
         invalidate_graph();
         const bool was_timing = timing;
         timing = false;
-        int rc = enqueue_front();
+        int rc = enqueue_front(false);
         timing = was_timing;
         CMAG_TRY(rc);
         CMAG_TRY(launch_integrate_vjp(P, pos, gpos, gvel, gvelLF, gaccU, ggrav_acc, n, stream));
