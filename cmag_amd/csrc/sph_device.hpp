@@ -947,13 +947,11 @@ __device__ __forceinline__ float density_sum_lookup(const cmag_params& P, const 
 // gets them whole in the other.
 constexpr int ROW_MASK_BITS = 32;
 
-// m shifted left, with the comparison's bit below: one compare and one add
-// with carry
+// m shifted left, with the bit a < b below (a >= 0 or NaN): the sign of |a| - b,
+// which is exact, and 0 for a NaN; a subtraction and a funnel shift, and no
+// mask register, which needs wait states between a comparison and its reader
 __device__ __forceinline__ uint32_t shift_in_less(uint32_t m, float a, float b) {
-    const uint64_t lt = __ballot(a < b);
-    uint64_t carry;
-    asm("v_addc_co_u32_e64 %0, %1, %0, %0, %2" : "+v"(m), "=s"(carry) : "s"(lt));
-    return m;
+    return __builtin_amdgcn_alignbit(m, __float_as_uint(__builtin_fabsf(a) - b), 31u);
 }
 
 // density_sum over whole rows two candidates at a time; with masks, leaving
