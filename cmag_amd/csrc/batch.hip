@@ -147,7 +147,7 @@ __global__ __launch_bounds__(256) void batch_force_kernel(const cmag_params* __r
                                                                       index, cells, n, mine);
         else if (P.system == CMAG_SYS_POISEUILLE)
             force_body<CMAG_SYS_POISEUILLE, DIM, HASH, FirstCells, CAP>(P, i, acc, measures, sortedPos, sortedVel,
-                                                                        index, cells, n, mine, nullptr, nullptr,
+                                                                        index, cells, n, mine, nullptr, false,
                                                                         nullptr, n, pairs, mk);
         else
             peristalsis_force_body<DIM, HASH, true, true, FirstCells, CAP>(P, i, acc, presF, measures, sortedPos,

@@ -90,15 +90,16 @@ int launch_density(const cmag_params& P, float* measures, const float* sortedPos
                    const uint32_t* cellFirst = nullptr, float* pairs = nullptr, uint32_t* row_masks = nullptr);
 // sub-cell walk order (DamBreak; the copies and pre from CellSort): density and
 // force over it; density writes the reference-order measures through w2r and
-// leaves -rho (fluid rows) in posW.w and p / rho^2 in velW.w for the force pass
+// leaves, for the force pass, -rho (fluid rows) in posW.w and p / rho^2 times the
+// pair terms' common factor in velW.w; keys: the sorted cell keys
 // masks (optional, 2 * MASK_ROWS words per particle): density leaves the
 // in-range masks of staged blocks there and force reads them
-int launch_density_sub(const cmag_params& P, float* measures, const uint32_t* w2r, float* posW, float* velW,
-                       const uint32_t* cellFirst, const uint32_t* pre, uint32_t n, hipStream_t s,
+int launch_density_sub(const cmag_params& P, float* measures, const uint32_t* keys, const uint32_t* w2r, float* posW,
+                       float* velW, const uint32_t* cellFirst, const uint32_t* pre, uint32_t n, hipStream_t s,
                        uint32_t* masks = nullptr);
 int launch_force_sub(const cmag_params& P, float* acc, const float* posW, const float* velW,
-                     const uint32_t* indexW, const uint32_t* cellFirst, const uint32_t* pre, uint32_t n,
-                     hipStream_t s, const uint32_t* masks = nullptr);
+                     const uint32_t* indexW, const uint32_t* keys, const uint32_t* cellFirst, const uint32_t* pre,
+                     uint32_t n, hipStream_t s, const uint32_t* masks = nullptr);
 int launch_force(const cmag_params& P, float* acc, const float* measures, const float* sortedPos,
                  const float* sortedVel, const uint32_t* index, const uint32_t* cellStart,
                  const uint32_t* cellEnd, uint32_t n, hipStream_t s,

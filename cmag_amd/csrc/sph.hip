@@ -29,7 +29,7 @@ __global__ __launch_bounds__(256) void force_kernel(const cmag_params P, float4*
     const uint32_t i = xcd_block() * blockDim.x + threadIdx.x;
     if (i >= n) return;
     force_body<SYS, DIM, HASH>(P, i, acc, measures, sortedPos, sortedVel, index, cells, n, nbl[threadIdx.x >> 6],
-                               nullptr, nullptr, nullptr, n, pairs, row_masks);
+                               nullptr, false, nullptr, n, pairs, row_masks);
 }
 
 // Peristalsis: pressure and viscous passes; the fused variant produces both
@@ -166,13 +166,14 @@ int launch_force(const cmag_params& P, float* acc, const float* measures, const 
 // and the candidate positions of four stencil rows as well).
 // The result goes to the reference-order row
 // measures[w2r[i]] and, for a fluid row, into the sub-cell copies that the
-// force pass reads: -rho in posW[i].w and p / rho^2 in velW[i].w.  Other threads read
-// posW rows during this pass, but only their x, y, z; a thread writes the w of
-// its own row only, after its walk.
+// force pass reads: -rho in posW[i].w and db_scale p / rho^2 in velW[i].w.
+// Other threads read posW rows during this pass, but only their x, y, z; a
+// thread writes the w of its own row only, after its walk.
 // With masks, staged blocks also leave the in-range masks of their rows for
 // the force pass (masks[r * n + i]).
 template <int DIM, int HASH>
 __global__ __launch_bounds__(256) void density_sub_kernel(const cmag_params P, float4* __restrict__ measures,
+                                                           const uint32_t* __restrict__ keys,
                                                            const uint32_t* __restrict__ w2r, float4* posW,
                                                            float4* velW, const SubCells cells, uint32_t n,
                                                            uint2* __restrict__ masks) {
@@ -182,23 +183,28 @@ __global__ __launch_bounds__(256) void density_sub_kernel(const cmag_params P, f
     const uint32_t i = b0 + threadIdx.x;
     __shared__ RowStage rs;
     __shared__ RowLds rows;
-    const bool staged = stage_lookups<DIM>(P, posW, cells, n, b0, lp, lt);
+    const bool staged = stage_lookups<DIM, HASH>(P, keys, cells, n, b0, lp, lt);
     if (staged) stage_rows<DIM>(lp, lt, posW, rows, rs);
     if (i >= n) return;
     const float4 pi = posW[i];
-    const float dens = !staged ? density_sum<CMAG_SYS_DAMBREAK, DIM, HASH>(P, pi, posW, cells)
-                       : masks ? density_sum_masks<DIM>(P, pi, lp, lt, rs, &rows, posW, masks, i, n)
-                               : density_sum_lookup<DIM>(P, pi, lp, lt, rs, &rows, posW);
+    float dens;
+    if (!staged) {
+        dens = density_sum<CMAG_SYS_DAMBREAK, DIM, HASH>(P, pi, posW, cells);
+    } else {
+        const LookupView v = lookup_view<DIM>(lp, lt, keys[i], key_masks<HASH>(P).x);
+        dens = masks ? density_sum_masks<DIM>(P, pi, v, rs, &rows, posW, masks, i, n)
+                     : density_sum_lookup<DIM>(P, pi, v, rs, &rows, posW);
+    }
     const float p = eos(P, dens);
     reinterpret_cast<float2*>(measures)[2 * (size_t)w2r[i]] = make_float2(dens, p);
     if (pi.w == CMAG_DB_FLUID) {
         reinterpret_cast<float*>(posW)[4 * (size_t)i + 3] = -dens;
-        reinterpret_cast<float*>(velW)[4 * (size_t)i + 3] = p / (dens * dens);
+        reinterpret_cast<float*>(velW)[4 * (size_t)i + 3] = p / (dens * dens) * db_scale(P);
     }
 }
 
-int launch_density_sub(const cmag_params& P, float* measures, const uint32_t* w2r, float* posW, float* velW,
-                       const uint32_t* cellFirst, const uint32_t* pre, uint32_t n, hipStream_t s,
+int launch_density_sub(const cmag_params& P, float* measures, const uint32_t* keys, const uint32_t* w2r, float* posW,
+                       float* velW, const uint32_t* cellFirst, const uint32_t* pre, uint32_t n, hipStream_t s,
                        uint32_t* masks) {
     if (n == 0) return CMAG_OK;
     if (P.system != CMAG_SYS_DAMBREAK) return fail(CMAG_E_INVALID, "the sub-cell walk is DamBreak's");
@@ -207,14 +213,14 @@ int launch_density_sub(const cmag_params& P, float* measures, const uint32_t* w2
     float4* pw = reinterpret_cast<float4*>(posW);
     float4* vw = reinterpret_cast<float4*>(velW);
     uint2* mk = reinterpret_cast<uint2*>(masks);
-    dim3 g(div_up(n, 256)), b(256);
+    const dim3 g(div_up(n, 256)), b(256);
     const bool m = P.hash_order == CMAG_HASH_MORTON;
     if (P.dim == 3) {
-        if (m) hipLaunchKernelGGL((density_sub_kernel<3, 1>), g, b, 0, s, P, m4, w2r, pw, vw, cells, n, mk);
-        else hipLaunchKernelGGL((density_sub_kernel<3, 0>), g, b, 0, s, P, m4, w2r, pw, vw, cells, n, mk);
+        if (m) hipLaunchKernelGGL((density_sub_kernel<3, 1>), g, b, 0, s, P, m4, keys, w2r, pw, vw, cells, n, mk);
+        else hipLaunchKernelGGL((density_sub_kernel<3, 0>), g, b, 0, s, P, m4, keys, w2r, pw, vw, cells, n, mk);
     } else {
-        if (m) hipLaunchKernelGGL((density_sub_kernel<2, 1>), g, b, 0, s, P, m4, w2r, pw, vw, cells, n, mk);
-        else hipLaunchKernelGGL((density_sub_kernel<2, 0>), g, b, 0, s, P, m4, w2r, pw, vw, cells, n, mk);
+        if (m) hipLaunchKernelGGL((density_sub_kernel<2, 1>), g, b, 0, s, P, m4, keys, w2r, pw, vw, cells, n, mk);
+        else hipLaunchKernelGGL((density_sub_kernel<2, 0>), g, b, 0, s, P, m4, keys, w2r, pw, vw, cells, n, mk);
     }
     return check_launch("density_sub_kernel");
 }
@@ -223,29 +229,32 @@ int launch_density_sub(const cmag_params& P, float* measures, const uint32_t* w2
 // its runs through the cell lookups staged in LDS (the same runs as the
 // global walk).  CAP: neighbour queue depth; with the in-range masks only
 // walked rows and blocks without staged lookups queue neighbours, and a
-// shallower queue leaves more LDS to the CU (16M dam break: 4.18 vs 4.29 ms
-// at depth 8 vs 16).  At depth 8 registers are held to 72 a lane so that 7
-// waves share a SIMD (16M dam break: 3.61 ms, against 3.75 ms at 76 registers
-// and 6 waves); at depth 16 the queues' LDS allows fewer waves anyway.
+// shallower queue leaves more LDS to the CU.  What bounds it: the rows gathered
+// for the pair terms (the data-return path of L1 is busy 88 % of the time, the
+// vector units 78 %), 32 B a neighbour.  16M dam break: 3.54 ms with registers
+// held so that six waves share a SIMD, 3.75 ms with seven (a spill inside the
+// pair loop), 3.56 ms with five.
 template <int DIM, int HASH, int CAP>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CAP <= 8 ? 7 : 1, 8))) void force_sub_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CAP <= 8 ? 6 : 1, 8))) void force_sub_kernel(
     const cmag_params P, float4* __restrict__ acc, const float4* __restrict__ posW, const float4* __restrict__ velW,
-    const uint32_t* __restrict__ indexW, const SubCells cells, uint32_t n, const uint2* __restrict__ masks) {
+    const uint32_t* __restrict__ indexW, const uint32_t* __restrict__ keys, const SubCells cells, uint32_t n,
+    const uint2* __restrict__ masks) {
     __shared__ uint32_t nbl[256 / 64][CAP][64];
     __shared__ LookupPlan lp;
     __shared__ LookupTables lt;
     const uint32_t b0 = xcd_block() * blockDim.x;
     const uint32_t i = b0 + threadIdx.x;
-    const bool staged = stage_lookups<DIM>(P, posW, cells, n, b0, lp, lt);
+    const bool staged = stage_lookups<DIM, HASH>(P, keys, cells, n, b0, lp, lt);
     if (i >= n) return;
+    // made in every block, so that the tables stay LDS addresses; used when staged
+    const LookupView v = lookup_view<DIM>(lp, lt, keys[i], key_masks<HASH>(P).x);
     force_body<CMAG_SYS_DAMBREAK, DIM, HASH, SubCells, CAP>(P, i, acc, nullptr, posW, velW, indexW, cells, n,
-                                                            nbl[threadIdx.x >> 6], staged ? &lp : nullptr, &lt,
-                                                            masks, n);
+                                                            nbl[threadIdx.x >> 6], &v, staged, masks, n);
 }
 
 int launch_force_sub(const cmag_params& P, float* acc, const float* posW, const float* velW,
-                     const uint32_t* indexW, const uint32_t* cellFirst, const uint32_t* pre, uint32_t n,
-                     hipStream_t s, const uint32_t* masks) {
+                     const uint32_t* indexW, const uint32_t* keys, const uint32_t* cellFirst, const uint32_t* pre,
+                     uint32_t n, hipStream_t s, const uint32_t* masks) {
     if (n == 0) return CMAG_OK;
     if (n >= (1u << NB_SHIFT_BITS)) return fail(CMAG_E_INVALID, "force passes take at most 2^27 particles");
     if (P.system != CMAG_SYS_DAMBREAK) return fail(CMAG_E_INVALID, "the sub-cell walk is DamBreak's");
@@ -255,12 +264,12 @@ int launch_force_sub(const cmag_params& P, float* acc, const float* posW, const 
         if (masks)
             hipLaunchKernelGGL((force_sub_kernel<D, H, 8>), dim3(div_up(n, 256)), dim3(256), 0, s, P,
                                reinterpret_cast<float4*>(acc), reinterpret_cast<const float4*>(posW),
-                               reinterpret_cast<const float4*>(velW), indexW, cells, n,
+                               reinterpret_cast<const float4*>(velW), indexW, keys, cells, n,
                                reinterpret_cast<const uint2*>(masks));
         else
             hipLaunchKernelGGL((force_sub_kernel<D, H, NB_CAP>), dim3(div_up(n, 256)), dim3(256), 0, s, P,
                                reinterpret_cast<float4*>(acc), reinterpret_cast<const float4*>(posW),
-                               reinterpret_cast<const float4*>(velW), indexW, cells, n, nullptr);
+                               reinterpret_cast<const float4*>(velW), indexW, keys, cells, n, nullptr);
     };
     const bool m = P.hash_order == CMAG_HASH_MORTON;
     using I2 = std::integral_constant<int, 2>;

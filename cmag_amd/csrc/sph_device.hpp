@@ -504,13 +504,10 @@ __device__ __forceinline__ void walk_stencil_pf(const cmag_params& P, const floa
 constexpr int LK_W = 32;
 
 struct LookupPlan {
-    uint32_t key[2][9];  // key of cell cx0 - 1 in each stencil row of each part
-    uint32_t width[2];   // cells per stencil row segment
-    int cx0[2];
-    int ry[2], rz[2];    // each part's row of cells (wrapped)
-    int parts;           // 0: not staged, 1 or 2 rows
-    int split;           // first target (block thread) of the second row
-    int bad;             // a target outside the two rows
+    uint32_t row[2];    // each part's row of cells: the key without its x bits
+    uint32_t x0[2];     // x bits of the key of the part's first target
+    uint32_t width[2];  // cells per stencil row segment
+    int parts;          // 0: not staged, 1 or 2 rows
 };
 
 // part p (width w_p) keeps its stencil rows r at first[f_p + r * (w_p + 1) + c]
@@ -531,15 +528,26 @@ struct LookupView {
     __device__ __forceinline__ const uint4* Pr(int r, uint32_t c) const { return pre + (uint32_t)r * ps + c; }
 };
 
+// the bits of each axis in a cell key; the linear order's are fields, so its
+// keys step by dilated_inc / dilated_dec too
+struct KeyMasks {
+    uint32_t x, y, z;
+};
+template <int HASH>
+__device__ __forceinline__ KeyMasks key_masks(const cmag_params& P) {
+    if (HASH == CMAG_HASH_MORTON) return KeyMasks{P.morton_mask[0], P.morton_mask[1], P.morton_mask[2]};
+    const uint32_t bx = P.grid_bits[0], by = P.grid_bits[1];
+    return KeyMasks{P.grid_size[0] - 1u, (P.grid_size[1] - 1u) << bx, (P.grid_size[2] - 1u) << (bx + by)};
+}
+
+// the view of a target whose cell has this key
 template <int DIM>
-__device__ __forceinline__ LookupView lookup_view(const cmag_params& P, const LookupPlan& lp, const LookupTables& lt,
-                                                  const Cell& gp) {
+__device__ __forceinline__ LookupView lookup_view(const LookupPlan& lp, const LookupTables& lt, uint32_t key,
+                                                  uint32_t xmask) {
     constexpr int R = DIM == 3 ? 9 : 3;
-    const int wx = gp.x & ((int)P.grid_size[0] - 1), wy = gp.y & ((int)P.grid_size[1] - 1),
-              wz = gp.z & ((int)P.grid_size[2] - 1);
-    const int part = (lp.parts == 2 && wy == lp.ry[1] && wz == lp.rz[1]) ? 1 : 0;
+    const int part = (lp.parts == 2 && (key & ~xmask) == lp.row[1]) ? 1 : 0;
     const uint32_t w0 = lp.width[0], w = part ? lp.width[1] : w0;
-    const uint32_t dx = (uint32_t)(wx - lp.cx0[part]);
+    const uint32_t dx = (key & xmask) - lp.x0[part];  // consecutive keys: cells
     LookupView v;
     v.fs = w + 1u;
     v.ps = w;
@@ -548,90 +556,79 @@ __device__ __forceinline__ LookupView lookup_view(const cmag_params& P, const Lo
     return v;
 }
 
-// all threads of the block call this; returns whether the block's lookups are staged
-template <int DIM>
-__device__ __forceinline__ bool stage_lookups(const cmag_params& P, const float4* __restrict__ pos,
+// All threads of the block (whole waves, at most four) call this; returns
+// whether the block's lookups are staged.  keys: the sorted cell keys (a sub-cell row lies in the same cell as
+// the reference-order row of its number).  Everything is found from the keys'
+// bits by every thread at once: one barrier and one pass of loads until the
+// tables are filled.  (When one thread worked out the block's 22 keys from
+// positions, with a division per coordinate and a bit deposit per key, that
+// chain was a tenth of a block's life.)
+template <int DIM, int HASH>
+__device__ __forceinline__ bool stage_lookups(const cmag_params& P, const uint32_t* __restrict__ keys,
                                               const SubCells& cells, uint32_t n, uint32_t b0, LookupPlan& lp,
                                               LookupTables& lt) {
     constexpr int R = DIM == 3 ? 9 : 3;
-    const int gx = (int)P.grid_size[0], gy = (int)P.grid_size[1], gz = (int)P.grid_size[2];
-    const bool eligible = b0 < n && P.cellcount == 1;
-    const uint32_t b1 = eligible ? min(b0 + blockDim.x, n) - 1u : 0u;
-    auto wrapped = [&](uint32_t k) {
-        const float4 p = pos[k];
-        Cell c = grid_pos(P, p.x, p.y, p.z);
-        c.x &= gx - 1;
-        c.y &= gy - 1;
-        c.z &= gz - 1;
-        return c;
+    if (P.cellcount != 1 || b0 >= n) return false;
+    const KeyMasks M = key_masks<HASH>(P);
+    const uint32_t count = min(blockDim.x, n - b0);
+    const uint32_t tid = threadIdx.x;
+    const uint32_t mine = keys[b0 + min(tid, count - 1u)];
+    const uint32_t k0 = keys[b0], k1 = keys[b0 + count - 1u];
+    const uint32_t rowa = k0 & ~M.x, rowb = k1 & ~M.x;
+    const uint32_t prev = tid == 0 ? k0 : keys[b0 + min(tid, count) - 1u];
+    // the only step between rows that may occur is one from the first target's
+    // to the last target's
+    const bool step = (prev & ~M.x) != (mine & ~M.x);
+    __shared__ uint32_t split_key[2];  // x bits of the last target of part 0, the first of part 1
+    if (step) {
+        split_key[0] = prev & M.x;
+        split_key[1] = mine & M.x;
+    }
+    __shared__ uint32_t bad_step[256 / 64];
+    const uint64_t bad = __ballot(step && ((prev & ~M.x) != rowa || (mine & ~M.x) != rowb));
+    if ((tid & 63u) == 0u) bad_step[tid >> 6] = bad != 0u ? 1u : 0u;
+    __syncthreads();
+    for (uint32_t w = 0; w < blockDim.x >> 6; ++w)
+        if (bad_step[w]) return false;
+    const int parts = rowa == rowb ? 1 : 2;
+    // cells x - 1 of the part's first target to x + 1 of its last: inside the
+    // grid and on consecutive keys (x bits that are the key's lowest)
+    auto part_width = [&](uint32_t a, uint32_t b) -> uint32_t {
+        if (a == 0u || b == M.x) return 0u;
+        const uint32_t lo = dilated_dec(a, M.x), hi = dilated_inc(b, M.x);
+        const uint32_t low = M.x & ~(M.x + 1u);  // the run of ones at the bottom
+        if (((lo ^ hi) & ~low) != 0u) return 0u;
+        const uint32_t w = hi - lo + 1u;
+        return w <= (uint32_t)LK_W ? w : 0u;
     };
-    if (threadIdx.x == 0) {
-        lp.split = 0x7fffffff;
-        lp.bad = 0;
-        if (eligible) {
-            const Cell a = wrapped(b0);
-            lp.ry[0] = a.y;
-            lp.rz[0] = a.z;
-        }
-    }
-    __syncthreads();
-    const uint32_t i = b0 + threadIdx.x;
-    Cell mine{0, 0, 0};
-    if (eligible && i <= b1) {
-        mine = wrapped(i);
-        if (mine.y != lp.ry[0] || mine.z != lp.rz[0]) atomicMin(&lp.split, (int)threadIdx.x);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0 && eligible && lp.split != 0x7fffffff) {
-        const Cell c = wrapped(b0 + (uint32_t)lp.split);
-        lp.ry[1] = c.y;
-        lp.rz[1] = c.z;
-    }
-    __syncthreads();
-    if (eligible && i <= b1 && (int)threadIdx.x > lp.split && (mine.y != lp.ry[1] || mine.z != lp.rz[1]))
-        lp.bad = 1;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int parts = 0;
-        if (eligible && !lp.bad) {
-            const int np = lp.split == 0x7fffffff ? 1 : 2;
-            uint32_t wsum = 0;
-            // each part's targets run from cell (ax) to cell (bx) of its row
-            const uint32_t first_t[2] = {b0, np == 2 ? b0 + (uint32_t)lp.split : 0u};
-            const uint32_t last_t[2] = {np == 2 ? b0 + (uint32_t)lp.split - 1u : b1, b1};
-            bool ok = true;
-            for (int pt = 0; pt < np && ok; ++pt) {
-                const Cell a = wrapped(first_t[pt]), b = wrapped(last_t[pt]);
-                const int ax = a.x, bx = b.x, ay = a.y, az = a.z;
-                ok = ax >= 1 && bx >= ax && bx + 1 < gx && bx - ax + 3 <= LK_W;
-                if (!ok) break;
-                const uint32_t width = (uint32_t)(bx - ax) + 3u;
-                wsum += width;
-                ok = wsum <= (uint32_t)LK_W;
-                if (!ok) break;
-                ok = grid_hash(P, bx + 1, ay, az) - grid_hash(P, ax - 1, ay, az) == width - 1u;
-                if (!ok) break;
-                int r = 0;
-                for (int dz = (DIM == 3 ? -1 : 0); dz <= (DIM == 3 ? 1 : 0); ++dz)
-                    for (int dy = -1; dy <= 1; ++dy, ++r) lp.key[pt][r] = grid_hash(P, ax - 1, ay + dy, az + dz);
-                lp.width[pt] = width;
-                lp.cx0[pt] = ax;
-            }
-            if (ok) parts = np;
-        }
+    const uint32_t xa = k0 & M.x, xb = parts == 2 ? split_key[1] : 0u;
+    const uint32_t w0 = part_width(xa, parts == 2 ? split_key[0] : k1 & M.x);
+    const uint32_t w1 = parts == 2 ? part_width(xb, k1 & M.x) : 0u;
+    if (w0 == 0u || (parts == 2 && w1 == 0u) || w0 + w1 > (uint32_t)LK_W) return false;
+    if (tid == 0) {
+        lp.row[0] = rowa;
+        lp.row[1] = rowb;
+        lp.x0[0] = xa;
+        lp.x0[1] = xb;
+        lp.width[0] = w0;
+        lp.width[1] = w1;
         lp.parts = parts;
     }
-    __syncthreads();
-    if (!lp.parts) return false;
     // part 0's entries first, then part 1's; entry t of first[] is t
-    const uint32_t w0 = lp.width[0], w1 = lp.parts == 2 ? lp.width[1] : 0u;
-    const uint32_t n0 = (uint32_t)R * (w0 + 1u), total = n0 + (lp.parts == 2 ? (uint32_t)R * (w1 + 1u) : 0u);
-    for (uint32_t t = threadIdx.x; t < total; t += blockDim.x) {
+    const uint32_t n0 = (uint32_t)R * (w0 + 1u), total = n0 + (parts == 2 ? (uint32_t)R * (w1 + 1u) : 0u);
+    for (uint32_t t = tid; t < total; t += blockDim.x) {
         const uint32_t pt = t >= n0 ? 1u : 0u, loc = pt ? t - n0 : t, w = pt ? w1 : w0;
         const uint32_t r = loc / (w + 1u), c = loc - r * (w + 1u);
-        const uint32_t key = lp.key[pt][r];
-        lt.first[t] = cells.first[key + c];
-        if (c < w) lt.pre[(pt ? (uint32_t)R * w0 : 0u) + r * w + c] = cells.pre[key + c];
+        const uint32_t rk = pt ? rowb : rowa;
+        uint32_t ky = rk & M.y, kz = rk & M.z;
+        const uint32_t iy = r % 3u, iz = DIM == 3 ? r / 3u : 1u;
+        if (iy == 0u) ky = dilated_dec(ky, M.y);
+        else if (iy == 2u) ky = dilated_inc(ky, M.y);
+        if (iz == 0u) kz = dilated_dec(kz, M.z);
+        else if (iz == 2u) kz = dilated_inc(kz, M.z);
+        const uint32_t key = (ky | kz | dilated_dec(pt ? xb : xa, M.x)) + c;
+        lt.first[t] = cells.first[key];
+        if (c < w) lt.pre[(pt ? (uint32_t)R * w0 : 0u) + r * w + c] = cells.pre[key];
     }
     __syncthreads();
     return true;
@@ -640,9 +637,11 @@ __device__ __forceinline__ bool stage_lookups(const cmag_params& P, const float4
 // The density pass also stages candidate rows: after the lookups, the
 // positions of the rows of four stencil rows of cells (r = 3..6: the three of
 // dz = 0 and the first of dz = +1 in 3-D), up to ROW_STAGE_CAP rows, are copied
-// into LDS as (x, y) pairs and z (12 B a row, 16 KB) and read from there.
+// into LDS (12 B a row, 16 KB) and read from there.
 // 16 KB keeps seven blocks per CU; more rows cost more in occupancy than they
-// save in loads, and the force pass has no LDS to spare (its queues take 16 KB).
+// save in loads.  A row's 12 bytes lie together, so one address serves a
+// candidate.  The force pass stages none: its lanes read one row each, at
+// unlike places, and the copies cost it waves.
 constexpr int ROW_STAGE_FIRST = 3, ROW_STAGE_ROWS = 4, ROW_STAGE_CAP = 1365;
 
 struct RowStage {
@@ -650,10 +649,13 @@ struct RowStage {
     int ok;
 };
 
-// ROW_STAGE_CAP + 1 rows: the walk reads one row past a run
+// ROW_STAGE_CAP + 1 rows: the walk reads one row past a run.  12 bytes a row,
+// together, so that one address serves a candidate
 struct RowLds {
-    float2 xy[ROW_STAGE_CAP + 1];
-    float z[ROW_STAGE_CAP + 1];
+    struct Row {
+        float x, y, z;
+    };
+    Row row[ROW_STAGE_CAP + 1];
 };
 
 // all threads of a staged block call this after stage_lookups
@@ -680,30 +682,27 @@ __device__ __forceinline__ void stage_rows(const LookupPlan& lp, const LookupTab
         const int32_t d0 = (int32_t)s + rs.off[k];
         for (uint32_t t = threadIdx.x; t < e - s; t += blockDim.x) {
             const float4 v = pos[s + t];
-            lds.xy[d0 + t] = make_float2(v.x, v.y);
-            lds.z[d0 + t] = v.z;
+            lds.row[d0 + t] = RowLds::Row{v.x, v.y, v.z};
         }
     }
     __syncthreads();
 }
 
-// the candidates of target pi (cell x wx, wrapped) through the staged
+// the candidates of target pi through its view of the staged
 // lookups, as walk_stencil_pf hands them; with ROWS, the stencil rows that
 // stage_rows copied are read from LDS; with FORCE_ORDER, rows in force_row order
 template <int DIM, bool ROWS = false, bool FORCE_ORDER = false, typename C>
-__device__ __forceinline__ void walk_lookup(const cmag_params& P, const float4& pi, const Cell& gp,
-                                            const LookupPlan& lp, const LookupTables& lt,
+__device__ __forceinline__ void walk_lookup(const cmag_params& P, const float4& pi, const LookupView& v,
                                             const float4* __restrict__ pos, C&& cand, const RowStage* rs = nullptr,
                                             const RowLds* lds = nullptr) {
     constexpr int R = DIM == 3 ? 9 : 3;
     const int q = x_sub(P, pi.x);
-    const LookupView v = lookup_view<DIM>(P, lp, lt, gp);
     auto run_lds = [&](uint32_t s, uint32_t e, int32_t off) {
         for (uint32_t j = s; j < e; j += 2u) {
             const int32_t l = (int32_t)j + off;  // in [0, staged rows]
-            const float2 a0 = lds->xy[l], a1 = lds->xy[l + 1];
-            const float4 p0 = make_float4(a0.x, a0.y, lds->z[l], 0.0f);
-            const float4 p1 = make_float4(a1.x, a1.y, lds->z[l + 1], 0.0f);
+            const RowLds::Row a0 = lds->row[l], a1 = lds->row[l + 1];
+            const float4 p0 = make_float4(a0.x, a0.y, a0.z, 0.0f);
+            const float4 p1 = make_float4(a1.x, a1.y, a1.z, 0.0f);
             cand(j, p0, true, pi.x, pi.y, pi.z, 13);
             cand(j + 1u, p1, j + 1u < e, pi.x, pi.y, pi.z, 13);
         }
@@ -734,39 +733,38 @@ __device__ __forceinline__ void walk_lookup(const cmag_params& P, const float4& 
 // or testing those candidates, and walks the walls apart.  Masks are stored
 // row-major, [r][target] (uint2: low word first); a row whose run is longer
 // than MASK_BITS is walked as before.
-// Layout: the run is scanned in pairs (t, t + 1) and each pair shifts two bits
-// in from the right, t's bit above t + 1's, so after the K = ceil(L / 2) pairs
-// of a run of L candidates, candidate t sits at bit 2K - 1 - t (a pair past the
-// run's end adds a zero bit).  Bit-reversed, t sits at 64 - 2K + t.
+// Layout: two words, bit t of the first for candidate t < 32 of the run, bit t
+// of the second for candidate 32 + t.  The scan takes the run's candidates in
+// pairs, the first 32 into one word, the rest into the other: a compare and an
+// add with carry a candidate.  (One 64-bit word shifted by two bits a pair took
+// four and a half, of which v_lshlrev_b64 and the selects most.)
 constexpr int MASK_BITS = 64;
 constexpr int MASK_ROWS = 9;
 
-// the mask bits of run candidates t in [lo, hi) for a run of K2 = 2K <= 64
-// shifted-in candidates (t at bit K2 - 1 - t)
-__device__ __forceinline__ uint64_t mask_bits(uint32_t K2, uint32_t lo, uint32_t hi) {
+// bits [lo, hi), hi <= 64
+__device__ __forceinline__ uint64_t mask_bits(uint32_t lo, uint32_t hi) {
     if (hi <= lo) return 0ull;
     const uint32_t len = hi - lo;
-    const uint64_t ones = len >= 64u ? ~0ull : ((1ull << len) - 1ull);
-    return ones << (K2 - hi);
+    return (len >= 64u ? ~0ull : (1ull << len) - 1ull) << lo;
 }
 
-__device__ __forceinline__ uint64_t mask_shift_in(uint64_t m, float r2a, float r2b, float r2max) {
-    const uint32_t b = (r2a < r2max ? 2u : 0u) | (r2b < r2max ? 1u : 0u);
-    return (m << 2) + (uint64_t)b;
+// m shifted left, with the bit a < b below (a >= 0 or NaN): the sign of |a| - b,
+// which is exact, and 0 for a NaN; a subtraction and a funnel shift, without
+// the wait a comparison's mask needs before it can be read
+__device__ __forceinline__ uint32_t shift_in_less(uint32_t m, float a, float b) {
+    return __builtin_amdgcn_alignbit(m, __float_as_uint(__builtin_fabsf(a) - b), 31u);
 }
 
 // density of the target pi over a staged block's lookups, as
 // density_sum_lookup, writing the in-range masks of its rows' main runs to
 // masks[r * stride + i] (fluid targets only)
 template <int DIM>
-__device__ __forceinline__ float density_sum_masks(const cmag_params& P, const float4& pi, const LookupPlan& lp,
-                                                   const LookupTables& lt, const RowStage& rs, const RowLds* lds,
+__device__ __forceinline__ float density_sum_masks(const cmag_params& P, const float4& pi, const LookupView& v,
+                                                   const RowStage& rs, const RowLds* lds,
                                                    const float4* __restrict__ pos, uint2* __restrict__ masks,
                                                    uint32_t i, uint32_t stride) {
     constexpr int R = DIM == 3 ? 9 : 3;
-    const Cell gp = grid_pos(P, pi.x, pi.y, pi.z);
     const int q = x_sub(P, pi.x);
-    const LookupView v = lookup_view<DIM>(P, lp, lt, gp);
     const float half_inv_h = -0.5f / P.smoothing_radius;
     const float r2max = 4.0f * P.smoothing_radius * P.smoothing_radius;
     // the force pass reads the masks of fluid targets only
@@ -788,47 +786,74 @@ __device__ __forceinline__ float density_sum_masks(const cmag_params& P, const f
         const uint32_t f1 = v.F(r, 2);
         const uint4* c1 = v.Pr(r, 2);
         const uint32_t e = f1 + SubCells::through(c1, q), ws = f1 + SubCells::fluid(c1), we = v.F(r, 3);
-        uint64_t m = 0;
+        uint32_t m0 = 0, m1 = 0;
         const bool in_lds = DIM == 3 && rs.ok && r >= ROW_STAGE_FIRST && r < ROW_STAGE_FIRST + ROW_STAGE_ROWS;
-        if (in_lds) {
-            const int32_t off = rs.off[r - ROW_STAGE_FIRST];
-            for (uint32_t j = s; j < e; j += 2u) {
-                const int32_t l = (int32_t)j + off;  // in [0, staged rows]
-                const float2 a0 = lds->xy[l], a1 = lds->xy[l + 1];
-                const float ra = d2(make_float4(a0.x, a0.y, lds->z[l], 0.0f));
-                const float rb = j + 1u < e ? d2(make_float4(a1.x, a1.y, lds->z[l + 1], 0.0f)) : 1e30f;
+        // two candidates per step; `at` steps through the run by `row` a candidate
+        auto scan = [&](auto at, auto row, auto&& ld) {
+            const auto end = at + (e - s) * row, last = end - row;
+            auto bits = [&](float ra, float rb) {
+                m1 = __builtin_amdgcn_alignbit(m1, m0, 30u);
+                m0 = shift_in_less(shift_in_less(m0, ra, r2max), rb, r2max);
+            };
+            // four at a time, then two
+            for (; at + 2u * row < end; at += 4u * row) {
+                float4 p0, p1, p2, p3;
+                ld(at, p0, p1);
+                ld(at + 2u * row, p2, p3);
+                const float ra = d2(p0), rb = d2(p1), rc = d2(p2);
+                const float rd = at + 2u * row < last ? d2(p3) : 1e30f;
                 term(ra);
                 term(rb);
-                m = mask_shift_in(m, ra, rb, r2max);
+                term(rc);
+                term(rd);
+                bits(ra, rb);
+                bits(rc, rd);
             }
-        } else {
-            // two rows per iteration over a byte offset
-            const char* base = reinterpret_cast<const char*>(pos);
-            auto ld = [&](uint32_t off) { return *reinterpret_cast<const float4*>(base + off); };
-            const uint32_t end = e << 4, end1 = end - 16u;
-            for (uint32_t off = s << 4; off < end; off += 32u) {
-                const float4 p0 = ld(off), p1 = ld(off + 16u);
+            if (at < end) {
+                float4 p0, p1;
+                ld(at, p0, p1);
                 const float ra = d2(p0);
-                const float rb = off < end1 ? d2(p1) : 1e30f;
+                const float rb = at < last ? d2(p1) : 1e30f;
                 term(ra);
                 term(rb);
-                m = mask_shift_in(m, ra, rb, r2max);
+                bits(ra, rb);
             }
+        };
+        if (in_lds) {
+            scan(lds->row + ((int32_t)s + rs.off[r - ROW_STAGE_FIRST]), 1u,
+                 [&](const RowLds::Row* q, float4& p0, float4& p1) {
+                     p0 = make_float4(q[0].x, q[0].y, q[0].z, 0.0f);
+                     p1 = make_float4(q[1].x, q[1].y, q[1].z, 0.0f);
+                 });
+        } else {
+            scan(s << 4, 16u, [&](uint32_t off, float4& p0, float4& p1) {
+                const char* base = reinterpret_cast<const char*>(pos);
+                const RowLds::Row a = *reinterpret_cast<const RowLds::Row*>(base + off);
+                const RowLds::Row b = *reinterpret_cast<const RowLds::Row*>(base + (off + 16u));
+                p0 = make_float4(a.x, a.y, a.z, 0.0f);
+                p1 = make_float4(b.x, b.y, b.z, 0.0f);
+            });
         }
+        // candidate t of K was shifted in K - 1 - t places from the right of m1:m0
+        const uint32_t len = e > s ? e - s : 0u, K = min((len + 1u) & ~1u, (uint32_t)MASK_BITS);
+        const uint64_t m = K ? __builtin_bitreverse64((uint64_t)m1 << 32 | m0) >> (64u - K) : 0ull;
+        uint32_t lo = (uint32_t)m, hi = (uint32_t)(m >> 32);
         // the walls of the run's first two cells are walked by the force pass
         // (every wall of the stencil acts): their bits are cleared
         const uint32_t fx = v.F(r, 1), cxw = SubCells::fluid(v.Pr(r, 1));
-        const uint32_t K2 = (e - s + 1u) & ~1u;
-        if ((f1 - f0) - SubCells::fluid(c0) - cxw != 0u && K2 <= (uint32_t)MASK_BITS)
-            m &= ~(mask_bits(K2, f0 + SubCells::fluid(c0) - s, fx - s) | mask_bits(K2, fx + cxw - s, f1 - s));
-        if (fluid) masks[(size_t)r * stride + i] = make_uint2((uint32_t)m, (uint32_t)(m >> 32));
+        if ((f1 - f0) - SubCells::fluid(c0) - cxw != 0u && len <= (uint32_t)MASK_BITS) {
+            const uint64_t w = mask_bits(f0 + SubCells::fluid(c0) - s, fx - s) | mask_bits(fx + cxw - s, f1 - s);
+            lo &= ~(uint32_t)w;
+            hi &= ~(uint32_t)(w >> 32);
+        }
+        if (fluid) masks[(size_t)r * stride + i] = make_uint2(lo, hi);
         if (in_lds) {
             const int32_t off = rs.off[r - ROW_STAGE_FIRST];
             for (uint32_t j = ws; j < we; j += 2u) {
                 const int32_t l = (int32_t)j + off;
-                const float2 a0 = lds->xy[l], a1 = lds->xy[l + 1];
-                cand(j, make_float4(a0.x, a0.y, lds->z[l], 0.0f), true, 0.f, 0.f, 0.f, 13);
-                cand(j + 1u, make_float4(a1.x, a1.y, lds->z[l + 1], 0.0f), j + 1u < we, 0.f, 0.f, 0.f, 13);
+                const RowLds::Row a0 = lds->row[l], a1 = lds->row[l + 1];
+                cand(j, make_float4(a0.x, a0.y, a0.z, 0.0f), true, 0.f, 0.f, 0.f, 13);
+                cand(j + 1u, make_float4(a1.x, a1.y, a1.z, 0.0f), j + 1u < we, 0.f, 0.f, 0.f, 13);
             }
         } else {
             walk_run_sub(pos, ws, we, pi.x, pi.y, pi.z, 13, cand);
@@ -919,13 +944,12 @@ __device__ __forceinline__ float density_sum(const cmag_params& P, const float4&
 }
 
 template <int DIM>
-__device__ __forceinline__ float density_sum_lookup(const cmag_params& P, const float4& pi, const LookupPlan& lp,
-                                                    const LookupTables& lt, const RowStage& rs, const RowLds* lds,
+__device__ __forceinline__ float density_sum_lookup(const cmag_params& P, const float4& pi, const LookupView& v,
+                                                    const RowStage& rs, const RowLds* lds,
                                                     const float4* __restrict__ pos) {
-    const Cell gp = grid_pos(P, pi.x, pi.y, pi.z);
     const float half_inv_h = -0.5f / P.smoothing_radius;
     float sum = 0.0f;
-    walk_lookup<DIM, true>(P, pi, gp, lp, lt, pos,
+    walk_lookup<DIM, true>(P, pi, v, pos,
                            [&](uint32_t, const float4& pj, bool valid, float px, float py, float pz, int) {
         const float r2 = valid ? norm2(px - pj.x, py - pj.y, pz - pj.z) : 1e30f;
         const float t = fminf(fmaxf(fmaf(half_inv_h, fsqrt(r2), 1.0f), 0.0f), 1.0f);
@@ -946,13 +970,6 @@ __device__ __forceinline__ float density_sum_lookup(const cmag_params& P, const 
 // passes map targets to lanes alike, so a wave that gets its rows whole in one
 // gets them whole in the other.
 constexpr int ROW_MASK_BITS = 32;
-
-// m shifted left, with the bit a < b below (a >= 0 or NaN): the sign of |a| - b,
-// which is exact, and 0 for a NaN; a subtraction and a funnel shift, and no
-// mask register, which needs wait states between a comparison and its reader
-__device__ __forceinline__ uint32_t shift_in_less(uint32_t m, float a, float b) {
-    return __builtin_amdgcn_alignbit(m, __float_as_uint(__builtin_fabsf(a) - b), 31u);
-}
 
 // density_sum over whole rows two candidates at a time; with masks, leaving
 // the rows' in-range masks at masks[row * stride + i]
@@ -1063,14 +1080,20 @@ __device__ __forceinline__ float3 image_target(const cmag_params& P, const float
 // once at the end, so the result does not depend on how the neighbours were
 // staged (list depth, which particles share the wave, lists from the density
 // pass).
+
+// the DamBreak pair terms' common factor (ForceSum::pair_db), 5 m gc / (2h)
+__device__ __forceinline__ float db_scale(const cmag_params& P) {
+    return 2.5f * P.particle_mass * P.grad_coeff / P.smoothing_radius;
+}
+
 template <int SYS>
 struct ForceSum {
     const cmag_params& P;
     float4 pi, vi;
-    float dens, inv_dens, pterm_i, inv_h, m, gc, av_k, av_eps, visc_k, t_k, w_k;
+    float dens, inv_dens, pterm_i, inv_h, m, gc, av_c, av_eps, visc_k, t_k, cterm_i;
     float fx = 0.f, fy = 0.f, fz = 0.f, wx = 0.f, wy = 0.f, wz = 0.f;
 
-    // rho, pterm: the target's density and p / rho^2
+    // rho, pterm: the target's density and p / rho^2 (DamBreak: times db_scale)
     __device__ __forceinline__ ForceSum(const cmag_params& P_, const float4& pi_, const float4& vi_, float rho,
                                         float pterm)
         : P(P_), pi(pi_), vi(vi_) {
@@ -1081,11 +1104,11 @@ struct ForceSum {
         inv_h = 1.0f / h;
         m = P.particle_mass;
         gc = P.grad_coeff;
-        av_k = 2.0f * P.alpha * h * P.soundspeed;  // nu * (rho_i + rho_j)
+        cterm_i = pterm;
+        av_c = -2.0f * P.alpha * h * P.soundspeed * db_scale(P);  // of nu * (rho_i + rho_j)
         av_eps = 0.001f * h * h;
         visc_k = m * (P.mu + P.mu);
         t_k = -0.5f * inv_h;
-        w_k = -5.0f * m * gc;
     }
 
     // Lennard-Jones wall term (DamBreak), fluid_kernel.cu:199-208
@@ -1099,26 +1122,27 @@ struct ForceSum {
     }
 
     // DamBreak pressure + artificial viscosity of an in-range fluid neighbour
-    // (fluid_kernel.cu:210-262) with density rho_j and pterm_j = p_j / rho_j^2.
-    // With t = 1 - q/2 the kernel gradient (1-q/2)^4 - (1-q/2)^3 (2q+1) is
-    // 5 t^3 (t - 1); the -m gc factors fold into one constant.  The viscosity
+    // (fluid_kernel.cu:210-262) with density rho_j and cp_j = db_scale p_j /
+    // rho_j^2.  With t = 1 - q/2 the kernel gradient over the distance,
+    // ((1-q/2)^4 - (1-q/2)^3 (2q+1)) / d = 5 t^3 (t - 1) / d, is -5 t^3 / (2h), so
+    // with the -m gc factors it is db_scale t^3, and db_scale is folded into
+    // the pressure and viscosity terms ahead of the pairs.  The viscosity
     // term is branch-free (min(v.r, 0) makes it +0 for separating pairs), which
     // also keeps rho_j's load with the rest of its row.  One reciprocal square
-    // root and one reciprocal per pair.  valid = false adds +0: the term is
-    // scaled by 0 rather than skipped (a skipped term would move its row loads
-    // into a branch); an invalid entry repeats a valid one, so its values are
-    // finite.
+    // root and one reciprocal per pair.  valid = false adds +0 (the term is
+    // computed and dropped: a skipped term would move its row loads into a
+    // branch).  28 VALU instructions; with the gradient as 5 t^3 (t - 1) and the
+    // constants in the pair it was 33.
     __device__ __forceinline__ void pair_db(const float3& q, const float4& pj, const float4& vj, float rho_j,
-                                            float pterm_j, bool valid = true) {
+                                            float cp_j, bool valid = true) {
         const float rx = q.x - pj.x, ry = q.y - pj.y, rz = q.z - pj.z;
         const float r2 = norm2(rx, ry, rz);
-        const float inv_d = frsq(r2);
-        const float t = fmaf(t_k, r2 * inv_d, 1.0f);
-        const float t3 = t * t * t;
+        const float t = fmaf(t_k, r2 * frsq(r2), 1.0f);
         const float vr = fmaf(vi.z - vj.z, rz, fmaf(vi.y - vj.y, ry, (vi.x - vj.x) * rx));
-        const float av = -av_k * fminf(vr, 0.0f) * frcp((dens + rho_j) * (r2 + av_eps));
-        const float s = (pterm_i + pterm_j) + av;
-        const float kk = s * inv_d * t3 * fmaf(w_k, t, -w_k) * (valid ? 1.0f : 0.0f);
+        const float av = fminf(vr, 0.0f) * frcp((dens + rho_j) * (r2 + av_eps));
+        const float s = fmaf(av_c, av, cterm_i + cp_j);
+        const float k = s * (t * t * t);
+        const float kk = valid ? k : 0.0f;
         fx = fmaf(kk, rx, fx); fy = fmaf(kk, ry, fy); fz = fmaf(kk, rz, fz);
     }
 
@@ -1209,7 +1233,7 @@ __device__ __forceinline__ float2 pair_values(const float2* __restrict__ pairs, 
 // nbl: this wave's queues in LDS, [CAP][64]
 // In the sub-cell walk (Cells::SUB, DamBreak) the row copies carry the
 // density pass's results: a fluid row holds -rho in pos.w, sign bit set (a wall
-// row keeps its type flag, 0..3, sign bit clear) and p / rho^2 in vel.w, so a
+// row keeps its type flag, 0..3, sign bit clear) and db_scale p / rho^2 in vel.w, so a
 // pair term gathers two rows instead of three and measures is not read.
 // With masks (staged blocks of the sub-cell walk), the in-range fluid
 // neighbours of a row whose main run holds at most MASK_BITS candidates come
@@ -1224,8 +1248,7 @@ __device__ __forceinline__ void force_body(const cmag_params& P, uint32_t i, flo
                                            const float4* __restrict__ sortedPos,
                                            const float4* __restrict__ sortedVel,
                                            const uint32_t* __restrict__ index, const Cells& cells, uint32_t n,
-                                           uint32_t (*nbl)[64], const LookupPlan* lp = nullptr,
-                                           const LookupTables* lt = nullptr,
+                                           uint32_t (*nbl)[64], const LookupView* lp = nullptr, bool staged = false,
                                            const uint2* __restrict__ masks = nullptr, uint32_t stride = 0,
                                            const float2* __restrict__ pv = nullptr,
                                            const uint32_t* __restrict__ row_masks = nullptr) {
@@ -1243,27 +1266,33 @@ __device__ __forceinline__ void force_body(const cmag_params& P, uint32_t i, flo
         const float4 mi = measures[i];
         rho_i = mi.x;
         pterm_i = mi.y / (mi.x * mi.x);
+        if (SYS == CMAG_SYS_DAMBREAK) pterm_i *= db_scale(P);
     }
     ForceSum<SYS> F(P, pi, vi, rho_i, pterm_i);
     const Cell gp = grid_pos(P, pi.x, pi.y, pi.z);
     const float r2max = 4.0f * P.smoothing_radius * P.smoothing_radius;
     NbQueue<CAP> nq(nbl, lane);
-    auto pairs = [&](uint32_t e0, uint32_t e1, bool second) {
-        const uint32_t j0 = NbEntry::index(e0), j1 = NbEntry::index(e1);
+    auto pairs = [&](uint32_t j0, uint32_t j1, bool second) {
         const float4 p0 = row4(sortedPos, j0), v0 = row4(sortedVel, j0);
         const float4 p1 = row4(sortedPos, j1), v1 = row4(sortedVel, j1);
-        if (SYS == CMAG_SYS_DAMBREAK) {
-            const float3 q = make_float3(pi.x, pi.y, pi.z);
-            if (PACKED) {
-                F.pair_db(q, p0, v0, -p0.w, v0.w);
-                F.pair_db(q, p1, v1, -p1.w, v1.w, second);
-            } else {
-                const float4 m0 = row4(measures, j0), m1 = row4(measures, j1);
-                const float i0 = frcp(m0.x), i1 = frcp(m1.x);
-                F.pair_db(q, p0, v0, m0.x, m0.y * i0 * i0);
-                F.pair_db(q, p1, v1, m1.x, m1.y * i1 * i1, second);
-            }
+        const float3 q = make_float3(pi.x, pi.y, pi.z);
+        if (PACKED) {
+            F.pair_db(q, p0, v0, -p0.w, v0.w);
+            F.pair_db(q, p1, v1, -p1.w, v1.w, second);
         } else {
+            const float4 m0 = row4(measures, j0), m1 = row4(measures, j1);
+            const float i0 = frcp(m0.x), i1 = frcp(m1.x), sc = db_scale(P);
+            F.pair_db(q, p0, v0, m0.x, m0.y * i0 * i0 * sc);
+            F.pair_db(q, p1, v1, m1.x, m1.y * i1 * i1 * sc, second);
+        }
+    };
+    auto queued_pairs = [&](uint32_t e0, uint32_t e1, bool second) {
+        const uint32_t j0 = NbEntry::index(e0), j1 = NbEntry::index(e1);
+        if constexpr (SYS == CMAG_SYS_DAMBREAK) {
+            pairs(j0, j1, second);
+        } else {
+            const float4 p0 = row4(sortedPos, j0), v0 = row4(sortedVel, j0);
+            const float4 p1 = row4(sortedPos, j1), v1 = row4(sortedVel, j1);
             const float2 m0 = pair_values<Cells::PADDED>(pv, measures, j0), m1 = pair_values<Cells::PADDED>(pv, measures, j1);
             F.pair(image_target(P, pi, NbEntry::code(e0)), p0, m0, v0);
             F.pair(image_target(P, pi, NbEntry::code(e1)), p1, m1, v1, second);
@@ -1281,7 +1310,7 @@ __device__ __forceinline__ void force_body(const cmag_params& P, uint32_t i, flo
                 nq.push(NbEntry::pack(j, code));
             }
         }
-        if (__ballot(nq.full())) nq.drain(NB_DRAIN, pairs);
+        if (__ballot(nq.full())) nq.drain(NB_DRAIN, queued_pairs);
     };
     // a run of wall rows only: every one acts (Lennard-Jones), none is queued
     auto wall_only = [&](uint32_t, const float4& pj, bool valid, float px, float py, float pz, int) {
@@ -1291,10 +1320,10 @@ __device__ __forceinline__ void force_body(const cmag_params& P, uint32_t i, flo
         }
     };
     if constexpr (Cells::SUB) {
-        if (lp && masks) {
+        if (staged && masks) {
             constexpr int R = DIM == 3 ? 9 : 3;
+            const LookupView& v = *lp;
             const int q = x_sub(P, pi.x);
-            const LookupView v = lookup_view<DIM>(P, *lp, *lt, gp);
             // the main run [s, e) of row r: cells x - 1 (from eighth q) to
             // x + 1 (through eighth q)
             auto main_run = [&](int r, uint32_t& s, uint32_t& e) {
@@ -1315,36 +1344,39 @@ __device__ __forceinline__ void force_body(const cmag_params& P, uint32_t i, flo
             auto last_walls = [&](int r) {
                 walk_run_sub(sortedPos, v.F(r, 2) + SubCells::fluid(v.Pr(r, 2)), v.F(r, 3), pi.x, pi.y, pi.z, 13, cand);
             };
-            // row r's mask, bit-reversed: candidate t of the run sits at bit
-            // 64 - 2K + t, i.e. candidate j at bit j - s0; the target's own bit
-            // is cleared
-            auto row_mask = [&](const uint2 w, uint32_t s, uint32_t e, uint32_t& s0) {
-                uint64_t m = __builtin_bitreverse64(((uint64_t)w.y << 32) | w.x);
-                s0 = s - (64u - ((e - s + 1u) & ~1u));
-                const uint32_t d = i - s0;
-                return m & ~(d < 64u ? (1ull << d) : 0ull);
+            // a row's mask without the target's own bit
+            auto row_mask = [&](uint2 w, uint32_t s) {
+                const uint32_t d = i - s;
+                w.x &= ~(d < 32u ? 1u << d : 0u);
+                w.y &= ~(d - 32u < 32u ? 1u << (d - 32u) : 0u);
+                return w;
             };
             // pair terms straight from masks, two neighbours per iteration in
             // walk order (a missing second repeats the first and adds nothing),
-            // without the queue: first mA's bits, then mB's
-            auto mask_pairs = [&](uint64_t mA, uint32_t sA0, uint64_t mB, uint32_t sB0) {
-                // row b's bits follow once row a's are used up
-                auto next = [&]() {
-                    if (mA == 0u) {
-                        mA = mB;
-                        sA0 = sB0;
-                        mB = 0u;
+            // without the queue: the words of row a's mask, then row b's.  A
+            // word at a time keeps the bit arithmetic in 32 bits; an iteration
+            // takes both its neighbours from one word.
+            auto mask_pairs = [&](uint2 a, uint32_t sa, uint2 b, uint32_t sb) {
+                uint32_t m0 = a.x, m1 = a.y, m2 = b.x, m3 = b.y;
+                uint32_t s0 = sa, s1 = sa + 32u, s2 = sb, s3 = sb + 32u;
+                // empty words out of the way: every shift below then finds a
+                // word with bits, or the end
+                if (m2 == 0u) { m2 = m3; s2 = s3; m3 = 0u; }
+                if (m1 == 0u) { m1 = m2; s1 = s2; m2 = m3; s2 = s3; m3 = 0u; }
+                if (m0 == 0u) { m0 = m1; s0 = s1; m1 = m2; s1 = s2; m2 = m3; s2 = s3; m3 = 0u; }
+                while (m0 != 0u) {
+                    const uint32_t j0 = s0 + (uint32_t)__builtin_ctz(m0);
+                    m0 &= m0 - 1u;
+                    const bool two = m0 != 0u;
+                    const uint32_t j1 = two ? s0 + (uint32_t)__builtin_ctz(m0) : j0;
+                    m0 &= m0 - 1u;  // 0 stays 0
+                    if (m0 == 0u) {
+                        m0 = m1; s0 = s1;
+                        m1 = m2; s1 = s2;
+                        m2 = m3; s2 = s3;
+                        m3 = 0u;
                     }
-                };
-                next();
-                while (mA != 0u) {
-                    const uint32_t j0 = sA0 + (uint32_t)__builtin_ctzll(mA);
-                    mA &= mA - 1u;
-                    const bool two = mA != 0u;
-                    const uint32_t j1 = two ? sA0 + (uint32_t)__builtin_ctzll(mA) : j0;
-                    if (two) mA &= mA - 1u;
-                    next();
-                    pairs(NbEntry::pack(j0, 13), NbEntry::pack(j1, 13), two);
+                    pairs(j0, j1, two);
                 }
             };
             // rows in force_row order, two at a time (the centre row alone)
@@ -1353,15 +1385,16 @@ __device__ __forceinline__ void force_body(const cmag_params& P, uint32_t i, flo
                 // both masks are loaded ahead of the walls (a walked row's is not used)
                 const uint2 wa = masks[(size_t)ra * stride + i];
                 const uint2 wb = rb >= 0 ? masks[(size_t)rb * stride + i] : make_uint2(0u, 0u);
-                uint32_t s, e, sA0 = 0u, sB0 = 0u;
-                uint64_t mA = 0u, mB = 0u;
+                uint32_t s, e, sa = 0u, sb = 0u;
+                uint2 mA = make_uint2(0u, 0u), mB = mA;
                 main_run(ra, s, e);
                 const bool walk_a = e - s > (uint32_t)MASK_BITS;
                 if (walk_a) {
                     walk_run_sub(sortedPos, s, e, pi.x, pi.y, pi.z, 13, cand);
                 } else {
                     run_walls(ra);
-                    mA = row_mask(wa, s, e, sA0);
+                    mA = row_mask(wa, s);
+                    sa = s;
                 }
                 last_walls(ra);
                 if (rb >= 0) {
@@ -1369,34 +1402,35 @@ __device__ __forceinline__ void force_body(const cmag_params& P, uint32_t i, flo
                     if (e - s > (uint32_t)MASK_BITS) {
                         // row a's pair terms come before the ones row b queues
                         if (!walk_a) {
-                            if (nq.count != 0) nq.drain(CAP, pairs);
-                            mask_pairs(mA, sA0, 0u, 0u);
-                            mA = 0u;
+                            if (nq.count != 0) nq.drain(CAP, queued_pairs);
+                            mask_pairs(mA, sa, make_uint2(0u, 0u), 0u);
+                            mA = make_uint2(0u, 0u);
                         }
                         walk_run_sub(sortedPos, s, e, pi.x, pi.y, pi.z, 13, cand);
                     } else {
                         run_walls(rb);
-                        mB = row_mask(wb, s, e, sB0);
+                        mB = row_mask(wb, s);
+                        sb = s;
                     }
                     last_walls(rb);
                 }
-                if (__ballot((mA | mB) != 0u)) {
+                if (__ballot((mA.x | mA.y | mB.x | mB.y) != 0u)) {
                     // neighbours queued by earlier walked rows come first
-                    if (__ballot(nq.count != 0)) nq.drain(CAP, pairs);
-                    mask_pairs(mA, sA0, mB, sB0);
+                    if (__ballot(nq.count != 0)) nq.drain(CAP, queued_pairs);
+                    mask_pairs(mA, sa, mB, sb);
                 }
             }
-        } else if (lp) {
-            walk_lookup<DIM, false, true>(P, pi, gp, *lp, *lt, sortedPos, cand);
+        } else if (staged) {
+            walk_lookup<DIM, false, true>(P, pi, *lp, sortedPos, cand);
         } else {
             walk_stencil_pf<DIM, HASH, false, true>(P, pi, gp, cells, sortedPos, cand);
         }
     } else if (SYS != CMAG_SYS_DAMBREAK && DIM == 2 && HASH == CMAG_HASH_LINEAR && Cells::PADDED && row_masks) {
-        walk_row_masks<HASH>(P, i, pi, gp, cells, sortedPos, row_masks, stride, nq, cand, pairs);
+        walk_row_masks<HASH>(P, i, pi, gp, cells, sortedPos, row_masks, stride, nq, cand, queued_pairs);
     } else {
         walk_stencil_pf<DIM, HASH, SYS != CMAG_SYS_DAMBREAK>(P, pi, gp, cells, sortedPos, cand);
     }
-    nq.drain(CAP, pairs);
+    nq.drain(CAP, queued_pairs);
     const uint32_t k = index[i];
     if (k < n) acc[k] = make_float4(F.fx + F.wx, F.fy + F.wy, F.fz + F.wz, 0.0f);
 }

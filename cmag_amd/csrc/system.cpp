@@ -183,7 +183,7 @@ struct cmag_system {
                               subwalk ? &rows : nullptr, stream));
         CMAG_TRY(mark(CMAG_STAGE_DENSITY));
         if (subwalk)
-            CMAG_TRY(launch_density_sub(P, measures, w2r, posW, velW, cellFirst, sort.pre, n, stream,
+            CMAG_TRY(launch_density_sub(P, measures, hash, w2r, posW, velW, cellFirst, sort.pre, n, stream,
                                         use_masks ? masks : nullptr));
         else
             CMAG_TRY(launch_density(P, measures, sortedPos, cellStart, cellEnd, n, stream, cellFirst,
@@ -199,7 +199,7 @@ struct cmag_system {
             CMAG_TRY(launch_peristalsis_forces(P, acc, presF, measures, sortedPos, sortedVel, index,
                                                cellStart, cellEnd, n, stream, cellFirst, pairs, rowMasks));
         } else if (subwalk) {
-            CMAG_TRY(launch_force_sub(P, acc, posW, velW, indexW, cellFirst, sort.pre, n, stream,
+            CMAG_TRY(launch_force_sub(P, acc, posW, velW, indexW, hash, cellFirst, sort.pre, n, stream,
                                       use_masks ? masks : nullptr));
         } else {
             CMAG_TRY(launch_force(P, acc, measures, sortedPos, sortedVel, index, cellStart, cellEnd, n,
