@@ -129,7 +129,8 @@ __global__ __launch_bounds__(256) void batch_force_kernel(const cmag_params* __r
                                                           const uint32_t* __restrict__ index,
                                                           const uint32_t* __restrict__ cellFirst,
                                                           const float2* __restrict__ pairs,
-                                                          const uint32_t* __restrict__ masks, uint32_t n) {
+                                                          const uint32_t* __restrict__ masks, uint32_t n,
+                                                          const StepArrays arrays) {
     __shared__ uint32_t nbl[256 / 64][CAP][64];
     uint32_t(*mine)[64] = nbl[threadIdx.x >> 6];
     uint32_t t0, t1;
@@ -142,17 +143,20 @@ __global__ __launch_bounds__(256) void batch_force_kernel(const cmag_params* __r
         const cmag_params& P = params[tile.x];
         const FirstCells cells{cellFirst + I.cell0};
         const uint32_t* const mk = masks && row_masks_apply(P) ? masks : nullptr;
+        StepArrays step = arrays;
+        step.state += tile.x;
         if (P.system == CMAG_SYS_DAMBREAK)
             force_body<CMAG_SYS_DAMBREAK, DIM, HASH, FirstCells, CAP>(P, i, acc, measures, sortedPos, sortedVel,
-                                                                      index, cells, n, mine);
+                                                                      index, cells, n, mine, nullptr, false,
+                                                                      nullptr, n, nullptr, nullptr, step);
         else if (P.system == CMAG_SYS_POISEUILLE)
             force_body<CMAG_SYS_POISEUILLE, DIM, HASH, FirstCells, CAP>(P, i, acc, measures, sortedPos, sortedVel,
                                                                         index, cells, n, mine, nullptr, false,
-                                                                        nullptr, n, pairs, mk);
+                                                                        nullptr, n, pairs, mk, step);
         else
             peristalsis_force_body<DIM, HASH, true, true, FirstCells, CAP>(P, i, acc, presF, measures, sortedPos,
                                                                            sortedVel, index, cells, n, mine, pairs, mk,
-                                                                           n);
+                                                                           n, step);
     }
 }
 
@@ -318,13 +322,13 @@ struct cmag_batch {
     }
 
     template <int DIM, int HASH>
-    int launch_force_cap(dim3 g, dim3 b) {
+    int launch_force_cap(dim3 g, dim3 b, const StepArrays& step) {
         auto f4 = [](float* q) { return reinterpret_cast<float4*>(q); };
         auto c4 = [](const float* q) { return reinterpret_cast<const float4*>(q); };
 #define CMAG_BATCH_FORCE(CAP)                                                                              \
     hipLaunchKernelGGL((batch_force_kernel<DIM, HASH, CAP>), g, b, 0, stream, dP, dI, dTiles, numTiles,     \
                        f4(acc), f4(presF), c4(measures), c4(sortedPos), c4(sortedVel), index, cellFirst,      \
-                       reinterpret_cast<const float2*>(pairs), rowMasks, n)
+                       reinterpret_cast<const float2*>(pairs), rowMasks, n, step)
         if (tune.nb_cap == 8) CMAG_BATCH_FORCE(8);
         else if (tune.nb_cap == 32) CMAG_BATCH_FORCE(32);
         else CMAG_BATCH_FORCE(16);
@@ -333,13 +337,13 @@ struct cmag_batch {
     }
 
     template <int DIM, int HASH>
-    int launch_passes(dim3 g, dim3 b) {
+    int launch_passes(dim3 g, dim3 b, const StepArrays& step) {
         hipLaunchKernelGGL((batch_density_kernel<DIM, HASH>), g, b, 0, stream, dP, dI, dTiles, numTiles,
                            reinterpret_cast<float4*>(measures), reinterpret_cast<const float4*>(sortedPos),
                            cellFirst, reinterpret_cast<float2*>(pairs), rowMasks, n);
         CMAG_TRY(check_launch("batch_density_kernel"));
         CMAG_TRY(mark(CMAG_STAGE_FORCE));
-        return launch_force_cap<DIM, HASH>(g, b);
+        return launch_force_cap<DIM, HASH>(g, b, step);
     }
 
     // one step of every instance
@@ -356,19 +360,26 @@ struct cmag_batch {
         CMAG_TRY(mark(CMAG_STAGE_REORDER));
         CMAG_TRY(sort.reorder(pos, velLF, cellFirst, hash, index, cellEnd, sortedPos, sortedVel, nullptr, stream));
         CMAG_TRY(mark(CMAG_STAGE_DENSITY));
+        // the force pass integrates its targets, or (stage timing on) the two run apart
+        StepArrays step{nullptr, nullptr, nullptr, dS};
+        if (!timing)
+            step = StepArrays{reinterpret_cast<float4*>(pos), reinterpret_cast<float4*>(vel),
+                              reinterpret_cast<float4*>(velLF), dS};
         if (dim == 3) {
-            if (hash_order == CMAG_HASH_MORTON) CMAG_TRY((launch_passes<3, 1>(g, b)));
-            else CMAG_TRY((launch_passes<3, 0>(g, b)));
+            if (hash_order == CMAG_HASH_MORTON) CMAG_TRY((launch_passes<3, 1>(g, b, step)));
+            else CMAG_TRY((launch_passes<3, 0>(g, b, step)));
         } else {
-            if (hash_order == CMAG_HASH_MORTON) CMAG_TRY((launch_passes<2, 1>(g, b)));
-            else CMAG_TRY((launch_passes<2, 0>(g, b)));
+            if (hash_order == CMAG_HASH_MORTON) CMAG_TRY((launch_passes<2, 1>(g, b, step)));
+            else CMAG_TRY((launch_passes<2, 0>(g, b, step)));
         }
         CMAG_TRY(mark(CMAG_STAGE_INTEGRATE));
-        hipLaunchKernelGGL(batch_integrate_kernel, g, b, 0, stream, dP, dI, dS, dTiles, numTiles,
-                           reinterpret_cast<float4*>(pos), reinterpret_cast<float4*>(vel),
-                           reinterpret_cast<float4*>(velLF), reinterpret_cast<const float4*>(acc),
-                           reinterpret_cast<const float4*>(presF));
-        CMAG_TRY(check_launch("batch_integrate_kernel"));
+        if (!step.pos) {
+            hipLaunchKernelGGL(batch_integrate_kernel, g, b, 0, stream, dP, dI, dS, dTiles, numTiles,
+                               reinterpret_cast<float4*>(pos), reinterpret_cast<float4*>(vel),
+                               reinterpret_cast<float4*>(velLF), reinterpret_cast<const float4*>(acc),
+                               reinterpret_cast<const float4*>(presF));
+            CMAG_TRY(check_launch("batch_integrate_kernel"));
+        }
         CMAG_TRY(mark(CMAG_NUM_STAGES));
         if (timing) pending = true;
         return CMAG_OK;

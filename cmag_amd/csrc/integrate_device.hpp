@@ -31,15 +31,14 @@ __device__ __forceinline__ float wall_vy(const cmag_params& P, float x, float w,
     return w > 0.0f ? d : -d;
 }
 
-// one particle of integrate; is_config is the Peristalsis boundary-configuration flag
+// one particle of integrate, its position p, the w of its leapfrog velocity and
+// its accelerations in hand; is_config is the Peristalsis boundary-configuration flag
 template <int SYS>
-__device__ __forceinline__ void integrate_body(const cmag_params& P, uint32_t i, float4* __restrict__ pos,
-                                               float4* __restrict__ vel, float4* __restrict__ velLF,
-                                               const float4* __restrict__ acc,
-                                               const float4* __restrict__ presF, float wave_time,
-                                               int is_config) {
+__device__ __forceinline__ void integrate_row(const cmag_params& P, uint32_t i, const float4& p, float lw,
+                                              const float4& a, const float4& pr, float4* __restrict__ pos,
+                                              float4* __restrict__ vel, float4* __restrict__ velLF, float wave_time,
+                                              int is_config) {
 #pragma clang fp contract(off)
-    const float4 p = pos[i];
     if (SYS == CMAG_SYS_DAMBREAK && p.w != CMAG_DB_FLUID) return;
     if (SYS == CMAG_SYS_POISEUILLE && p.w == CMAG_PO_WALL) return;
     if (SYS == CMAG_SYS_PERISTALSIS && p.w != 0.0f) {
@@ -48,17 +47,14 @@ __device__ __forceinline__ void integrate_body(const cmag_params& P, uint32_t i,
         if (P.wall_velocity) {
             const float vy = wall_vy(P, p.x, p.w, P.amplitude, wave_time);
             vel[i] = make_float4(0.0f, vy, 0.0f, vel[i].w);
-            velLF[i] = make_float4(0.0f, vy, 0.0f, velLF[i].w);
+            velLF[i] = make_float4(0.0f, vy, 0.0f, lw);
         }
         return;
     }
     const float dt = P.delta_time;
     const float4 v = vel[i];
-    const float4 a = acc[i];
-    const float4 l = velLF[i];
     float ax = P.gravity[0] + a.x, ay = P.gravity[1] + a.y, az = P.gravity[2] + a.z;
     if (SYS == CMAG_SYS_PERISTALSIS) {
-        const float4 pr = presF[i];
         ax += pr.x; ay += pr.y; az += pr.z;
     }
     float nx = v.x + ax * dt, ny = v.y + ay * dt, nz = v.z + az * dt;
@@ -80,7 +76,21 @@ __device__ __forceinline__ void integrate_body(const cmag_params& P, uint32_t i,
     }
     pos[i] = make_float4(px, py, pz, p.w);
     vel[i] = make_float4(nx, ny, nz, v.w);
-    velLF[i] = make_float4(lx, ly, lz, l.w);
+    velLF[i] = make_float4(lx, ly, lz, lw);
+}
+
+// the same from the arrays
+template <int SYS>
+__device__ __forceinline__ void integrate_body(const cmag_params& P, uint32_t i, float4* __restrict__ pos,
+                                               float4* __restrict__ vel, float4* __restrict__ velLF,
+                                               const float4* __restrict__ acc,
+                                               const float4* __restrict__ presF, float wave_time,
+                                               int is_config) {
+    const float4 p = pos[i];
+    if (SYS == CMAG_SYS_DAMBREAK && p.w != CMAG_DB_FLUID) return;
+    if (SYS == CMAG_SYS_POISEUILLE && p.w == CMAG_PO_WALL) return;
+    const float4 pr = SYS == CMAG_SYS_PERISTALSIS ? presF[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    integrate_row<SYS>(P, i, p, velLF[i].w, acc[i], pr, pos, vel, velLF, wave_time, is_config);
 }
 
 }  // namespace cmag

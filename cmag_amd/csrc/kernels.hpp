@@ -85,6 +85,12 @@ __host__ __device__ inline bool row_masks_apply(const cmag_params& P) {
     return P.dim == 2 && P.system != CMAG_SYS_DAMBREAK && P.hash_order == CMAG_HASH_LINEAR &&
            2 * P.cellcount + 1 <= ROW_MASK_ROWS;
 }
+// where a step's force pass integrates its targets (in place, at their particle
+// numbers); pos null: it only writes the accelerations
+struct StepArrays {
+    float4 *pos = nullptr, *vel = nullptr, *velLF = nullptr;
+    const StepState* state = nullptr;  // Peristalsis: the time record(s)
+};
 int launch_density(const cmag_params& P, float* measures, const float* sortedPos,
                    const uint32_t* cellStart, const uint32_t* cellEnd, uint32_t n, hipStream_t s,
                    const uint32_t* cellFirst = nullptr, float* pairs = nullptr, uint32_t* row_masks = nullptr);
@@ -104,12 +110,12 @@ int launch_force(const cmag_params& P, float* acc, const float* measures, const 
                  const float* sortedVel, const uint32_t* index, const uint32_t* cellStart,
                  const uint32_t* cellEnd, uint32_t n, hipStream_t s,
                  const uint32_t* cellFirst = nullptr, const float* pairs = nullptr,
-                 const uint32_t* row_masks = nullptr);
+                 const uint32_t* row_masks = nullptr, const StepArrays& step = {});
 int launch_peristalsis_forces(const cmag_params& P, float* viscF, float* presF, const float* measures,
                               const float* sortedPos, const float* sortedVel, const uint32_t* index,
                               const uint32_t* cellStart, const uint32_t* cellEnd, uint32_t n,
                               hipStream_t s, const uint32_t* cellFirst = nullptr, const float* pairs = nullptr,
-                              const uint32_t* row_masks = nullptr);
+                              const uint32_t* row_masks = nullptr, const StepArrays& step = {});
 int launch_pressure_force(const cmag_params& P, float* presF, const float* measures,
                           const float* sortedPos, const uint32_t* index, const uint32_t* cellStart,
                           const uint32_t* cellEnd, uint32_t n, hipStream_t s);

@@ -24,12 +24,12 @@ __global__ __launch_bounds__(256) void force_kernel(const cmag_params P, float4*
                                                      const float4* __restrict__ sortedVel,
                                                      const uint32_t* __restrict__ index, const Cells cells,
                                                      uint32_t n, const float2* __restrict__ pairs,
-                                                     const uint32_t* __restrict__ row_masks) {
+                                                     const uint32_t* __restrict__ row_masks, const StepArrays step) {
     __shared__ uint32_t nbl[256 / 64][NB_CAP][64];
     const uint32_t i = xcd_block() * blockDim.x + threadIdx.x;
     if (i >= n) return;
     force_body<SYS, DIM, HASH>(P, i, acc, measures, sortedPos, sortedVel, index, cells, n, nbl[threadIdx.x >> 6],
-                               nullptr, false, nullptr, n, pairs, row_masks);
+                               nullptr, false, nullptr, n, pairs, row_masks, step);
 }
 
 // Peristalsis: pressure and viscous passes; the fused variant produces both
@@ -39,13 +39,13 @@ __global__ __launch_bounds__(256) void peristalsis_force_kernel(
     const cmag_params P, float4* __restrict__ viscF, float4* __restrict__ presF,
     const float4* __restrict__ measures, const float4* __restrict__ sortedPos,
     const float4* __restrict__ sortedVel, const uint32_t* __restrict__ index, const Cells cells,
-    uint32_t n, const float2* __restrict__ pairs, const uint32_t* __restrict__ row_masks) {
+    uint32_t n, const float2* __restrict__ pairs, const uint32_t* __restrict__ row_masks, const StepArrays step) {
     __shared__ uint32_t nbl[256 / 64][NB_CAP][64];
     const uint32_t i = xcd_block() * blockDim.x + threadIdx.x;
     if (i >= n) return;
     peristalsis_force_body<DIM, HASH, WANT_VISC, WANT_PRES>(P, i, viscF, presF, measures, sortedPos, sortedVel,
                                                             index, cells, n, nbl[threadIdx.x >> 6], pairs, row_masks,
-                                                            n);
+                                                            n, step);
 }
 
 // in-range neighbours (j != i, r^2 < 4h^2) of each sorted particle: the pair
@@ -126,30 +126,30 @@ struct ForceGo {
     template <typename Cells>
     static void run(const cmag_params& P, float* acc, const float* measures, const float* sortedPos,
                     const float* sortedVel, const uint32_t* index, const Cells& cells, uint32_t n,
-                    const float* pairs, const uint32_t* row_masks, hipStream_t s) {
+                    const float* pairs, const uint32_t* row_masks, const StepArrays& step, hipStream_t s) {
         if constexpr (SYS != CMAG_SYS_PERISTALSIS)
             hipLaunchKernelGGL((force_kernel<SYS, DIM, H, Cells>), dim3(div_up(n, 256)), dim3(256), 0, s, P,
                                reinterpret_cast<float4*>(acc), reinterpret_cast<const float4*>(measures),
                                reinterpret_cast<const float4*>(sortedPos),
                                reinterpret_cast<const float4*>(sortedVel), index, cells, n,
-                               reinterpret_cast<const float2*>(pairs), row_masks);
+                               reinterpret_cast<const float2*>(pairs), row_masks, step);
     }
     static void go(const cmag_params& P, float* acc, const float* measures, const float* sortedPos,
                    const float* sortedVel, const uint32_t* index, const uint32_t* cellStart,
                    const uint32_t* cellEnd, const uint32_t* cellFirst, uint32_t n, const float* pairs,
-                   const uint32_t* row_masks, hipStream_t s) {
+                   const uint32_t* row_masks, const StepArrays& step, hipStream_t s) {
         if (cellFirst)
-            run(P, acc, measures, sortedPos, sortedVel, index, FirstCells{cellFirst}, n, pairs, row_masks, s);
+            run(P, acc, measures, sortedPos, sortedVel, index, FirstCells{cellFirst}, n, pairs, row_masks, step, s);
         else
             run(P, acc, measures, sortedPos, sortedVel, index, RefCells{cellStart, cellEnd, n}, n, nullptr, nullptr,
-                s);
+                StepArrays{}, s);
     }
 };
 
 int launch_force(const cmag_params& P, float* acc, const float* measures, const float* sortedPos,
                  const float* sortedVel, const uint32_t* index, const uint32_t* cellStart,
                  const uint32_t* cellEnd, uint32_t n, hipStream_t s, const uint32_t* cellFirst, const float* pairs,
-                 const uint32_t* row_masks) {
+                 const uint32_t* row_masks, const StepArrays& step) {
     if (n == 0) return CMAG_OK;
     if (n >= (1u << NB_SHIFT_BITS)) return fail(CMAG_E_INVALID, "force passes take at most 2^27 particles");
     if (P.system == CMAG_SYS_PERISTALSIS)
@@ -157,7 +157,7 @@ int launch_force(const cmag_params& P, float* acc, const float* measures, const 
     if (cellFirst && P.system != CMAG_SYS_DAMBREAK && !pairs)
         return fail(CMAG_E_INVALID, "the force pass over compact offsets takes the density pass's pair values");
     dispatch3<ForceGo>(P, P, acc, measures, sortedPos, sortedVel, index, cellStart, cellEnd, cellFirst, n, pairs,
-                       row_masks && row_masks_apply(P) ? row_masks : nullptr, s);
+                       row_masks && row_masks_apply(P) ? row_masks : nullptr, step, s);
     return check_launch("force_kernel");
 }
 
@@ -285,13 +285,13 @@ template <bool V, bool PR, typename Cells>
 static void go_peri_cells(const cmag_params& P, float* viscF, float* presF, const float* measures,
                           const float* sortedPos, const float* sortedVel, const uint32_t* index,
                           const Cells& cells, uint32_t n, const float* pairs, const uint32_t* row_masks,
-                          hipStream_t s) {
+                          const StepArrays& step, hipStream_t s) {
     const bool m = P.hash_order == CMAG_HASH_MORTON;
     auto launch = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3(div_up(n, 256)), dim3(256), 0, s, P, reinterpret_cast<float4*>(viscF),
                            reinterpret_cast<float4*>(presF), reinterpret_cast<const float4*>(measures),
                            reinterpret_cast<const float4*>(sortedPos), reinterpret_cast<const float4*>(sortedVel),
-                           index, cells, n, reinterpret_cast<const float2*>(pairs), row_masks);
+                           index, cells, n, reinterpret_cast<const float2*>(pairs), row_masks, step);
     };
     if (P.dim == 3) {
         if (m) launch(peristalsis_force_kernel<3, 1, V, PR, Cells>);
@@ -308,7 +308,7 @@ static void go_peri(const cmag_params& P, float* viscF, float* presF, const floa
                     const uint32_t* cellStart, const uint32_t* cellEnd, uint32_t n, hipStream_t s) {
     if (n >= (1u << NB_SHIFT_BITS)) return;  // rejected by the callers
     go_peri_cells<V, PR>(P, viscF, presF, measures, sortedPos, sortedVel, index, RefCells{cellStart, cellEnd, n}, n,
-                         nullptr, nullptr, s);
+                         nullptr, nullptr, StepArrays{}, s);
 }
 
 int launch_pressure_force(const cmag_params& P, float* presF, const float* measures,
@@ -334,7 +334,7 @@ int launch_peristalsis_forces(const cmag_params& P, float* viscF, float* presF, 
                               const float* sortedPos, const float* sortedVel, const uint32_t* index,
                               const uint32_t* cellStart, const uint32_t* cellEnd, uint32_t n,
                               hipStream_t s, const uint32_t* cellFirst, const float* pairs,
-                              const uint32_t* row_masks) {
+                              const uint32_t* row_masks, const StepArrays& step) {
     if (n == 0) return CMAG_OK;
     if (n >= (1u << NB_SHIFT_BITS)) return fail(CMAG_E_INVALID, "force passes take at most 2^27 particles");
     if (!cellFirst) {
@@ -343,7 +343,7 @@ int launch_peristalsis_forces(const cmag_params& P, float* viscF, float* presF, 
     }
     if (!pairs) return fail(CMAG_E_INVALID, "the force pass over compact offsets takes the density pass's pair values");
     go_peri_cells<true, true>(P, viscF, presF, measures, sortedPos, sortedVel, index, FirstCells{cellFirst}, n, pairs,
-                              row_masks && row_masks_apply(P) ? row_masks : nullptr, s);
+                              row_masks && row_masks_apply(P) ? row_masks : nullptr, step, s);
     return check_launch("peristalsis_force_kernel<fused>");
 }
 

@@ -1,0 +1,61 @@
+"""The channels' force pass integrates its targets; with stage timing on the two
+stages run as launches of their own.  The operations are the same, so the states
+are the same bit for bit."""
+import numpy as np
+import pytest
+
+from cmag_amd import _lib as L
+from cmag_amd import scenarios as S
+from cmag_amd.batch import Batch
+from cmag_amd.systems import ParamSystem
+
+pytestmark = pytest.mark.gpu
+
+ARRAYS = (L.ARRAY_POSITION, L.ARRAY_VELOCITY, L.ARRAY_VELOCITYLEAPFROG, L.ARRAY_ACCELERATION)
+
+
+def scene(kind, n):
+    sc = S.channel_poiseuille(n, nu=2e-2, seed=3) if kind == "poiseuille" else S.channel_peristalsis(n, 0.3, 1.2, seed=3)
+    vel = np.zeros_like(sc.pos)
+    vel[:sc.num_fluid, 0] = 1e-2
+    vel[:, 3] = np.arange(len(vel), dtype=np.float32)  # w is carried along
+    return sc.params, sc.pos, vel
+
+
+def states(s, arrays=ARRAYS):
+    return [np.asarray(s.getArray(a)) for a in arrays]
+
+
+@pytest.mark.parametrize("kind", ["poiseuille", "peristalsis"])
+@pytest.mark.parametrize("moving", [False, True])
+@pytest.mark.parametrize("n", [1000, 2500])
+def test_system(device, kind, moving, n):
+    p, pos, vel = scene(kind, n)
+    if moving:
+        p = p.copy()
+        p.is_boundary_configuration = 0
+        p.wall_velocity = 1
+    out = []
+    for timing in (False, True):
+        s = ParamSystem(p, pos.shape[0])
+        for a, x in zip(ARRAYS, (pos, vel, vel)):
+            s.setArray(a, x)
+        s.enable_timing(timing)
+        for _ in range(3):
+            s.update()
+        out.append(states(s))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
+def test_batch(device):
+    inst = [scene(k, n) for k, n in (("poiseuille", 1000), ("peristalsis", 1100), ("poiseuille", 1500))]
+    out = []
+    for timing in (False, True):
+        b = Batch(inst)
+        b.enable_timing(timing)
+        for _ in range(3):
+            b.update()
+        out.append([np.asarray(b.getArray(k, a)) for k in range(3) for a in ARRAYS])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
