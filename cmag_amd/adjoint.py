@@ -10,7 +10,7 @@
 The forward pass is the plain System's update() (HIP graphs between
 checkpoints).  The backward pass is hand-written: the state is checkpointed
 every `checkpoint_every` steps; each segment is recomputed forward from its
-checkpoint and walked backwards with cmag_system_vjp_step, whose kernels
+checkpoint and walked backwards by cmag_system_vjp_segment, whose kernels
 (adjoint.hip) are the vector-Jacobian products of density, force and
 integrate with the step's neighbour structure held fixed.  The viscosity
 enters as mu = rho0 * nu (the parameter block's mu), the body force as
@@ -55,9 +55,6 @@ class ChannelRollout:
         self.state0 = (_f4(pos, dev), _f4(vel, dev), _f4(vel_lf, dev))
         self.system = ParamSystem(self.params, self.n)
         self._ncp = (self.steps + self.checkpoint_every - 1) // self.checkpoint_every
-        # the recomputed states of one segment: scratch of a single backward
-        # pass (autograd runs backward passes one after another)
-        self._seg = [self._state() for _ in range(self.checkpoint_every)]
 
     def _state(self):
         return tuple(torch.empty((self.n, 4), dtype=torch.float32, device=self.device) for _ in range(3))
@@ -141,13 +138,7 @@ class _Rollout(torch.autograd.Function):
             t0 = c * ce
             t1 = min(t0 + ce, run.steps)
             run._put(ctx.cps[c])
-            for t in range(t0, t1):
-                run._take(run._seg[t - t0])
-                if t < t1 - 1:
-                    s.update()
-            for t in reversed(range(t0, t1)):
-                run._put(run._seg[t - t0])
-                s.vjp_step(gpos.data_ptr(), gvel.data_ptr(), glf.data_ptr(), gmu.data_ptr(), ggrav.data_ptr())
+            s.vjp_segment(t1 - t0, gpos.data_ptr(), gvel.data_ptr(), glf.data_ptr(), gmu.data_ptr(), ggrav.data_ptr())
         s.synchronize()
         dtype, device, shape = ctx.mu_like
         dmu = gmu.sum().to(dtype=dtype, device=device).reshape(shape)

@@ -34,16 +34,39 @@
 
 namespace cmag {
 
-// d/dq of the dW/dr bracket: -4 t^3 + 1.5 t^2 (2q + 1), t = 1 - q/2
-__device__ __forceinline__ float grad_bracket_dq(float q) {
-    const float t = 1.0f - 0.5f * q;
-    return -4.0f * t * t * t + 1.5f * t * t * (2.0f * q + 1.0f);
+// With q = d / h and t = 1 - q/2, the dW/dr bracket t^4 - t^3 (2q + 1) is
+// 5 t^3 (t - 1) = -2.5 q t^3, so
+//   G    = (dW/dr) / d = g_k t^3,     g_k  = -2.5 grad_coeff / h
+//   G'/d = (dG/dd) / d = gp_k t^2 / d, gp_k = 3.75 grad_coeff / h^2
+// without the differences of the bracket's own form, and with one division a
+// pair instead of six.
+struct GradKernel {
+    float t_k, g_k, gp_k, r2max;
+    __device__ __forceinline__ explicit GradKernel(const cmag_params& P) {
+        const float h = P.smoothing_radius, gc = P.grad_coeff;
+        t_k = -0.5f / h;
+        g_k = -2.5f * gc / h;
+        gp_k = 3.75f * gc / (h * h);
+        r2max = 4.0f * h * h;
+    }
+};
+
+// p / rho^2 and 1 / rho of a row
+__device__ __forceinline__ float2 row_terms(const float4& m) { return make_float2(m.y / (m.x * m.x), 1.0f / m.x); }
+
+// sum over the VJP_LANES lanes of a target, in every one of them
+constexpr int VJP_LANES = 4;
+__device__ __forceinline__ float lanes_sum(float v) {
+    // quad_perm [1,0,3,2], then [2,3,0,1]
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true));
+    return v;
 }
 
-__device__ __forceinline__ float grad_bracket(float q) {
-    const float t = 1.0f - 0.5f * q;
-    const float t2 = t * t;
-    return t2 * t2 - t2 * t * (2.0f * q + 1.0f);
+// target and lane of a thread: the lanes of a target are neighbours
+__device__ __forceinline__ void vjp_target(uint32_t& i, uint32_t& part) {
+    i = xcd_block() * (blockDim.x / VJP_LANES) + threadIdx.x / VJP_LANES;
+    part = threadIdx.x % VJP_LANES;
 }
 
 // d p / d rho of the equation of state
@@ -59,29 +82,24 @@ __device__ __forceinline__ float dot3(float ax, float ay, float az, float bx, fl
 }
 
 // ---- integrate ----------------------------------------------------------------
-// unsorted order; gpos/gvel/gvelLF: adjoints of the step outputs in, of its
-// inputs out (velLF is no input of integrate); gacc out; ggrav[i] += share of
+// gpos/gvel/gvelLF: adjoints of the step outputs in, of its inputs out (velLF is
+// no input of integrate); returns the acceleration's; ggrav[i] += share of
 // the body-force adjoint
-__global__ __launch_bounds__(256) void integrate_vjp_kernel(const cmag_params P, const float4* __restrict__ pos,
-                                                            float4* __restrict__ gpos, float4* __restrict__ gvel,
-                                                            float4* __restrict__ gvelLF, float4* __restrict__ gacc,
-                                                            double* __restrict__ ggrav, uint32_t n) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+__device__ __forceinline__ float4 integrate_vjp_row(const cmag_params& P, uint32_t i, bool wall,
+                                                    float4* __restrict__ gpos, float4* __restrict__ gvel,
+                                                    float4* __restrict__ gvelLF, double* __restrict__ ggrav) {
     const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (pos[i].w == CMAG_PO_WALL) {
+    if (wall) {
         gpos[i] = z;
         gvel[i] = z;
         gvelLF[i] = z;
-        gacc[i] = z;
-        return;
+        return z;
     }
     const float dt = P.delta_time;
     const float4 gx = gpos[i], gv = gvel[i], gl = gvelLF[i];
     const float ux = gv.x + 0.5f * gl.x + dt * gx.x;
     const float uy = gv.y + 0.5f * gl.y + dt * gx.y;
     const float uz = gv.z + 0.5f * gl.z + dt * gx.z;
-    gacc[i] = make_float4(dt * ux, dt * uy, dt * uz, 0.f);
     gvel[i] = make_float4(ux + 0.5f * gl.x, uy + 0.5f * gl.y, uz + 0.5f * gl.z, 0.f);
     gvelLF[i] = z;
     if (ggrav) {
@@ -89,19 +107,51 @@ __global__ __launch_bounds__(256) void integrate_vjp_kernel(const cmag_params P,
         ggrav[4 * (size_t)i + 1] += (double)(dt * uy);
         ggrav[4 * (size_t)i + 2] += (double)(dt * uz);
     }
+    return make_float4(dt * ux, dt * uy, dt * uz, 0.f);
 }
 
-__global__ __launch_bounds__(256) void gather_f4_kernel(float4* __restrict__ dst, const float4* __restrict__ src,
-                                                        const uint32_t* __restrict__ index, uint32_t n) {
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const uint32_t i = index[k];
-    dst[k] = i < n ? src[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+// unsorted order
+__global__ __launch_bounds__(256) void integrate_vjp_kernel(const cmag_params P, const float4* __restrict__ pos,
+                                                            float4* __restrict__ gpos, float4* __restrict__ gvel,
+                                                            float4* __restrict__ gvelLF, float4* __restrict__ gacc,
+                                                            double* __restrict__ ggrav, uint32_t n) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    gacc[i] = integrate_vjp_row(P, i, pos[i].w == CMAG_PO_WALL, gpos, gvel, gvelLF, ggrav);
+}
+
+// The same by sorted row, for a step whose density has run: the acceleration
+// adjoint goes to the row itself, and the row's terms of the pair sums are
+// formed once.  A launch and a pass over gacc less than integrate_vjp and a
+// gather, and no division by a neighbour's density in the pair loops.
+__global__ __launch_bounds__(256) void step_vjp_kernel(const cmag_params P, const float4* __restrict__ sortedPos,
+                                                       const float4* __restrict__ measures,
+                                                       const uint32_t* __restrict__ index, float4* __restrict__ gpos,
+                                                       float4* __restrict__ gvel, float4* __restrict__ gvelLF,
+                                                       float4* __restrict__ gaccS, float2* __restrict__ terms,
+                                                       double* __restrict__ ggrav, uint32_t n) {
+    const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= n) return;
+    terms[r] = row_terms(measures[r]);
+    const uint32_t i = index[r];
+    if (i >= n) {
+        gaccS[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+        return;
+    }
+    const bool wall = sortedPos[r].w == CMAG_PO_WALL;
+    gaccS[r] = integrate_vjp_row(P, i, wall, gpos, gvel, gvelLF, ggrav);
 }
 
 // ---- force ----------------------------------------------------------------------
 // sorted order.  gmu_acc (optional) += the target's share of d/d mu in FP64;
-// gmu (optional) = the same share in FP32
+// gmu (optional) = the same share in FP32; terms: row_terms of every row, or
+// null (a caller's rows: formed here)
+//
+// Both neighbour passes give a target to VJP_LANES lanes, each with every
+// fourth stencil row (the rows of 5 + 1, 5, 5 + 1 and 5 in-range neighbours at h =
+// 1.5 spacings), and fold their sums: the passes are one serial chain per
+// target, too long for the few waves of a channel.  A row's loads are issued
+// one candidate ahead.
 template <int DIM, int HASH, typename Cells>
 __global__ __launch_bounds__(256) void force_vjp_kernel(const cmag_params P, float4* __restrict__ gpos,
                                                         float4* __restrict__ gvel, float* __restrict__ grho,
@@ -110,84 +160,102 @@ __global__ __launch_bounds__(256) void force_vjp_kernel(const cmag_params P, flo
                                                         const float4* __restrict__ measures,
                                                         const float4* __restrict__ sortedPos,
                                                         const float4* __restrict__ sortedVel, const Cells cells,
-                                                        uint32_t n) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+                                                        uint32_t n, const float2* __restrict__ terms) {
+    uint32_t i, part;
+    vjp_target(i, part);
     if (i >= n) return;
     const float4 pi = sortedPos[i];
     const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
     if (pi.w == CMAG_PO_WALL) {
-        gpos[i] = z;
-        gvel[i] = z;
-        grho[i] = 0.f;
-        if (gmu) gmu[i] = 0.f;
+        if (part == 0) {
+            gpos[i] = z;
+            gvel[i] = z;
+            grho[i] = 0.f;
+            if (gmu) gmu[i] = 0.f;
+        }
         return;
     }
     const float4 li = sortedVel[i], ai = gacc[i], mi = measures[i];
-    const float rho_i = mi.x, pi_i = mi.y / (mi.x * mi.x);
-    const float m = P.particle_mass, h = P.smoothing_radius, gc = P.grad_coeff;
-    const float r2max = 4.0f * h * h;
+    const float2 ti = row_terms(mi);
+    const float rho_i = mi.x;
+    const float m = P.particle_mass;
+    const GradKernel K(P);
     const float top = P.wall_top, bottom = P.wall_bottom;
-    float pibar = 0.f, rhobar = 0.f, mubar = 0.f;
+    const float mu2 = 2.f * m * ti.y;  // 2 m / rho_i
+    float pibar = 0.f, vd = 0.f, mubar = 0.f;
     float gx = 0.f, gy = 0.f, gz = 0.f, lx = 0.f, ly = 0.f, lz = 0.f;
-    const Cell gp = grid_pos(P, pi.x, pi.y, pi.z);
-    walk_stencil<DIM, HASH>(P, pi, gp, cells, [&](uint32_t j, float qx, float qy, float qz, int) {
-        if (j == i) return;
-        const float4 pj = sortedPos[j];
-        const float rx = qx - pj.x, ry = qy - pj.y, rz = qz - pj.z;
+    struct Row {
+        float4 p, l, a;
+        float2 t;
+    };
+    auto load = [&](uint32_t j) {
+        return Row{sortedPos[j], sortedVel[j], gacc[j], Cells::PADDED ? terms[j] : row_terms(measures[j])};
+    };
+    auto pair = [&](uint32_t j, const Row& J, float qx, float qy, float qz) {
+        const float rx = qx - J.p.x, ry = qy - J.p.y, rz = qz - J.p.z;
         const float r2 = rx * rx + ry * ry + rz * rz;
-        if (!(r2 < r2max)) return;
+        if (j == i || !(r2 < K.r2max)) return;
         const float dist = sqrtf(r2);
-        const float q = dist / h;
-        const float4 lj = sortedVel[j], aj = gacc[j], mj = measures[j];
-        const float rho_j = mj.x, pi_j = mj.y / (mj.x * mj.x);
-        const float temp = gc * grad_bracket(q);
-        const float dtemp = gc / h * grad_bracket_dq(q);
-        const float G = temp / dist;
-        const float Gp = (dtemp * dist - temp) / r2;
+        const float t = fmaf(K.t_k, dist, 1.0f);
+        const float t2 = t * t;
+        const float G = K.g_k * (t2 * t);
+        const float Gpd = K.gp_k * t2 / dist;
         float bt = 1.f, dbeta = 0.f;
         bool wall_beyond = false;
-        if (pj.w == CMAG_PO_WALL && pj.y > top) {
-            const float dA = top - pi.y, dB = pj.y - top;
+        if (J.p.w == CMAG_PO_WALL && (J.p.y > top || J.p.y < bottom)) {
+            const bool up = J.p.y > top;
+            const float dA = up ? top - pi.y : pi.y - bottom, dB = up ? J.p.y - top : bottom - J.p.y;
             const float b = 1.f + dB / dA;
             wall_beyond = true;
             bt = fminf(P.beta_max, b);
-            if (b < P.beta_max) dbeta = dB / (dA * dA);
-        } else if (pj.w == CMAG_PO_WALL && pj.y < bottom) {
-            const float dA = pi.y - bottom, dB = bottom - pj.y;
-            const float b = 1.f + dB / dA;
-            wall_beyond = true;
-            bt = fminf(P.beta_max, b);
-            if (b < P.beta_max) dbeta = -dB / (dA * dA);
+            if (b < P.beta_max) dbeta = up ? dB / (dA * dA) : -dB / (dA * dA);
         }
-        float Vx, Vy, Vz;
-        if (wall_beyond) {
-            Vx = bt * li.x; Vy = bt * li.y; Vz = bt * li.z;
-        } else {
-            Vx = li.x - lj.x; Vy = li.y - lj.y; Vz = li.z - lj.z;
-        }
-        const float Dx = ai.x - aj.x, Dy = ai.y - aj.y, Dz = ai.z - aj.z;
-        const float A = -m * (pi_i + pi_j);
-        const float B = 2.f * m * P.mu / (rho_i * rho_j);
+        const float Vx = wall_beyond ? bt * li.x : li.x - J.l.x;
+        const float Vy = wall_beyond ? bt * li.y : li.y - J.l.y;
+        const float Vz = wall_beyond ? bt * li.z : li.z - J.l.z;
+        const float Dx = ai.x - J.a.x, Dy = ai.y - J.a.y, Dz = ai.z - J.a.z;
+        const float A = -m * (ti.x + J.t.x);
+        const float B0 = mu2 * J.t.y;  // 2 m / (rho_i rho_j)
+        const float B = B0 * P.mu;
         const float c = B * G;
         const float rD = dot3(rx, ry, rz, Dx, Dy, Dz);
         const float VD = dot3(Vx, Vy, Vz, Dx, Dy, Dz);
-        pibar += -m * G * rD;
-        rhobar += -(c / rho_i) * VD;
-        mubar += 2.f * m * G / (rho_i * rho_j) * dot3(ai.x, ai.y, ai.z, Vx, Vy, Vz);
-        const float lt = wall_beyond ? bt : 1.f;
-        lx += c * (lt * ai.x - aj.x);
-        ly += c * (lt * ai.y - aj.y);
-        lz += c * (lt * ai.z - aj.z);
-        const float k1 = A * G, k2 = (A * rD + B * VD) * Gp / dist;
+        pibar = fmaf(G, rD, pibar);
+        vd = fmaf(c, VD, vd);
+        mubar = fmaf(B0 * G, dot3(ai.x, ai.y, ai.z, Vx, Vy, Vz), mubar);
+        lx = fmaf(c, bt * ai.x - J.a.x, lx);
+        ly = fmaf(c, bt * ai.y - J.a.y, ly);
+        lz = fmaf(c, bt * ai.z - J.a.z, lz);
+        const float k1 = A * G, k2 = (A * rD + B * VD) * Gpd;
         gx += k1 * Dx + k2 * rx;
         gy += k1 * Dy + k2 * ry;
         gz += k1 * Dz + k2 * rz;
         if (wall_beyond) gy += c * dot3(ai.x, ai.y, ai.z, li.x, li.y, li.z) * dbeta;
-    });
+    };
+    const Cell gp = grid_pos(P, pi.x, pi.y, pi.z);
+    walk_rows<DIM, HASH, true, false, VJP_LANES>(P, pi, gp, cells,
+                                                 [&](const Run& a, const Run& b, float py, float pz, bool) {
+        const uint32_t total = a.len + b.len, off_b = b.s - a.len;
+        if (total == 0) return;
+        auto row = [&](uint32_t t) { return (t >= a.len ? off_b : a.s) + t; };
+        uint32_t j = row(0);
+        Row J = load(j);
+        for (uint32_t t = 0; t < total; ++t) {
+            const uint32_t jn = row(min(t + 1u, total - 1u));
+            const Row N = load(jn);
+            pair(j, J, t >= a.len ? b.px : a.px, py, pz);
+            j = jn;
+            J = N;
+        }
+    }, part);
+    pibar = lanes_sum(pibar); vd = lanes_sum(vd); mubar = lanes_sum(mubar);
+    gx = lanes_sum(gx); gy = lanes_sum(gy); gz = lanes_sum(gz);
+    lx = lanes_sum(lx); ly = lanes_sum(ly); lz = lanes_sum(lz);
+    if (part != 0) return;
     const float dpi = deos(P, rho_i) / (rho_i * rho_i) - 2.f * mi.y / (rho_i * rho_i * rho_i);
     gpos[i] = make_float4(gx, gy, gz, 0.f);
     gvel[i] = make_float4(lx, ly, lz, 0.f);
-    grho[i] = pibar * dpi + rhobar;
+    grho[i] = -m * pibar * dpi - ti.y * vd;
     if (gmu) gmu[i] = mubar;
     if (gmu_acc) gmu_acc[i] += (double)mubar;
 }
@@ -203,28 +271,44 @@ __global__ __launch_bounds__(256) void density_vjp_kernel(const cmag_params P, f
                                                           uint32_t n, const uint32_t* __restrict__ index,
                                                           const float4* __restrict__ gvelS,
                                                           float4* __restrict__ gpos, float4* __restrict__ gvelLF) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t i, part;
+    vjp_target(i, part);
     if (i >= n) return;
     const float4 pi = sortedPos[i];
     if (pi.w == CMAG_PO_WALL) return;
-    const float m = P.particle_mass, h = P.smoothing_radius, gc = P.grad_coeff;
-    const float r2max = 4.0f * h * h;
+    const GradKernel K(P);
     const float gi = grho[i];
     float gx = 0.f, gy = 0.f, gz = 0.f;
     const Cell gp = grid_pos(P, pi.x, pi.y, pi.z);
-    walk_stencil<DIM, HASH>(P, pi, gp, cells, [&](uint32_t j, float qx, float qy, float qz, int) {
-        if (j == i) return;
-        const float4 pj = sortedPos[j];
-        const float rx = qx - pj.x, ry = qy - pj.y, rz = qz - pj.z;
-        const float r2 = rx * rx + ry * ry + rz * rz;
-        if (!(r2 < r2max)) return;
-        const float dist = sqrtf(r2);
-        const float G = gc * grad_bracket(dist / h) / dist;
-        const float c = m * G * (gi + grho[j]);
-        gx += c * rx; gy += c * ry; gz += c * rz;
-    });
+    walk_rows<DIM, HASH, true, false, VJP_LANES>(P, pi, gp, cells,
+                                                 [&](const Run& a, const Run& b, float py, float pz, bool) {
+        const uint32_t total = a.len + b.len, off_b = b.s - a.len;
+        if (total == 0) return;
+        auto row = [&](uint32_t t) { return (t >= a.len ? off_b : a.s) + t; };
+        uint32_t j = row(0);
+        float4 pj = sortedPos[j];
+        float gj = grho[j];
+        for (uint32_t t = 0; t < total; ++t) {
+            const uint32_t jn = row(min(t + 1u, total - 1u));
+            const float4 pn = sortedPos[jn];
+            const float gn = grho[jn];
+            const float rx = (t >= a.len ? b.px : a.px) - pj.x, ry = py - pj.y, rz = pz - pj.z;
+            const float r2 = rx * rx + ry * ry + rz * rz;
+            if (j != i && r2 < K.r2max) {
+                const float w = fmaf(K.t_k, sqrtf(r2), 1.0f);
+                const float c = w * w * w * (gi + gj);
+                gx = fmaf(c, rx, gx); gy = fmaf(c, ry, gy); gz = fmaf(c, rz, gz);
+            }
+            j = jn;
+            pj = pn;
+            gj = gn;
+        }
+    }, part);
+    gx = lanes_sum(gx); gy = lanes_sum(gy); gz = lanes_sum(gz);
+    if (part != 0) return;
+    const float mg = P.particle_mass * K.g_k;
     float4 g = gposS[i];
-    g.x += gx; g.y += gy; g.z += gz;
+    g.x = fmaf(mg, gx, g.x); g.y = fmaf(mg, gy, g.y); g.z = fmaf(mg, gz, g.z);
     if (!index) {
         gposS[i] = g;
         return;
@@ -267,31 +351,38 @@ int launch_integrate_vjp(const cmag_params& P, const float* pos, float* gpos, fl
     return check_launch("integrate_vjp_kernel");
 }
 
-int launch_gather_f4(float* dst, const float* src, const uint32_t* index, uint32_t n, hipStream_t s) {
+int launch_step_vjp(const cmag_params& P, const float* sortedPos, const float* measures, const uint32_t* index,
+                    float* gpos, float* gvel, float* gvelLF, float* gaccS, float* terms, double* ggrav, uint32_t n,
+                    hipStream_t s) {
+    CMAG_TRY(need_poiseuille(P, "step_vjp"));
     if (n == 0) return CMAG_OK;
-    hipLaunchKernelGGL(gather_f4_kernel, dim3(div_up(n, 256)), dim3(256), 0, s, reinterpret_cast<float4*>(dst),
-                       reinterpret_cast<const float4*>(src), index, n);
-    return check_launch("gather_f4_kernel");
+    hipLaunchKernelGGL(step_vjp_kernel, dim3(div_up(n, 256)), dim3(256), 0, s, P,
+                       reinterpret_cast<const float4*>(sortedPos), reinterpret_cast<const float4*>(measures), index,
+                       reinterpret_cast<float4*>(gpos), reinterpret_cast<float4*>(gvel),
+                       reinterpret_cast<float4*>(gvelLF), reinterpret_cast<float4*>(gaccS),
+                       reinterpret_cast<float2*>(terms), ggrav, n);
+    return check_launch("step_vjp_kernel");
 }
 
 int launch_force_vjp(const cmag_params& P, float* gposS, float* gvelS, float* grho, float* gmu, double* gmu_acc,
                      const float* gaccS, const float* measures, const float* sortedPos, const float* sortedVel,
                      const uint32_t* cellStart, const uint32_t* cellEnd, const uint32_t* cellFirst, uint32_t n,
-                     hipStream_t s) {
+                     const float* terms, hipStream_t s) {
     CMAG_TRY(need_poiseuille(P, "force_vjp"));
     if (n == 0) return CMAG_OK;
+    if (cellFirst && !terms) return fail(CMAG_E_INVALID, "force_vjp over compact offsets takes the rows' terms");
     auto f4 = [](float* q) { return reinterpret_cast<float4*>(q); };
     auto c4 = [](const float* q) { return reinterpret_cast<const float4*>(q); };
     dispatch_dh(P, [&](auto D, auto H) {
         constexpr int DIM = decltype(D)::value, HASH = decltype(H)::value;
         if (cellFirst)
-            hipLaunchKernelGGL((force_vjp_kernel<DIM, HASH, FirstCells>), dim3(div_up(n, 256)), dim3(256), 0, s,
+            hipLaunchKernelGGL((force_vjp_kernel<DIM, HASH, FirstCells>), dim3(div_up(n, 256 / VJP_LANES)), dim3(256), 0, s,
                                P, f4(gposS), f4(gvelS), grho, gmu, gmu_acc, c4(gaccS), c4(measures), c4(sortedPos),
-                               c4(sortedVel), FirstCells{cellFirst}, n);
+                               c4(sortedVel), FirstCells{cellFirst}, n, reinterpret_cast<const float2*>(terms));
         else
-            hipLaunchKernelGGL((force_vjp_kernel<DIM, HASH, RefCells>), dim3(div_up(n, 256)), dim3(256), 0, s, P,
+            hipLaunchKernelGGL((force_vjp_kernel<DIM, HASH, RefCells>), dim3(div_up(n, 256 / VJP_LANES)), dim3(256), 0, s, P,
                                f4(gposS), f4(gvelS), grho, gmu, gmu_acc, c4(gaccS), c4(measures), c4(sortedPos),
-                               c4(sortedVel), RefCells{cellStart, cellEnd, n}, n);
+                               c4(sortedVel), RefCells{cellStart, cellEnd, n}, n, nullptr);
     });
     return check_launch("force_vjp_kernel");
 }
@@ -306,11 +397,11 @@ int launch_density_vjp(const cmag_params& P, float* gposS, const float* grho, co
     dispatch_dh(P, [&](auto D, auto H) {
         constexpr int DIM = decltype(D)::value, HASH = decltype(H)::value;
         if (cellFirst)
-            hipLaunchKernelGGL((density_vjp_kernel<DIM, HASH, FirstCells>), dim3(div_up(n, 256)), dim3(256), 0, s,
+            hipLaunchKernelGGL((density_vjp_kernel<DIM, HASH, FirstCells>), dim3(div_up(n, 256 / VJP_LANES)), dim3(256), 0, s,
                                P, f4(gposS), grho, c4(sortedPos), FirstCells{cellFirst}, n, index, c4(gvelS),
                                f4(gpos), f4(gvelLF));
         else
-            hipLaunchKernelGGL((density_vjp_kernel<DIM, HASH, RefCells>), dim3(div_up(n, 256)), dim3(256), 0, s, P,
+            hipLaunchKernelGGL((density_vjp_kernel<DIM, HASH, RefCells>), dim3(div_up(n, 256 / VJP_LANES)), dim3(256), 0, s, P,
                                f4(gposS), grho, c4(sortedPos), RefCells{cellStart, cellEnd, n}, n, index,
                                c4(gvelS), f4(gpos), f4(gvelLF));
     });
@@ -339,7 +430,7 @@ int cmag_force_vjp(const cmag_params* p, float* gposS, float* gvelS, float* grho
               !cellEnd))
         return fail(CMAG_E_INVALID, "cmag_force_vjp: null pointer");
     return launch_force_vjp(*p, gposS, gvelS, grho, gmu, nullptr, gaccS, measures, sortedPos, sortedVel, cellStart,
-                            cellEnd, nullptr, n, as_stream(stream));
+                            cellEnd, nullptr, n, nullptr, as_stream(stream));
 }
 
 int cmag_density_vjp(const cmag_params* p, float* gposS, const float* grho, const float* sortedPos,

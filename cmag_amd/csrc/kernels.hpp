@@ -136,11 +136,14 @@ int launch_remove_right_boundary(const cmag_params& P, float* pos, uint32_t n, h
 // adjoints of the Poiseuille step (adjoint.hip)
 int launch_integrate_vjp(const cmag_params& P, const float* pos, float* gpos, float* gvel, float* gvelLF,
                          float* gacc, double* ggrav, uint32_t n, hipStream_t s);
-int launch_gather_f4(float* dst, const float* src, const uint32_t* index, uint32_t n, hipStream_t s);
+// integrate_vjp by sorted row: gaccS, and terms (2 floats a row) for launch_force_vjp
+int launch_step_vjp(const cmag_params& P, const float* sortedPos, const float* measures, const uint32_t* index,
+                    float* gpos, float* gvel, float* gvelLF, float* gaccS, float* terms, double* ggrav, uint32_t n,
+                    hipStream_t s);
 int launch_force_vjp(const cmag_params& P, float* gposS, float* gvelS, float* grho, float* gmu, double* gmu_acc,
                      const float* gaccS, const float* measures, const float* sortedPos, const float* sortedVel,
                      const uint32_t* cellStart, const uint32_t* cellEnd, const uint32_t* cellFirst, uint32_t n,
-                     hipStream_t s);
+                     const float* terms, hipStream_t s);
 int launch_density_vjp(const cmag_params& P, float* gposS, const float* grho, const float* sortedPos,
                        const uint32_t* cellStart, const uint32_t* cellEnd, const uint32_t* cellFirst, uint32_t n,
                        const uint32_t* index, const float* gvelS, float* gpos, float* gvelLF, hipStream_t s);

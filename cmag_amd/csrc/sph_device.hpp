@@ -189,9 +189,11 @@ __device__ __forceinline__ int force_row(int dim, int k) {
 // whole: the whole row comes in this one call (in every lane of the wave).
 // walk_stencil and walk_stencil_pf turn them into candidate calls.  With
 // FORCE_ORDER and one cell per stencil side, the rows come in force_row order.
-template <int DIM, int HASH, bool PERIODIC = true, bool FORCE_ORDER = false, typename Cells, typename R>
+// With LANES > 1 that many lanes share the target: this one takes the rows
+// part, part + LANES, ...
+template <int DIM, int HASH, bool PERIODIC = true, bool FORCE_ORDER = false, int LANES = 1, typename Cells, typename R>
 __device__ __forceinline__ void walk_rows(const cmag_params& P, const float4& pi, const Cell& gp,
-                                          const Cells& cells, R&& run_pair) {
+                                          const Cells& cells, R&& run_pair, uint32_t part = 0) {
     const int cc = P.cellcount;
     const int sub = Cells::SUB ? x_sub(P, pi.x) : 0;
     const uint32_t gxm = P.grid_size[0] - 1u, gym = P.grid_size[1] - 1u, gzm = P.grid_size[2] - 1u;
@@ -362,6 +364,19 @@ __device__ __forceinline__ void walk_rows(const cmag_params& P, const float4& pi
                 for (int t = 0; t < iz; ++t) kz = dilated_inc(kz, Mz);
             }
             row_body(iy - 1, DIM == 3 ? iz - 1 : 0, ky, kz);
+        }
+        return;
+    }
+    if (LANES > 1) {
+        const int side = 2 * cc + 1, rows = DIM == 2 ? side : side * side;
+        for (int r = (int)part; r < rows; r += LANES) {
+            const int iz = DIM == 2 ? 0 : r / side, iy = r - iz * side;
+            uint32_t ky = ky0, kz = kz0;
+            if (HASH == CMAG_HASH_MORTON) {
+                for (int t = 0; t < iy; ++t) ky = dilated_inc(ky, My);
+                for (int t = 0; t < iz; ++t) kz = dilated_inc(kz, Mz);
+            }
+            row_body(iy - cc, DIM == 2 ? 0 : iz - cc, ky, kz);
         }
         return;
     }

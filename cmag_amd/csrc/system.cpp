@@ -33,7 +33,15 @@ struct cmag_system {
     uint32_t* cellFirst = nullptr;  // compact cell offsets for the walkers
     CellSort sort;
     // adjoint scratch (sorted order), allocated by the first vjp_step
-    float *gaccU = nullptr, *gaccS = nullptr, *gposS = nullptr, *gvelS = nullptr, *grho = nullptr;
+    float *gaccS = nullptr, *gposS = nullptr, *gvelS = nullptr, *grho = nullptr, *gterms = nullptr;
+    // what the adjoint needs of each step of a segment, allocated by
+    // vjp_segment (one block per step): the sorted rows, their densities,
+    // particle numbers and cell offsets
+    struct Kept {
+        float *sortedPos, *sortedVel, *measures;
+        uint32_t *index, *cellFirst;
+    };
+    std::vector<void*> kept;
     // sub-cell walk order (DamBreak): the neighbour passes run over copies of
     // the sorted rows in bucket order inside each cell; the density pass writes
     // measures in the reference order, so every array a caller sees keeps its
@@ -97,9 +105,10 @@ struct cmag_system {
             if (e) (void)hipEventDestroy(e);
         void* bufs[] = {pos, vel, velLF, acc, presF, measures, sortedPos, sortedVel, predicted,
                         hash, index, cellStart, cellEnd, cellFirst,
-                        gaccU, gaccS, gposS, gvelS, grho, dState, posW, velW, indexW, w2r, masks, pairs, rowMasks, color};
+                        gaccS, gposS, gvelS, grho, gterms, dState, posW, velW, indexW, w2r, masks, pairs, rowMasks, color};
         for (void* b : bufs)
             if (b) (void)hipFree(b);
+        for (void* b : kept) (void)hipFree(b);
         sort.release();
         if (own_stream) (void)hipStreamDestroy(own_stream);
     }
@@ -305,24 +314,94 @@ struct cmag_system {
         if (P.system != CMAG_SYS_POISEUILLE)
             return fail(CMAG_E_INVALID, "vjp_step: the adjoint covers the Poiseuille system");
         if (n && (!gpos || !gvel || !gvelLF)) return fail(CMAG_E_INVALID, "vjp_step: null adjoint");
-        if (!gaccU) {
-            const size_t f4 = sizeof(float) * 4 * (size_t)(n ? n : 1);
-            float** fb[] = {&gaccU, &gaccS, &gposS, &gvelS};
-            for (float** b : fb) CMAG_HIP_TRY(hipMalloc((void**)b, f4));
-            CMAG_HIP_TRY(hipMalloc((void**)&grho, sizeof(float) * (size_t)(n ? n : 1)));
-        }
+        CMAG_TRY(alloc_vjp());
         invalidate_graph();
         const bool was_timing = timing;
         timing = false;
         int rc = enqueue_front(false);
         timing = was_timing;
         CMAG_TRY(rc);
-        CMAG_TRY(launch_integrate_vjp(P, pos, gpos, gvel, gvelLF, gaccU, ggrav_acc, n, stream));
-        CMAG_TRY(launch_gather_f4(gaccS, gaccU, index, n, stream));
-        CMAG_TRY(launch_force_vjp(P, gposS, gvelS, grho, nullptr, gmu_acc, gaccS, measures, sortedPos, sortedVel,
-                                  cellStart, cellEnd, cellFirst, n, stream));
-        CMAG_TRY(launch_density_vjp(P, gposS, grho, sortedPos, cellStart, cellEnd, cellFirst, n, index, gvelS,
-                                    gpos, gvelLF, stream));
+        return enqueue_vjp(current(), gpos, gvel, gvelLF, gmu_acc, ggrav_acc);
+    }
+
+    int alloc_vjp() {
+        if (gterms) return CMAG_OK;
+        const size_t f4 = sizeof(float) * 4 * (size_t)(n ? n : 1);
+        float** fb[] = {&gaccS, &gposS, &gvelS};
+        for (float** b : fb)
+            if (!*b) CMAG_HIP_TRY(hipMalloc((void**)b, f4));
+        if (!grho) CMAG_HIP_TRY(hipMalloc((void**)&grho, f4 / 4));
+        CMAG_HIP_TRY(hipMalloc((void**)&gterms, f4 / 2));
+        return CMAG_OK;
+    }
+
+    Kept current() const { return Kept{sortedPos, sortedVel, measures, index, cellFirst}; }
+    void use(const Kept& k) {
+        sortedPos = k.sortedPos;
+        sortedVel = k.sortedVel;
+        measures = k.measures;
+        index = k.index;
+        cellFirst = k.cellFirst;
+    }
+
+    // the backward half of one step whose front left f
+    int enqueue_vjp(const Kept& f, float* gpos, float* gvel, float* gvelLF, double* gmu_acc, double* ggrav_acc) {
+        CMAG_TRY(launch_step_vjp(P, f.sortedPos, f.measures, f.index, gpos, gvel, gvelLF, gaccS, gterms, ggrav_acc, n,
+                                 stream));
+        CMAG_TRY(launch_force_vjp(P, gposS, gvelS, grho, nullptr, gmu_acc, gaccS, f.measures, f.sortedPos,
+                                  f.sortedVel, cellStart, cellEnd, f.cellFirst, n, gterms, stream));
+        return launch_density_vjp(P, gposS, grho, f.sortedPos, cellStart, cellEnd, f.cellFirst, n, f.index, gvelS,
+                                  gpos, gvelLF, stream);
+    }
+
+    // adjoint of `steps` update()s from the current state, which is stepped
+    // steps - 1 times on the way.  Each step's front leaves what the backward
+    // half reads in a block of its own, so a step is made once: keeping the
+    // states instead took six copies a step and its front a second time
+    int vjp_segment(uint32_t steps, float* gpos, float* gvel, float* gvelLF, double* gmu_acc, double* ggrav_acc) {
+        if (P.system != CMAG_SYS_POISEUILLE)
+            return fail(CMAG_E_INVALID, "vjp_segment: the adjoint covers the Poiseuille system");
+        if (n && (!gpos || !gvel || !gvelLF)) return fail(CMAG_E_INVALID, "vjp_segment: null adjoint");
+        if (steps == 0) return CMAG_OK;
+        CMAG_TRY(alloc_vjp());
+        // parts of a block on 256-byte boundaries; the walks read up to two rows past the sorted positions
+        auto part = [](size_t bytes) { return (bytes + 255) & ~(size_t)255; };
+        const size_t rows = part(sizeof(float) * 4 * (size_t)n + 64), nums = part(sizeof(uint32_t) * ((size_t)n + 1));
+        const size_t block = 3 * rows + nums + part(sizeof(uint32_t) * ((size_t)numCells + 1));
+        try {
+            kept.reserve(steps);
+        } catch (...) {
+            return fail(CMAG_E_INVALID, "vjp_segment: out of host memory");
+        }
+        while (kept.size() < steps) {
+            void* b = nullptr;
+            CMAG_HIP_TRY(hipMalloc(&b, block));
+            kept.push_back(b);
+        }
+        auto slot = [&](uint32_t t) {
+            char* b = static_cast<char*>(kept[t]);
+            auto f = [&](size_t at) { return reinterpret_cast<float*>(b + at); };
+            auto u = [&](size_t at) { return reinterpret_cast<uint32_t*>(b + at); };
+            return Kept{f(0), f(rows), f(2 * rows), u(3 * rows), u(3 * rows + nums)};
+        };
+        invalidate_graph();
+        const bool was_timing = timing;
+        timing = false;
+        const Kept own = current();
+        int rc = CMAG_OK;
+        for (uint32_t t = 0; t < steps && rc == CMAG_OK; ++t) {
+            use(slot(t));
+            if (t + 1 < steps) {
+                rc = enqueue_step();
+                if (rc == CMAG_OK) advance_clock();
+            } else {
+                rc = enqueue_front(false);
+            }
+        }
+        use(own);
+        timing = was_timing;
+        CMAG_TRY(rc);
+        for (uint32_t t = steps; t-- > 0;) CMAG_TRY(enqueue_vjp(slot(t), gpos, gvel, gvelLF, gmu_acc, ggrav_acc));
         return CMAG_OK;
     }
 
@@ -624,6 +703,13 @@ int cmag_system_set_stream(cmag_system* s, cmag_stream_t stream) {
     s->stream = stream ? as_stream(stream) : s->own_stream;
     s->invalidate_graph();
     return CMAG_OK;
+}
+
+int cmag_system_vjp_segment(cmag_system* s, uint32_t steps, float* gpos, float* gvel, float* gvelLF, double* gmu_acc,
+                            double* ggrav_acc) {
+    if (!s) return fail(CMAG_E_INVALID, "null system");
+    CMAG_TRY(s->collect());
+    return s->vjp_segment(steps, gpos, gvel, gvelLF, gmu_acc, ggrav_acc);
 }
 
 int cmag_system_vjp_step(cmag_system* s, float* gpos, float* gvel, float* gvelLF, double* gmu_acc,

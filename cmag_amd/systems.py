@@ -163,6 +163,11 @@ class SystemBase:
         cmag_system_vjp_step)"""
         call("cmag_system_vjp_step", self._h, gpos, gvel, gvel_lf, gmu_acc or None, ggrav_acc or None)
 
+    def vjp_segment(self, steps: int, gpos: int, gvel: int, gvel_lf: int, gmu_acc: int = 0, ggrav_acc: int = 0) -> None:
+        """adjoint of `steps` updates from the current state (device pointers; see
+        cmag_system_vjp_segment)"""
+        call("cmag_system_vjp_segment", self._h, steps, gpos, gvel, gvel_lf, gmu_acc or None, ggrav_acc or None)
+
     def set_stream(self, stream: int) -> None:
         call("cmag_system_set_stream", self._h, stream)
 
