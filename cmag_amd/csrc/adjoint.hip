@@ -54,19 +54,10 @@ struct GradKernel {
 // p / rho^2 and 1 / rho of a row
 __device__ __forceinline__ float2 row_terms(const float4& m) { return make_float2(m.y / (m.x * m.x), 1.0f / m.x); }
 
-// sum over the VJP_LANES lanes of a target, in every one of them
-constexpr int VJP_LANES = 4;
-__device__ __forceinline__ float lanes_sum(float v) {
-    // quad_perm [1,0,3,2], then [2,3,0,1]
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true));
-    return v;
-}
-
 // target and lane of a thread: the lanes of a target are neighbours
 __device__ __forceinline__ void vjp_target(uint32_t& i, uint32_t& part) {
-    i = xcd_block() * (blockDim.x / VJP_LANES) + threadIdx.x / VJP_LANES;
-    part = threadIdx.x % VJP_LANES;
+    i = xcd_block() * (blockDim.x / TARGET_LANES) + threadIdx.x / TARGET_LANES;
+    part = threadIdx.x % TARGET_LANES;
 }
 
 // d p / d rho of the equation of state
@@ -147,7 +138,7 @@ __global__ __launch_bounds__(256) void step_vjp_kernel(const cmag_params P, cons
 // gmu (optional) = the same share in FP32; terms: row_terms of every row, or
 // null (a caller's rows: formed here)
 //
-// Both neighbour passes give a target to VJP_LANES lanes, each with every
+// Both neighbour passes give a target to TARGET_LANES lanes, each with every
 // fourth stencil row (the rows of 5 + 1, 5, 5 + 1 and 5 in-range neighbours at h =
 // 1.5 spacings), and fold their sums: the passes are one serial chain per
 // target, too long for the few waves of a channel.  A row's loads are issued
@@ -233,7 +224,7 @@ __global__ __launch_bounds__(256) void force_vjp_kernel(const cmag_params P, flo
         if (wall_beyond) gy += c * dot3(ai.x, ai.y, ai.z, li.x, li.y, li.z) * dbeta;
     };
     const Cell gp = grid_pos(P, pi.x, pi.y, pi.z);
-    walk_rows<DIM, HASH, true, false, VJP_LANES>(P, pi, gp, cells,
+    walk_rows<DIM, HASH, true, false, TARGET_LANES>(P, pi, gp, cells,
                                                  [&](const Run& a, const Run& b, float py, float pz, bool) {
         const uint32_t total = a.len + b.len, off_b = b.s - a.len;
         if (total == 0) return;
@@ -248,9 +239,9 @@ __global__ __launch_bounds__(256) void force_vjp_kernel(const cmag_params P, flo
             J = N;
         }
     }, part);
-    pibar = lanes_sum(pibar); vd = lanes_sum(vd); mubar = lanes_sum(mubar);
-    gx = lanes_sum(gx); gy = lanes_sum(gy); gz = lanes_sum(gz);
-    lx = lanes_sum(lx); ly = lanes_sum(ly); lz = lanes_sum(lz);
+    pibar = quad_sum(pibar); vd = quad_sum(vd); mubar = quad_sum(mubar);
+    gx = quad_sum(gx); gy = quad_sum(gy); gz = quad_sum(gz);
+    lx = quad_sum(lx); ly = quad_sum(ly); lz = quad_sum(lz);
     if (part != 0) return;
     const float dpi = deos(P, rho_i) / (rho_i * rho_i) - 2.f * mi.y / (rho_i * rho_i * rho_i);
     gpos[i] = make_float4(gx, gy, gz, 0.f);
@@ -280,7 +271,7 @@ __global__ __launch_bounds__(256) void density_vjp_kernel(const cmag_params P, f
     const float gi = grho[i];
     float gx = 0.f, gy = 0.f, gz = 0.f;
     const Cell gp = grid_pos(P, pi.x, pi.y, pi.z);
-    walk_rows<DIM, HASH, true, false, VJP_LANES>(P, pi, gp, cells,
+    walk_rows<DIM, HASH, true, false, TARGET_LANES>(P, pi, gp, cells,
                                                  [&](const Run& a, const Run& b, float py, float pz, bool) {
         const uint32_t total = a.len + b.len, off_b = b.s - a.len;
         if (total == 0) return;
@@ -304,7 +295,7 @@ __global__ __launch_bounds__(256) void density_vjp_kernel(const cmag_params P, f
             gj = gn;
         }
     }, part);
-    gx = lanes_sum(gx); gy = lanes_sum(gy); gz = lanes_sum(gz);
+    gx = quad_sum(gx); gy = quad_sum(gy); gz = quad_sum(gz);
     if (part != 0) return;
     const float mg = P.particle_mass * K.g_k;
     float4 g = gposS[i];
@@ -376,11 +367,11 @@ int launch_force_vjp(const cmag_params& P, float* gposS, float* gvelS, float* gr
     dispatch_dh(P, [&](auto D, auto H) {
         constexpr int DIM = decltype(D)::value, HASH = decltype(H)::value;
         if (cellFirst)
-            hipLaunchKernelGGL((force_vjp_kernel<DIM, HASH, FirstCells>), dim3(div_up(n, 256 / VJP_LANES)), dim3(256), 0, s,
+            hipLaunchKernelGGL((force_vjp_kernel<DIM, HASH, FirstCells>), dim3(div_up(n, 256 / TARGET_LANES)), dim3(256), 0, s,
                                P, f4(gposS), f4(gvelS), grho, gmu, gmu_acc, c4(gaccS), c4(measures), c4(sortedPos),
                                c4(sortedVel), FirstCells{cellFirst}, n, reinterpret_cast<const float2*>(terms));
         else
-            hipLaunchKernelGGL((force_vjp_kernel<DIM, HASH, RefCells>), dim3(div_up(n, 256 / VJP_LANES)), dim3(256), 0, s, P,
+            hipLaunchKernelGGL((force_vjp_kernel<DIM, HASH, RefCells>), dim3(div_up(n, 256 / TARGET_LANES)), dim3(256), 0, s, P,
                                f4(gposS), f4(gvelS), grho, gmu, gmu_acc, c4(gaccS), c4(measures), c4(sortedPos),
                                c4(sortedVel), RefCells{cellStart, cellEnd, n}, n, nullptr);
     });
@@ -397,11 +388,11 @@ int launch_density_vjp(const cmag_params& P, float* gposS, const float* grho, co
     dispatch_dh(P, [&](auto D, auto H) {
         constexpr int DIM = decltype(D)::value, HASH = decltype(H)::value;
         if (cellFirst)
-            hipLaunchKernelGGL((density_vjp_kernel<DIM, HASH, FirstCells>), dim3(div_up(n, 256 / VJP_LANES)), dim3(256), 0, s,
+            hipLaunchKernelGGL((density_vjp_kernel<DIM, HASH, FirstCells>), dim3(div_up(n, 256 / TARGET_LANES)), dim3(256), 0, s,
                                P, f4(gposS), grho, c4(sortedPos), FirstCells{cellFirst}, n, index, c4(gvelS),
                                f4(gpos), f4(gvelLF));
         else
-            hipLaunchKernelGGL((density_vjp_kernel<DIM, HASH, RefCells>), dim3(div_up(n, 256 / VJP_LANES)), dim3(256), 0, s, P,
+            hipLaunchKernelGGL((density_vjp_kernel<DIM, HASH, RefCells>), dim3(div_up(n, 256 / TARGET_LANES)), dim3(256), 0, s, P,
                                f4(gposS), grho, c4(sortedPos), RefCells{cellStart, cellEnd, n}, n, index,
                                c4(gvelS), f4(gpos), f4(gvelLF));
     });

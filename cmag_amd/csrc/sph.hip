@@ -7,17 +7,27 @@
 
 namespace cmag {
 
-template <int SYS, int DIM, int HASH, typename Cells>
+// Dam-break targets are shared between TARGET_LANES lanes up to this many rows.
+// Two steps of a 3-D dam break by itself / of four at once on their own streams,
+// a lane to a target against four: 25,168 rows 395 / 104 us against 169 / 56,
+// 54,508: 412 / 115 against 260 / 95, 82,188: 399 / 126 against 261 / 120,
+// 117,260: 414 / 136 against 310 / 159 (four at once fill the chip either way,
+// and a shared target costs more work); 160,492: 466 / 161 against 389 / 223.
+// The stage launchers over a caller's arrays: 54,508 rows 214 against 137 us,
+// 82,188: 210 against 186, 117,260: 223 against 237.
+constexpr uint32_t SHARED_TARGETS = 3u << 15;
+
+template <int SYS, int DIM, int HASH, typename Cells, int LANES = 1>
 __global__ __launch_bounds__(256) void density_kernel(const cmag_params P, float4* __restrict__ measures,
                                                        const float4* __restrict__ sortedPos, const Cells cells,
                                                        uint32_t n, float2* __restrict__ pairs,
                                                        uint32_t* __restrict__ row_masks) {
-    const uint32_t i = xcd_block() * blockDim.x + threadIdx.x;
+    const uint32_t i = xcd_block() * (256 / LANES) + threadIdx.x / LANES;
     if (i >= n) return;
-    density_body<SYS, DIM, HASH>(P, i, measures, sortedPos, cells, pairs, row_masks, n);
+    density_body<SYS, DIM, HASH, LANES>(P, i, measures, sortedPos, cells, pairs, row_masks, n, threadIdx.x % LANES);
 }
 
-template <int SYS, int DIM, int HASH, typename Cells>
+template <int SYS, int DIM, int HASH, typename Cells, int LANES = 1>
 __global__ __launch_bounds__(256) void force_kernel(const cmag_params P, float4* __restrict__ acc,
                                                      const float4* __restrict__ measures,
                                                      const float4* __restrict__ sortedPos,
@@ -26,10 +36,11 @@ __global__ __launch_bounds__(256) void force_kernel(const cmag_params P, float4*
                                                      uint32_t n, const float2* __restrict__ pairs,
                                                      const uint32_t* __restrict__ row_masks, const StepArrays step) {
     __shared__ uint32_t nbl[256 / 64][NB_CAP][64];
-    const uint32_t i = xcd_block() * blockDim.x + threadIdx.x;
+    const uint32_t i = xcd_block() * (256 / LANES) + threadIdx.x / LANES;
     if (i >= n) return;
-    force_body<SYS, DIM, HASH>(P, i, acc, measures, sortedPos, sortedVel, index, cells, n, nbl[threadIdx.x >> 6],
-                               nullptr, false, nullptr, n, pairs, row_masks, step);
+    force_body<SYS, DIM, HASH, Cells, NB_CAP, LANES>(P, i, acc, measures, sortedPos, sortedVel, index, cells, n,
+                                                     nbl[threadIdx.x >> 6], nullptr, false, nullptr, n, pairs,
+                                                     row_masks, step, threadIdx.x % LANES);
 }
 
 // Peristalsis: pressure and viscous passes; the fused variant produces both
@@ -88,18 +99,21 @@ static void dispatch3(const cmag_params& P, Args&&... args) {
 
 template <int SYS, int DIM, int H>
 struct DensityGo {
-    template <typename Cells>
+    template <int LANES = 1, typename Cells>
     static void run(const cmag_params& P, float* measures, const float* sortedPos, const Cells& cells,
                     uint32_t n, float* pairs, uint32_t* row_masks, hipStream_t s) {
-        hipLaunchKernelGGL((density_kernel<SYS, DIM, H, Cells>), dim3(div_up(n, 256)), dim3(256), 0, s, P,
+        hipLaunchKernelGGL((density_kernel<SYS, DIM, H, Cells, LANES>), dim3(div_up(n, 256 / LANES)), dim3(256), 0, s, P,
                            reinterpret_cast<float4*>(measures), reinterpret_cast<const float4*>(sortedPos),
                            cells, n, reinterpret_cast<float2*>(pairs), row_masks);
     }
     static void go(const cmag_params& P, float* measures, const float* sortedPos, const uint32_t* cellStart,
                    const uint32_t* cellEnd, const uint32_t* cellFirst, uint32_t n, float* pairs, uint32_t* row_masks,
                    hipStream_t s) {
+        constexpr int SHARE = SYS == CMAG_SYS_DAMBREAK ? TARGET_LANES : 1;
+        const RefCells ref{cellStart, cellEnd, n};
         if (cellFirst) run(P, measures, sortedPos, FirstCells{cellFirst}, n, pairs, row_masks, s);
-        else run(P, measures, sortedPos, RefCells{cellStart, cellEnd, n}, n, nullptr, nullptr, s);
+        else if (n <= SHARED_TARGETS) run<SHARE>(P, measures, sortedPos, ref, n, nullptr, nullptr, s);
+        else run(P, measures, sortedPos, ref, n, nullptr, nullptr, s);
     }
 };
 
@@ -123,12 +137,12 @@ struct CountGo {
 
 template <int SYS, int DIM, int H>
 struct ForceGo {
-    template <typename Cells>
+    template <int LANES = 1, typename Cells>
     static void run(const cmag_params& P, float* acc, const float* measures, const float* sortedPos,
                     const float* sortedVel, const uint32_t* index, const Cells& cells, uint32_t n,
                     const float* pairs, const uint32_t* row_masks, const StepArrays& step, hipStream_t s) {
         if constexpr (SYS != CMAG_SYS_PERISTALSIS)
-            hipLaunchKernelGGL((force_kernel<SYS, DIM, H, Cells>), dim3(div_up(n, 256)), dim3(256), 0, s, P,
+            hipLaunchKernelGGL((force_kernel<SYS, DIM, H, Cells, LANES>), dim3(div_up(n, 256 / LANES)), dim3(256), 0, s, P,
                                reinterpret_cast<float4*>(acc), reinterpret_cast<const float4*>(measures),
                                reinterpret_cast<const float4*>(sortedPos),
                                reinterpret_cast<const float4*>(sortedVel), index, cells, n,
@@ -138,11 +152,14 @@ struct ForceGo {
                    const float* sortedVel, const uint32_t* index, const uint32_t* cellStart,
                    const uint32_t* cellEnd, const uint32_t* cellFirst, uint32_t n, const float* pairs,
                    const uint32_t* row_masks, const StepArrays& step, hipStream_t s) {
+        constexpr int SHARE = SYS == CMAG_SYS_DAMBREAK ? TARGET_LANES : 1;
+        const RefCells ref{cellStart, cellEnd, n};
         if (cellFirst)
             run(P, acc, measures, sortedPos, sortedVel, index, FirstCells{cellFirst}, n, pairs, row_masks, step, s);
+        else if (n <= SHARED_TARGETS)
+            run<SHARE>(P, acc, measures, sortedPos, sortedVel, index, ref, n, nullptr, nullptr, StepArrays{}, s);
         else
-            run(P, acc, measures, sortedPos, sortedVel, index, RefCells{cellStart, cellEnd, n}, n, nullptr, nullptr,
-                StepArrays{}, s);
+            run(P, acc, measures, sortedPos, sortedVel, index, ref, n, nullptr, nullptr, StepArrays{}, s);
     }
 };
 
@@ -171,7 +188,7 @@ int launch_force(const cmag_params& P, float* acc, const float* measures, const 
 // thread writes the w of its own row only, after its walk.
 // With masks, staged blocks also leave the in-range masks of their rows for
 // the force pass (masks[r * n + i]).
-template <int DIM, int HASH>
+template <int DIM, int HASH, int LANES>
 __global__ __launch_bounds__(256) void density_sub_kernel(const cmag_params P, float4* __restrict__ measures,
                                                            const uint32_t* __restrict__ keys,
                                                            const uint32_t* __restrict__ w2r, float4* posW,
@@ -179,22 +196,33 @@ __global__ __launch_bounds__(256) void density_sub_kernel(const cmag_params P, f
                                                            uint2* __restrict__ masks) {
     __shared__ LookupPlan lp;
     __shared__ LookupTables lt;
-    const uint32_t b0 = xcd_block() * blockDim.x;
-    const uint32_t i = b0 + threadIdx.x;
-    __shared__ RowStage rs;
-    __shared__ RowLds rows;
-    const bool staged = stage_lookups<DIM, HASH>(P, keys, cells, n, b0, lp, lt);
-    if (staged) stage_rows<DIM>(lp, lt, posW, rows, rs);
+    const uint32_t b0 = xcd_block() * (256 / LANES);
+    const uint32_t i = b0 + threadIdx.x / LANES, part = threadIdx.x % LANES;
+    // the lanes of a shared target are in different rows: none of theirs is staged
+    constexpr bool ROWS = LANES == 1;
+    using Stage = std::conditional_t<ROWS, RowStage, char>;
+    using Rows = std::conditional_t<ROWS, RowLds, char>;
+    __shared__ Stage stage;
+    __shared__ Rows rows;
+    const RowStage* rs = nullptr;
+    const RowLds* rl = nullptr;
+    const bool staged = stage_lookups<DIM, HASH>(P, keys, cells, n, b0, 256 / LANES, lp, lt);
+    if constexpr (ROWS) {
+        if (staged) stage_rows<DIM>(lp, lt, posW, rows, stage);
+        rs = &stage;
+        rl = &rows;
+    }
     if (i >= n) return;
     const float4 pi = posW[i];
     float dens;
     if (!staged) {
-        dens = density_sum<CMAG_SYS_DAMBREAK, DIM, HASH>(P, pi, posW, cells);
+        dens = density_sum<CMAG_SYS_DAMBREAK, DIM, HASH, LANES>(P, pi, posW, cells, part);
     } else {
         const LookupView v = lookup_view<DIM>(lp, lt, keys[i], key_masks<HASH>(P).x);
-        dens = masks ? density_sum_masks<DIM>(P, pi, v, rs, &rows, posW, masks, i, n)
-                     : density_sum_lookup<DIM>(P, pi, v, rs, &rows, posW);
+        dens = masks ? density_sum_masks<DIM, LANES>(P, pi, v, rs, rl, posW, masks, i, n, part)
+                     : density_sum_lookup<DIM, LANES>(P, pi, v, rs, rl, posW, part);
     }
+    if (part != 0) return;
     const float p = eos(P, dens);
     reinterpret_cast<float2*>(measures)[2 * (size_t)w2r[i]] = make_float2(dens, p);
     if (pi.w == CMAG_DB_FLUID) {
@@ -213,15 +241,23 @@ int launch_density_sub(const cmag_params& P, float* measures, const uint32_t* ke
     float4* pw = reinterpret_cast<float4*>(posW);
     float4* vw = reinterpret_cast<float4*>(velW);
     uint2* mk = reinterpret_cast<uint2*>(masks);
-    const dim3 g(div_up(n, 256)), b(256);
     const bool m = P.hash_order == CMAG_HASH_MORTON;
-    if (P.dim == 3) {
-        if (m) hipLaunchKernelGGL((density_sub_kernel<3, 1>), g, b, 0, s, P, m4, keys, w2r, pw, vw, cells, n, mk);
-        else hipLaunchKernelGGL((density_sub_kernel<3, 0>), g, b, 0, s, P, m4, keys, w2r, pw, vw, cells, n, mk);
-    } else {
-        if (m) hipLaunchKernelGGL((density_sub_kernel<2, 1>), g, b, 0, s, P, m4, keys, w2r, pw, vw, cells, n, mk);
-        else hipLaunchKernelGGL((density_sub_kernel<2, 0>), g, b, 0, s, P, m4, keys, w2r, pw, vw, cells, n, mk);
-    }
+    auto run = [&](auto lanes) {
+        constexpr int LANES = decltype(lanes)::value;
+        const dim3 g(div_up(n, 256 / LANES)), b(256);
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, g, b, 0, s, P, m4, keys, w2r, pw, vw, cells, n, mk);
+        };
+        if (P.dim == 3) {
+            if (m) go(density_sub_kernel<3, 1, LANES>);
+            else go(density_sub_kernel<3, 0, LANES>);
+        } else {
+            if (m) go(density_sub_kernel<2, 1, LANES>);
+            else go(density_sub_kernel<2, 0, LANES>);
+        }
+    };
+    if (n <= SHARED_TARGETS) run(std::integral_constant<int, TARGET_LANES>{});
+    else run(std::integral_constant<int, 1>{});
     return check_launch("density_sub_kernel");
 }
 
@@ -234,22 +270,23 @@ int launch_density_sub(const cmag_params& P, float* measures, const uint32_t* ke
 // vector units 78 %), 32 B a neighbour.  16M dam break: 3.54 ms with registers
 // held so that six waves share a SIMD, 3.75 ms with seven (a spill inside the
 // pair loop), 3.56 ms with five.
-template <int DIM, int HASH, int CAP>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CAP <= 8 ? 6 : 1, 8))) void force_sub_kernel(
+template <int DIM, int HASH, int CAP, int LANES>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CAP <= 8 && LANES == 1 ? 6 : 1, 8))) void force_sub_kernel(
     const cmag_params P, float4* __restrict__ acc, const float4* __restrict__ posW, const float4* __restrict__ velW,
     const uint32_t* __restrict__ indexW, const uint32_t* __restrict__ keys, const SubCells cells, uint32_t n,
     const uint2* __restrict__ masks) {
     __shared__ uint32_t nbl[256 / 64][CAP][64];
     __shared__ LookupPlan lp;
     __shared__ LookupTables lt;
-    const uint32_t b0 = xcd_block() * blockDim.x;
-    const uint32_t i = b0 + threadIdx.x;
-    const bool staged = stage_lookups<DIM, HASH>(P, keys, cells, n, b0, lp, lt);
+    const uint32_t b0 = xcd_block() * (256 / LANES);
+    const uint32_t i = b0 + threadIdx.x / LANES;
+    const bool staged = stage_lookups<DIM, HASH>(P, keys, cells, n, b0, 256 / LANES, lp, lt);
     if (i >= n) return;
     // made in every block, so that the tables stay LDS addresses; used when staged
     const LookupView v = lookup_view<DIM>(lp, lt, keys[i], key_masks<HASH>(P).x);
-    force_body<CMAG_SYS_DAMBREAK, DIM, HASH, SubCells, CAP>(P, i, acc, nullptr, posW, velW, indexW, cells, n,
-                                                            nbl[threadIdx.x >> 6], &v, staged, masks, n);
+    force_body<CMAG_SYS_DAMBREAK, DIM, HASH, SubCells, CAP, LANES>(P, i, acc, nullptr, posW, velW, indexW, cells, n,
+                                                                   nbl[threadIdx.x >> 6], &v, staged, masks, n,
+                                                                   nullptr, nullptr, {}, threadIdx.x % LANES);
 }
 
 int launch_force_sub(const cmag_params& P, float* acc, const float* posW, const float* velW,
@@ -259,25 +296,27 @@ int launch_force_sub(const cmag_params& P, float* acc, const float* posW, const 
     if (n >= (1u << NB_SHIFT_BITS)) return fail(CMAG_E_INVALID, "force passes take at most 2^27 particles");
     if (P.system != CMAG_SYS_DAMBREAK) return fail(CMAG_E_INVALID, "the sub-cell walk is DamBreak's");
     const SubCells cells{cellFirst, reinterpret_cast<const uint4*>(pre)};
-    auto run = [&](auto dim, auto hash) {
-        constexpr int D = decltype(dim)::value, H = decltype(hash)::value;
-        if (masks)
-            hipLaunchKernelGGL((force_sub_kernel<D, H, 8>), dim3(div_up(n, 256)), dim3(256), 0, s, P,
-                               reinterpret_cast<float4*>(acc), reinterpret_cast<const float4*>(posW),
-                               reinterpret_cast<const float4*>(velW), indexW, keys, cells, n,
-                               reinterpret_cast<const uint2*>(masks));
-        else
-            hipLaunchKernelGGL((force_sub_kernel<D, H, NB_CAP>), dim3(div_up(n, 256)), dim3(256), 0, s, P,
-                               reinterpret_cast<float4*>(acc), reinterpret_cast<const float4*>(posW),
-                               reinterpret_cast<const float4*>(velW), indexW, keys, cells, n, nullptr);
+    auto run = [&](auto dim, auto hash, auto lanes) {
+        constexpr int D = decltype(dim)::value, H = decltype(hash)::value, LANES = decltype(lanes)::value;
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(div_up(n, 256 / LANES)), dim3(256), 0, s, P, reinterpret_cast<float4*>(acc),
+                               reinterpret_cast<const float4*>(posW), reinterpret_cast<const float4*>(velW), indexW,
+                               keys, cells, n, reinterpret_cast<const uint2*>(masks));
+        };
+        if (masks) go(force_sub_kernel<D, H, 8, LANES>);
+        else go(force_sub_kernel<D, H, NB_CAP, LANES>);
     };
-    const bool m = P.hash_order == CMAG_HASH_MORTON;
     using I2 = std::integral_constant<int, 2>;
     using I3 = std::integral_constant<int, 3>;
     using H0 = std::integral_constant<int, 0>;
     using H1 = std::integral_constant<int, 1>;
-    if (P.dim == 3) { if (m) run(I3{}, H1{}); else run(I3{}, H0{}); }
-    else { if (m) run(I2{}, H1{}); else run(I2{}, H0{}); }
+    auto pick = [&](auto lanes) {
+        const bool m = P.hash_order == CMAG_HASH_MORTON;
+        if (P.dim == 3) { if (m) run(I3{}, H1{}, lanes); else run(I3{}, H0{}, lanes); }
+        else { if (m) run(I2{}, H1{}, lanes); else run(I2{}, H0{}, lanes); }
+    };
+    if (n <= SHARED_TARGETS) pick(std::integral_constant<int, TARGET_LANES>{});
+    else pick(std::integral_constant<int, 1>{});
     return check_launch("force_sub_kernel");
 }
 

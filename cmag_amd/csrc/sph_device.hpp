@@ -69,14 +69,23 @@ struct RefCells {
     const uint32_t* __restrict__ cellEnd;
     uint32_t n;
     __device__ __forceinline__ bool range(uint32_t k0, uint32_t k1, uint32_t& s, uint32_t& e) const {
+        // up to three cells (a stencil of one cell a side) with their loads side
+        // by side; e clamped to the particle count: consistent cell arrays
+        // never need it, inconsistent ones cannot read past n
+        if (k1 - k0 <= 2u) {
+            const uint32_t km = min(k0 + 1u, k1);
+            const uint32_t s0 = cellStart[k0], s1 = cellStart[km], s2 = cellStart[k1];
+            const uint32_t e0 = cellEnd[k0], e1 = cellEnd[km], e2 = cellEnd[k1];
+            s = s0 != CMAG_CELL_EMPTY ? s0 : s1 != CMAG_CELL_EMPTY ? s1 : s2;
+            e = min(s2 != CMAG_CELL_EMPTY ? e2 : s1 != CMAG_CELL_EMPTY ? e1 : e0, n);
+            return s != CMAG_CELL_EMPTY && s < e;
+        }
         s = CMAG_CELL_EMPTY;
         e = 0;
         for (uint32_t k = k0; k <= k1; ++k) {
             const uint32_t st = cellStart[k];
             if (st == CMAG_CELL_EMPTY) continue;
             if (s == CMAG_CELL_EMPTY) s = st;
-            // clamped to the particle count: consistent cell arrays never
-            // need it, inconsistent ones cannot read past n
             e = min(cellEnd[k], n);
         }
         return s != CMAG_CELL_EMPTY && s < e;
@@ -162,9 +171,39 @@ struct Run {
 // target near the top of its cell has most of them above), so taking a pair's
 // mask bits as one sequence per lane evens the lanes' work out; the walks
 // without masks take the rows in the same order, so the sums are the same.
-__device__ __forceinline__ int force_row(int dim, int k) {
+struct RowList {
+    uint64_t rows;  // four bits each, first lowest
+    int count;
+    __device__ __forceinline__ int operator[](int k) const { return (int)((rows >> (4 * k)) & 15u); }
+};
+
+// Targets shared between lanes.  A neighbour pass is one serial chain per
+// target; with few targets the chip waits for it (20,000 rows fill a third of
+// the SIMDs with one wave).  TARGET_LANES lanes then share a target, each with
+// some of its stencil rows, and fold their sums: pairs of lanes first, then
+// both pairs.  The same lanes take the same rows in the same order wherever
+// the neighbours come from (global walk, staged lookups, masks).
+constexpr int TARGET_LANES = 4;
+__device__ __forceinline__ float quad_sum(float v) {
+    // quad_perm [1,0,3,2], then [2,3,0,1]
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true));
+    return v;
+}
+
+// the rows of lane `part` of LANES in the force pass.  Shared: two edge pairs,
+// each with one row of a corner pair, the centre row, and the other corner
+// pair: about 24, 24, 16 and 10 of the 74 in-range neighbours, in two turns
+template <int LANES>
+__device__ __forceinline__ RowList force_rows(int dim, uint32_t part) {
+    static_assert(LANES == 1 || LANES == TARGET_LANES, "one lane or a quad");
     // 3-D: 0 8 2 6 3 5 1 7 4; 2-D: 0 2 1
-    return dim == 3 ? (int)((0x471536280ull >> (4 * k)) & 15u) : (k == 0 ? 0 : k == 1 ? 2 : 1);
+    if (LANES == 1) return dim == 3 ? RowList{0x471536280ull, 9} : RowList{0x120ull, 3};
+    if (dim == 3) {
+        const uint64_t rows = part == 0 ? 0x253ull : part == 1 ? 0x671ull : part == 2 ? 0x4ull : 0x80ull;
+        return RowList{rows, part < 2 ? 3 : part == 2 ? 1 : 2};
+    }
+    return RowList{part == 0 ? 0x0ull : part == 1 ? 0x2ull : 0x1ull, part < 3 ? 1 : 0};
 }
 
 // Walk the stencil of gp in z, y, x order and call cand(j, qx, qy, qz, code)
@@ -188,7 +227,7 @@ __device__ __forceinline__ int force_row(int dim, int k) {
 // walk_rows does the walk and hands each row's runs to row(a, b, qy, qz, whole);
 // whole: the whole row comes in this one call (in every lane of the wave).
 // walk_stencil and walk_stencil_pf turn them into candidate calls.  With
-// FORCE_ORDER and one cell per stencil side, the rows come in force_row order.
+// FORCE_ORDER and one cell per stencil side, the rows come in force_rows order.
 // With LANES > 1 that many lanes share the target: this one takes the rows
 // part, part + LANES, ...
 template <int DIM, int HASH, bool PERIODIC = true, bool FORCE_ORDER = false, int LANES = 1, typename Cells, typename R>
@@ -352,11 +391,11 @@ __device__ __forceinline__ void walk_rows(const cmag_params& P, const float4& pi
     };
     const int zlo = DIM == 2 ? 0 : -cc, zhi = DIM == 2 ? 0 : cc;
     if (FORCE_ORDER && cc == 1) {
-        // the force pass's row order (force_row), as its staged blocks take it;
+        // the force pass's row order (force_rows), as its staged blocks take it;
         // the Morton key parts are stepped from the stencil's first row each time
-        constexpr int NR = DIM == 3 ? 9 : 3;
-        for (int k = 0; k < NR; ++k) {
-            const int r = force_row(DIM, k);
+        const RowList list = force_rows<LANES>(DIM, part);
+        for (int k = 0; k < list.count; ++k) {
+            const int r = list[k];
             const int iy = r % 3, iz = DIM == 3 ? r / 3 : 0;
             uint32_t ky = ky0, kz = kz0;
             if (HASH == CMAG_HASH_MORTON) {
@@ -493,20 +532,22 @@ __device__ __forceinline__ void walk_row_two(const Run& a, const Run& b, const f
     }
 }
 
-template <int DIM, int HASH, bool PERIODIC = true, bool FORCE_ORDER = false, typename Cells, typename C>
+template <int DIM, int HASH, bool PERIODIC = true, bool FORCE_ORDER = false, int LANES = 1, typename Cells, typename C>
 __device__ __forceinline__ void walk_stencil_pf(const cmag_params& P, const float4& pi, const Cell& gp,
-                                                const Cells& cells, const float4* __restrict__ pos, C&& cand) {
+                                                const Cells& cells, const float4* __restrict__ pos, C&& cand,
+                                                uint32_t part = 0) {
     if constexpr (Cells::SUB) {
-        walk_rows<DIM, HASH, PERIODIC, FORCE_ORDER>(P, pi, gp, cells,
+        walk_rows<DIM, HASH, PERIODIC, FORCE_ORDER, LANES>(P, pi, gp, cells,
                                                     [&](const Run& a, const Run& b, float py, float pz, bool) {
             walk_run_sub(pos, a.s, a.s + a.len, a.px, py, pz, a.code, cand);
             walk_run_sub(pos, b.s, b.s + b.len, b.px, py, pz, b.code, cand);
-        });
+        }, part);
         return;
     }
-    walk_rows<DIM, HASH, PERIODIC>(P, pi, gp, cells, [&](const Run& a, const Run& b, float py, float pz, bool) {
+    walk_rows<DIM, HASH, PERIODIC, false, LANES>(P, pi, gp, cells,
+                                                 [&](const Run& a, const Run& b, float py, float pz, bool) {
         walk_row_pf<Cells::PADDED>(a, b, py, pz, pos, cand);
-    });
+    }, part);
 }
 
 // ---- cell lookups staged in LDS (sub-cell walk) -----------------------------
@@ -573,8 +614,9 @@ __device__ __forceinline__ LookupView lookup_view(const LookupPlan& lp, const Lo
     return v;
 }
 
-// All threads of the block (whole waves, at most four) call this; returns
-// whether the block's lookups are staged.  keys: the sorted cell keys (a sub-cell row lies in the same cell as
+// All threads of the block (whole waves, at most four) call this for its
+// targets b0, b0 + 1, ... (at most one a thread); returns whether the block's
+// lookups are staged.  keys: the sorted cell keys (a sub-cell row lies in the same cell as
 // the reference-order row of its number).  Everything is found from the keys'
 // bits by every thread at once: one barrier and one pass of loads until the
 // tables are filled.  (When one thread worked out the block's 22 keys from
@@ -582,12 +624,12 @@ __device__ __forceinline__ LookupView lookup_view(const LookupPlan& lp, const Lo
 // chain was a tenth of a block's life.)
 template <int DIM, int HASH>
 __device__ __forceinline__ bool stage_lookups(const cmag_params& P, const uint32_t* __restrict__ keys,
-                                              const SubCells& cells, uint32_t n, uint32_t b0, LookupPlan& lp,
-                                              LookupTables& lt) {
+                                              const SubCells& cells, uint32_t n, uint32_t b0, uint32_t targets,
+                                              LookupPlan& lp, LookupTables& lt) {
     constexpr int R = DIM == 3 ? 9 : 3;
     if (P.cellcount != 1 || b0 >= n) return false;
     const KeyMasks M = key_masks<HASH>(P);
-    const uint32_t count = min(blockDim.x, n - b0);
+    const uint32_t count = min(targets, n - b0);
     const uint32_t tid = threadIdx.x;
     const uint32_t mine = keys[b0 + min(tid, count - 1u)];
     const uint32_t k0 = keys[b0], k1 = keys[b0 + count - 1u];
@@ -707,11 +749,11 @@ __device__ __forceinline__ void stage_rows(const LookupPlan& lp, const LookupTab
 
 // the candidates of target pi through its view of the staged
 // lookups, as walk_stencil_pf hands them; with ROWS, the stencil rows that
-// stage_rows copied are read from LDS; with FORCE_ORDER, rows in force_row order
-template <int DIM, bool ROWS = false, bool FORCE_ORDER = false, typename C>
+// stage_rows copied are read from LDS; with FORCE_ORDER, rows in force_rows order
+template <int DIM, bool ROWS = false, bool FORCE_ORDER = false, int LANES = 1, typename C>
 __device__ __forceinline__ void walk_lookup(const cmag_params& P, const float4& pi, const LookupView& v,
                                             const float4* __restrict__ pos, C&& cand, const RowStage* rs = nullptr,
-                                            const RowLds* lds = nullptr) {
+                                            const RowLds* lds = nullptr, uint32_t part = 0) {
     constexpr int R = DIM == 3 ? 9 : 3;
     const int q = x_sub(P, pi.x);
     auto run_lds = [&](uint32_t s, uint32_t e, int32_t off) {
@@ -724,8 +766,10 @@ __device__ __forceinline__ void walk_lookup(const cmag_params& P, const float4& 
             cand(j + 1u, p1, j + 1u < e, pi.x, pi.y, pi.z, 13);
         }
     };
-    for (int k = 0; k < R; ++k) {
-        const int r = FORCE_ORDER ? force_row(DIM, k) : k;
+    const RowList list = force_rows<LANES>(DIM, part);
+    const int k0 = FORCE_ORDER ? 0 : (int)part, k1 = FORCE_ORDER ? list.count : R;
+    for (int k = k0; k < k1; k += FORCE_ORDER ? 1 : LANES) {
+        const int r = FORCE_ORDER ? list[k] : k;
         const uint32_t s = v.F(r, 0) + SubCells::below(v.Pr(r, 0), q);
         const uint32_t f1 = v.F(r, 2);
         const uint4* c1 = v.Pr(r, 2);
@@ -775,11 +819,11 @@ __device__ __forceinline__ uint32_t shift_in_less(uint32_t m, float a, float b) 
 // density of the target pi over a staged block's lookups, as
 // density_sum_lookup, writing the in-range masks of its rows' main runs to
 // masks[r * stride + i] (fluid targets only)
-template <int DIM>
+template <int DIM, int LANES>
 __device__ __forceinline__ float density_sum_masks(const cmag_params& P, const float4& pi, const LookupView& v,
-                                                   const RowStage& rs, const RowLds* lds,
+                                                   const RowStage* rs, const RowLds* lds,
                                                    const float4* __restrict__ pos, uint2* __restrict__ masks,
-                                                   uint32_t i, uint32_t stride) {
+                                                   uint32_t i, uint32_t stride, uint32_t part) {
     constexpr int R = DIM == 3 ? 9 : 3;
     const int q = x_sub(P, pi.x);
     const float half_inv_h = -0.5f / P.smoothing_radius;
@@ -796,7 +840,7 @@ __device__ __forceinline__ float density_sum_masks(const cmag_params& P, const f
     auto cand = [&](uint32_t, const float4& pj, bool valid, float, float, float, int) {
         term(valid ? d2(pj) : 1e30f);
     };
-    for (int r = 0; r < R; ++r) {
+    for (int r = (int)part; r < R; r += LANES) {
         const uint4* c0 = v.Pr(r, 0);
         const uint32_t f0 = v.F(r, 0);
         const uint32_t s = f0 + SubCells::below(c0, q);
@@ -804,7 +848,7 @@ __device__ __forceinline__ float density_sum_masks(const cmag_params& P, const f
         const uint4* c1 = v.Pr(r, 2);
         const uint32_t e = f1 + SubCells::through(c1, q), ws = f1 + SubCells::fluid(c1), we = v.F(r, 3);
         uint32_t m0 = 0, m1 = 0;
-        const bool in_lds = DIM == 3 && rs.ok && r >= ROW_STAGE_FIRST && r < ROW_STAGE_FIRST + ROW_STAGE_ROWS;
+        const bool in_lds = DIM == 3 && LANES == 1 && rs->ok && r >= ROW_STAGE_FIRST && r < ROW_STAGE_FIRST + ROW_STAGE_ROWS;
         // two candidates per step; `at` steps through the run by `row` a candidate
         auto scan = [&](auto at, auto row, auto&& ld) {
             const auto end = at + (e - s) * row, last = end - row;
@@ -837,7 +881,7 @@ __device__ __forceinline__ float density_sum_masks(const cmag_params& P, const f
             }
         };
         if (in_lds) {
-            scan(lds->row + ((int32_t)s + rs.off[r - ROW_STAGE_FIRST]), 1u,
+            scan(lds->row + ((int32_t)s + rs->off[r - ROW_STAGE_FIRST]), 1u,
                  [&](const RowLds::Row* q, float4& p0, float4& p1) {
                      p0 = make_float4(q[0].x, q[0].y, q[0].z, 0.0f);
                      p1 = make_float4(q[1].x, q[1].y, q[1].z, 0.0f);
@@ -865,7 +909,7 @@ __device__ __forceinline__ float density_sum_masks(const cmag_params& P, const f
         }
         if (fluid) masks[(size_t)r * stride + i] = make_uint2(lo, hi);
         if (in_lds) {
-            const int32_t off = rs.off[r - ROW_STAGE_FIRST];
+            const int32_t off = rs->off[r - ROW_STAGE_FIRST];
             for (uint32_t j = ws; j < we; j += 2u) {
                 const int32_t l = (int32_t)j + off;
                 const RowLds::Row a0 = lds->row[l], a1 = lds->row[l + 1];
@@ -876,6 +920,7 @@ __device__ __forceinline__ float density_sum_masks(const cmag_params& P, const f
             walk_run_sub(pos, ws, we, pi.x, pi.y, pi.z, 13, cand);
         }
     }
+    if (LANES > 1) sum = quad_sum(sum);
     return sum * P.kernel_coeff * P.particle_mass;
 }
 
@@ -939,13 +984,14 @@ struct NbQueue {
 // ---------------------------------------------------------------------------
 // the density of the particle at pi: the mass-weighted kernel sum over the
 // stencil (the particle itself included)
-template <int SYS, int DIM, int HASH, typename Cells>
+template <int SYS, int DIM, int HASH, int LANES = 1, typename Cells>
 __device__ __forceinline__ float density_sum(const cmag_params& P, const float4& pi,
-                                             const float4* __restrict__ sortedPos, const Cells& cells) {
+                                             const float4* __restrict__ sortedPos, const Cells& cells,
+                                             uint32_t part = 0) {
     const Cell gp = grid_pos(P, pi.x, pi.y, pi.z);
     const float half_inv_h = -0.5f / P.smoothing_radius;
     float sum = 0.0f;
-    walk_stencil_pf<DIM, HASH, SYS != CMAG_SYS_DAMBREAK>(P, pi, gp, cells, sortedPos,
+    walk_stencil_pf<DIM, HASH, SYS != CMAG_SYS_DAMBREAK, false, LANES>(P, pi, gp, cells, sortedPos,
                                                          [&](uint32_t, const float4& pj, bool valid, float px,
                                                              float py, float pz, int) {
         // a candidate past the run sits at r^2 = 1e30: t = 0 and it adds +0
@@ -956,23 +1002,25 @@ __device__ __forceinline__ float density_sum(const cmag_params& P, const float4&
         const float t = fminf(fmaxf(fmaf(half_inv_h, fsqrt(r2), 1.0f), 0.0f), 1.0f);
         const float t2 = t * t;
         sum = fmaf(t2 * t2, fmaf(-4.0f, t, 5.0f), sum);
-    });
+    }, part);
+    if (LANES > 1) sum = quad_sum(sum);
     return sum * P.kernel_coeff * P.particle_mass;
 }
 
-template <int DIM>
+template <int DIM, int LANES>
 __device__ __forceinline__ float density_sum_lookup(const cmag_params& P, const float4& pi, const LookupView& v,
-                                                    const RowStage& rs, const RowLds* lds,
-                                                    const float4* __restrict__ pos) {
+                                                    const RowStage* rs, const RowLds* lds,
+                                                    const float4* __restrict__ pos, uint32_t part) {
     const float half_inv_h = -0.5f / P.smoothing_radius;
     float sum = 0.0f;
-    walk_lookup<DIM, true>(P, pi, v, pos,
+    walk_lookup<DIM, LANES == 1, false, LANES>(P, pi, v, pos,
                            [&](uint32_t, const float4& pj, bool valid, float px, float py, float pz, int) {
         const float r2 = valid ? norm2(px - pj.x, py - pj.y, pz - pj.z) : 1e30f;
         const float t = fminf(fmaxf(fmaf(half_inv_h, fsqrt(r2), 1.0f), 0.0f), 1.0f);
         const float t2 = t * t;
         sum = fmaf(t2 * t2, fmaf(-4.0f, t, 5.0f), sum);
-    }, &rs, lds);
+    }, rs, lds, part);
+    if (LANES > 1) sum = quad_sum(sum);
     return sum * P.kernel_coeff * P.particle_mass;
 }
 
@@ -997,7 +1045,7 @@ __device__ __forceinline__ float density_sum_rows(const cmag_params& P, const fl
     const Cell gp = grid_pos(P, pi.x, pi.y, pi.z);
     const float half_inv_h = -0.5f / P.smoothing_radius;
     const float r2max = 4.0f * P.smoothing_radius * P.smoothing_radius;
-    float sum = 0.0f;
+    float sum = 0.0f, total_sum = 0.0f;
     uint32_t* out = MASKS ? masks + i : nullptr;
     walk_rows<DIM, HASH, SYS != CMAG_SYS_DAMBREAK>(P, pi, gp, cells,
                                                    [&](const Run& a, const Run& b, float py, float pz, bool whole) {
@@ -1017,6 +1065,12 @@ __device__ __forceinline__ float density_sum_rows(const cmag_params& P, const fl
                 m = shift_in_less(m, rb, r2max);
             }
         });
+        // the dam break's 100 to 500 candidates a target: a sum per row, as the
+        // lanes of a shared target form them, keeps the error at a row's
+        if (SYS == CMAG_SYS_DAMBREAK) {
+            total_sum += sum;
+            sum = 0.0f;
+        }
         if (MASKS && whole) {
             // candidate t was shifted in K - 1 - t places from the right, K even
             const uint32_t total = a.len + b.len, K = (total + 1u) & ~1u;
@@ -1025,16 +1079,18 @@ __device__ __forceinline__ float density_sum_rows(const cmag_params& P, const fl
             out += stride;
         }
     });
+    if (SYS == CMAG_SYS_DAMBREAK) sum = total_sum;
     return sum * P.kernel_coeff * P.particle_mass;
 }
 
 // pairs (optional): what a neighbour's pair terms need of the density pass,
 // (p / rho, 1 / rho) in the reciprocal the terms use; masks (optional): as above
-template <int SYS, int DIM, int HASH, typename Cells>
+template <int SYS, int DIM, int HASH, int LANES = 1, typename Cells>
 __device__ __forceinline__ void density_body(const cmag_params& P, uint32_t i, float4* __restrict__ measures,
                                              const float4* __restrict__ sortedPos, const Cells& cells,
                                              float2* __restrict__ pairs = nullptr,
-                                             uint32_t* __restrict__ masks = nullptr, uint32_t stride = 0) {
+                                             uint32_t* __restrict__ masks = nullptr, uint32_t stride = 0,
+                                             uint32_t part = 0) {
     const float4 pi = sortedPos[i];
     float2* m2 = reinterpret_cast<float2*>(measures);
     const bool rest = SYS == CMAG_SYS_POISEUILLE && pi.w == CMAG_PO_WALL;
@@ -1046,8 +1102,9 @@ __device__ __forceinline__ void density_body(const cmag_params& P, uint32_t i, f
         else if (!rest)
             dens = density_sum_rows<SYS, DIM, HASH, false>(P, pi, sortedPos, cells, nullptr, i, stride);
     } else {
-        if (!rest) dens = density_sum<SYS, DIM, HASH>(P, pi, sortedPos, cells);
+        if (!rest) dens = density_sum<SYS, DIM, HASH, LANES>(P, pi, sortedPos, cells, part);
     }
+    if (LANES > 1 && part != 0) return;
     if (rest) dens = P.rest_density;
     const float p = eos(P, dens);
     if (SYS == CMAG_SYS_PERISTALSIS) {
@@ -1259,7 +1316,7 @@ __device__ __forceinline__ float2 pair_values(const float2* __restrict__ pairs, 
 // queue; the walls of the row's first two cells are walked on their own.  Pair
 // terms keep the walk's order and wall terms accumulate apart, so the sums are
 // the same bit for bit.
-template <int SYS, int DIM, int HASH, typename Cells, int CAP = NB_CAP>
+template <int SYS, int DIM, int HASH, typename Cells, int CAP = NB_CAP, int LANES = 1>
 __device__ __forceinline__ void force_body(const cmag_params& P, uint32_t i, float4* __restrict__ acc,
                                            const float4* __restrict__ measures,
                                            const float4* __restrict__ sortedPos,
@@ -1269,7 +1326,7 @@ __device__ __forceinline__ void force_body(const cmag_params& P, uint32_t i, flo
                                            const uint2* __restrict__ masks = nullptr, uint32_t stride = 0,
                                            const float2* __restrict__ pv = nullptr,
                                            const uint32_t* __restrict__ row_masks = nullptr,
-                                           const StepArrays& step = {}) {
+                                           const StepArrays& step = {}, uint32_t part = 0) {
     const int lane = threadIdx.x & 63;
     constexpr bool PACKED = SYS == CMAG_SYS_DAMBREAK && Cells::SUB;
     auto is_wall = [](float w) { return PACKED ? __float_as_int(w) >= 0 : w != CMAG_DB_FLUID; };
@@ -1339,7 +1396,6 @@ __device__ __forceinline__ void force_body(const cmag_params& P, uint32_t i, flo
     };
     if constexpr (Cells::SUB) {
         if (staged && masks) {
-            constexpr int R = DIM == 3 ? 9 : 3;
             const LookupView& v = *lp;
             const int q = x_sub(P, pi.x);
             // the main run [s, e) of row r: cells x - 1 (from eighth q) to
@@ -1397,9 +1453,10 @@ __device__ __forceinline__ void force_body(const cmag_params& P, uint32_t i, flo
                     pairs(j0, j1, two);
                 }
             };
-            // rows in force_row order, two at a time (the centre row alone)
-            for (int k = 0; k < R; k += 2) {
-                const int ra = force_row(DIM, k), rb = k + 1 < R ? force_row(DIM, k + 1) : -1;
+            // rows in force_rows order, two at a time (the last alone)
+            const RowList list = force_rows<LANES>(DIM, part);
+            for (int k = 0; k < list.count; k += 2) {
+                const int ra = list[k], rb = k + 1 < list.count ? list[k + 1] : -1;
                 // both masks are loaded ahead of the walls (a walked row's is not used)
                 const uint2 wa = masks[(size_t)ra * stride + i];
                 const uint2 wb = rb >= 0 ? masks[(size_t)rb * stride + i] : make_uint2(0u, 0u);
@@ -1439,16 +1496,21 @@ __device__ __forceinline__ void force_body(const cmag_params& P, uint32_t i, flo
                 }
             }
         } else if (staged) {
-            walk_lookup<DIM, false, true>(P, pi, *lp, sortedPos, cand);
+            walk_lookup<DIM, false, true, LANES>(P, pi, *lp, sortedPos, cand, nullptr, nullptr, part);
         } else {
-            walk_stencil_pf<DIM, HASH, false, true>(P, pi, gp, cells, sortedPos, cand);
+            walk_stencil_pf<DIM, HASH, false, true, LANES>(P, pi, gp, cells, sortedPos, cand, part);
         }
     } else if (SYS != CMAG_SYS_DAMBREAK && DIM == 2 && HASH == CMAG_HASH_LINEAR && Cells::PADDED && row_masks) {
         walk_row_masks<HASH>(P, i, pi, gp, cells, sortedPos, row_masks, stride, nq, cand, queued_pairs);
     } else {
-        walk_stencil_pf<DIM, HASH, SYS != CMAG_SYS_DAMBREAK>(P, pi, gp, cells, sortedPos, cand);
+        walk_stencil_pf<DIM, HASH, SYS != CMAG_SYS_DAMBREAK, false, LANES>(P, pi, gp, cells, sortedPos, cand, part);
     }
     nq.drain(CAP, queued_pairs);
+    if (LANES > 1) {
+        F.fx = quad_sum(F.fx); F.fy = quad_sum(F.fy); F.fz = quad_sum(F.fz);
+        F.wx = quad_sum(F.wx); F.wy = quad_sum(F.wy); F.wz = quad_sum(F.wz);
+        if (part != 0) return;
+    }
     const uint32_t k = index[i];
     if (k >= n) return;
     const float4 a = make_float4(F.fx + F.wx, F.fy + F.wy, F.fz + F.wz, 0.0f);
