@@ -314,16 +314,18 @@ int CellSort::alloc(size_t cells_, uint32_t n_, hipStream_t s) {
 }
 
 int CellSort::alloc_walk(hipStream_t s) {
-    const size_t halves = (cells + OFF_ITEMS - 1) / OFF_ITEMS;
-    CMAG_HIP_TRY(hipMalloc((void**)&occ, sizeof(uint16_t) * halves));
-    CMAG_HIP_TRY(hipMemsetAsync(occ, 0, sizeof(uint16_t) * halves, s));
-    CMAG_HIP_TRY(hipMalloc((void**)&pre, sizeof(uint32_t) * 4 * cells));
-    CMAG_HIP_TRY(hipMemsetAsync(pre, 0, sizeof(uint32_t) * 4 * cells, s));
+    if (pre) return CMAG_OK;
+    // pre, then occ, in one allocation that starts as zeros
+    const size_t counts = sizeof(uint32_t) * 4 * cells, halves = (cells + OFF_ITEMS - 1) / OFF_ITEMS;
+    const size_t bytes = counts + sizeof(uint16_t) * halves;
+    CMAG_HIP_TRY(hipMalloc((void**)&pre, bytes));
+    occ = reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(pre) + counts);
+    CMAG_HIP_TRY(hipMemsetAsync(pre, 0, bytes, s));
     return CMAG_OK;
 }
 
 void CellSort::release() {
-    void* bufs[] = {arena, occ, pre};
+    void* bufs[] = {arena, pre};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
 }

@@ -8,6 +8,7 @@
 
 #include <cmath>
 #include <cstring>
+#include <initializer_list>
 #include <new>
 #include <vector>
 
@@ -26,6 +27,7 @@ struct cmag_system {
     hipStream_t stream = nullptr;
     hipStream_t own_stream = nullptr;
 
+    void *arena = nullptr, *walk_arena = nullptr;  // the buffers below; those of the sub-cell walk
     float *pos = nullptr, *vel = nullptr, *velLF = nullptr, *acc = nullptr, *presF = nullptr;
     float *measures = nullptr, *sortedPos = nullptr, *sortedVel = nullptr, *predicted = nullptr;
     uint32_t *hash = nullptr, *index = nullptr;
@@ -103,9 +105,7 @@ struct cmag_system {
         if (graph) (void)hipGraphExecDestroy(graph);
         for (hipEvent_t e : ev)
             if (e) (void)hipEventDestroy(e);
-        void* bufs[] = {pos, vel, velLF, acc, presF, measures, sortedPos, sortedVel, predicted,
-                        hash, index, cellStart, cellEnd, cellFirst,
-                        gaccS, gposS, gvelS, grho, gterms, dState, posW, velW, indexW, w2r, masks, pairs, rowMasks, color};
+        void* bufs[] = {arena, walk_arena, gaccS, gposS, gvelS, grho, gterms, color};
         for (void* b : bufs)
             if (b) (void)hipFree(b);
         for (void* b : kept) (void)hipFree(b);
@@ -113,35 +113,49 @@ struct cmag_system {
         if (own_stream) (void)hipStreamDestroy(own_stream);
     }
 
+    // one allocation for all of bufs, each on a 256-byte boundary: an
+    // allocation costs 20 to 60 us, a System has some twenty buffers
+    struct Buf {
+        void** at;
+        size_t bytes;
+    };
+    static int alloc_arena(void** arena, std::initializer_list<Buf> bufs) {
+        auto part = [](size_t bytes) { return (bytes + 255) & ~(size_t)255; };
+        size_t total = 0;
+        for (const Buf& b : bufs) total += part(b.bytes);
+        CMAG_HIP_TRY(hipMalloc(arena, total));
+        char* at = static_cast<char*>(*arena);
+        for (const Buf& b : bufs) {
+            *b.at = b.bytes ? at : nullptr;
+            at += part(b.bytes);
+        }
+        return CMAG_OK;
+    }
+    template <typename T>
+    static Buf buf(T*& p, size_t bytes) {
+        return Buf{reinterpret_cast<void**>(&p), bytes};
+    }
+
     int alloc() {
         const size_t f4 = sizeof(float) * 4 * (size_t)(n ? n : 1);
         const size_t u = sizeof(uint32_t) * (size_t)(n ? n : 1);
+        const size_t c = sizeof(uint32_t) * (size_t)numCells;
+        const bool peri = P.system == CMAG_SYS_PERISTALSIS, channel = P.system != CMAG_SYS_DAMBREAK;
         CMAG_HIP_TRY(hipStreamCreate(&own_stream));
         stream = own_stream;
-        float** fb[] = {&pos, &vel, &velLF, &acc, &measures, &sortedPos, &sortedVel};
-        // padding rows: the neighbour walks read up to two rows past a run
-        for (float** b : fb) CMAG_HIP_TRY(hipMalloc((void**)b, f4 + (b == &sortedPos ? 64 : 0)));
-        if (P.system == CMAG_SYS_PERISTALSIS) {
-            CMAG_HIP_TRY(hipMalloc((void**)&presF, f4));
-            CMAG_HIP_TRY(hipMalloc((void**)&predicted, f4));
-            CMAG_HIP_TRY(hipMalloc((void**)&dState, sizeof(StepState)));
-        }
-        if (P.system != CMAG_SYS_DAMBREAK) {
-            CMAG_HIP_TRY(hipMalloc((void**)&pairs, f4 / 2));
-            if (row_masks_apply(P)) CMAG_HIP_TRY(hipMalloc((void**)&rowMasks, u * ROW_MASK_ROWS));
-        }
-        uint32_t** ub[] = {&hash, &index};
-        for (uint32_t** b : ub) CMAG_HIP_TRY(hipMalloc((void**)b, u));
-        CMAG_HIP_TRY(hipMalloc((void**)&cellStart, sizeof(uint32_t) * (size_t)numCells));
-        CMAG_HIP_TRY(hipMalloc((void**)&cellEnd, sizeof(uint32_t) * (size_t)numCells));
-        CMAG_HIP_TRY(hipMalloc((void**)&cellFirst, sizeof(uint32_t) * ((size_t)numCells + 1)));
+        // what starts as zeros comes first; padding rows: the neighbour walks
+        // read up to two rows past a run
+        CMAG_TRY(alloc_arena(&arena, {buf(pos, f4), buf(vel, f4), buf(velLF, f4), buf(acc, f4), buf(measures, f4),
+                                      buf(sortedPos, f4 + 64), buf(sortedVel, f4), buf(presF, peri ? f4 : 0),
+                                      buf(predicted, peri ? f4 : 0), buf(hash, u), buf(index, u), buf(cellEnd, c),
+                                      buf(cellStart, c), buf(cellFirst, c + sizeof(uint32_t)),
+                                      buf(pairs, channel ? f4 / 2 : 0),
+                                      buf(rowMasks, row_masks_apply(P) ? u * ROW_MASK_ROWS : 0),
+                                      buf(dState, peri ? sizeof(StepState) : 0)}));
         CMAG_TRY(sort.alloc(numCells, n, stream));
-        float* zb[] = {pos, vel, velLF, acc, measures, sortedPos, sortedVel, presF, predicted};
-        for (float* b : zb)
-            if (b) CMAG_HIP_TRY(hipMemsetAsync(b, 0, f4, stream));
-        for (uint32_t* b : {hash, index}) CMAG_HIP_TRY(hipMemsetAsync(b, 0, u, stream));
-        CMAG_HIP_TRY(hipMemsetAsync(cellStart, 0xff, sizeof(uint32_t) * (size_t)numCells, stream));
-        CMAG_HIP_TRY(hipMemsetAsync(cellEnd, 0, sizeof(uint32_t) * (size_t)numCells, stream));
+        CMAG_HIP_TRY(hipMemsetAsync(arena, 0, (size_t)(reinterpret_cast<char*>(cellStart) - static_cast<char*>(arena)),
+                                    stream));
+        CMAG_HIP_TRY(hipMemsetAsync(cellStart, 0xff, c, stream));
         CMAG_HIP_TRY(hipStreamSynchronize(stream));
         return CMAG_OK;
     }
@@ -163,11 +177,10 @@ struct cmag_system {
         if (on && !posW) {
             const size_t f4 = sizeof(float) * 4 * (size_t)(n ? n : 1);
             const size_t u = sizeof(uint32_t) * (size_t)(n ? n : 1);
-            // padding rows: the walk reads up to two rows past a run
-            for (float** b : {&posW, &velW}) CMAG_HIP_TRY(hipMalloc((void**)b, f4 + 64));
-            for (uint32_t** b : {&indexW, &w2r}) CMAG_HIP_TRY(hipMalloc((void**)b, u));
             CMAG_TRY(sort.alloc_walk(stream));
-            CMAG_HIP_TRY(hipMalloc((void**)&masks, sizeof(uint32_t) * MASK_WORDS * (size_t)(n ? n : 1)));
+            // padding rows: the walk reads up to two rows past a run
+            CMAG_TRY(alloc_arena(&walk_arena, {buf(posW, f4 + 64), buf(velW, f4 + 64), buf(indexW, u), buf(w2r, u),
+                                               buf(masks, u * MASK_WORDS)}));
         }
         if (on != subwalk) invalidate_graph();
         subwalk = on;
