@@ -72,8 +72,10 @@ struct cmag_system {
     StepState* dState = nullptr;
     bool state_dirty = true;
 
-    hipGraphExec_t graph = nullptr;
+    // one captured step, and many_steps of them
+    hipGraphExec_t graph = nullptr, many = nullptr;
     bool graph_valid = false;
+    uint32_t many_steps = 0, last_run = 0;
 
     // per-stage event timing: ev[k] recorded before stage k, ev[NUM] after the last
     bool timing = false;
@@ -102,7 +104,7 @@ struct cmag_system {
     }
 
     ~cmag_system() {
-        if (graph) (void)hipGraphExecDestroy(graph);
+        invalidate_graph();
         for (hipEvent_t e : ev)
             if (e) (void)hipEventDestroy(e);
         void* bufs[] = {arena, walk_arena, gaccS, gposS, gvelS, grho, gterms, color};
@@ -277,18 +279,20 @@ struct cmag_system {
 
     void invalidate_graph() {
         if (graph) (void)hipGraphExecDestroy(graph);
-        graph = nullptr;
+        if (many) (void)hipGraphExecDestroy(many);
+        graph = many = nullptr;
         graph_valid = false;
+        many_steps = last_run = 0;
     }
 
-    int build_graph() {
-        invalidate_graph();
+    int capture_steps(uint32_t steps, hipGraphExec_t* out) {
         if (stream == nullptr) return fail(CMAG_E_STATE, "graph capture needs a non-default stream");
         hipGraph_t g = nullptr;
         const bool was_timing = timing;
         timing = false;  // no event nodes inside the graph
         CMAG_HIP_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-        int rc = enqueue_step();
+        int rc = CMAG_OK;
+        for (uint32_t k = 0; k < steps && rc == CMAG_OK; ++k) rc = enqueue_step();
         timing = was_timing;
         hipError_t e = hipStreamEndCapture(stream, &g);
         if (rc != CMAG_OK) {
@@ -296,10 +300,41 @@ struct cmag_system {
             return rc;
         }
         if (e != hipSuccess) return hip_fail(e, "hipStreamEndCapture");
-        e = hipGraphInstantiate(&graph, g, nullptr, nullptr, 0);
+        e = hipGraphInstantiate(out, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
-        if (e != hipSuccess) return hip_fail(e, "hipGraphInstantiate");
+        if (e != hipSuccess) {
+            *out = nullptr;
+            return hip_fail(e, "hipGraphInstantiate");
+        }
+        return CMAG_OK;
+    }
+
+    int build_graph() {
+        invalidate_graph();
+        CMAG_TRY(capture_steps(1, &graph));
         graph_valid = true;
+        return CMAG_OK;
+    }
+
+    // A graph launch costs the host and the gap to the next one what two or
+    // three of a step's six or seven kernels do, so steps are launched several
+    // at a time once a second run() in a row asks for as many: the first pass
+    // captures one step only, and counts that change never capture again (a
+    // larger graph replaces a smaller one, so MANY_STEPS - 1 times at most).
+    static constexpr uint32_t MANY_STEPS = 16;
+    int grow_graph(uint32_t steps) {
+        const uint32_t want = steps < MANY_STEPS ? steps : MANY_STEPS;
+        const bool again = want == last_run;
+        last_run = want;
+        if (!again || want < 2 || want <= many_steps) return CMAG_OK;
+        hipGraphExec_t g = nullptr;
+        CMAG_TRY(capture_steps(want, &g));
+        if (many) {
+            (void)hipStreamSynchronize(stream);  // it may be running
+            (void)hipGraphExecDestroy(many);
+        }
+        many = g;
+        many_steps = want;
         return CMAG_OK;
     }
 
@@ -310,11 +345,13 @@ struct cmag_system {
         }
         CMAG_TRY(collect());
         CMAG_TRY(upload_state());
-        if (!graph_valid) CMAG_TRY(build_graph());
         CMAG_TRY(sort.ready(stream));
-        for (uint32_t k = 0; k < steps; ++k) {
-            CMAG_HIP_TRY(hipGraphLaunch(graph, stream));
-            advance_clock();
+        if (!graph_valid) CMAG_TRY(build_graph());
+        CMAG_TRY(grow_graph(steps));
+        for (uint32_t k = 0; k < steps;) {
+            const bool several = many && steps - k >= many_steps;
+            CMAG_HIP_TRY(hipGraphLaunch(several ? many : graph, stream));
+            for (uint32_t t = several ? many_steps : 1; t > 0; --t, ++k) advance_clock();
         }
         return CMAG_OK;
     }

@@ -48,6 +48,39 @@ def test_system(device, kind, moving, n):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("kind", ["poiseuille", "peristalsis", "dambreak"])
+def test_runs_of_several_steps_replay_the_single_steps(device, kind):
+    """run() launches several captured steps at a time once counts repeat (up to
+    16): every state along growing, shrinking and mixed counts, with eager steps,
+    array writes and parameter changes between them, equals the eager steps' """
+    if kind == "dambreak":
+        sc = S.dambreak3d(dx=0.4 / 7)
+        p, pos, vel = sc.params, sc.pos, np.zeros_like(sc.pos)
+    else:
+        p, pos, vel = scene(kind, 1000)
+    a, b = (ParamSystem(p, pos.shape[0]) for _ in range(2))
+    for s in (a, b):
+        for arr, x in zip(ARRAYS, (pos, vel, vel)):
+            s.setArray(arr, x)
+    for k, steps in enumerate([3, 3, 3, 10, 10, 3, 3, 0, 40, 40, 1, 1, 17, 17, 2, 10]):
+        a.run(steps)
+        b.run(steps, use_graph=False)
+        if k % 5 == 2:
+            a.update()
+            b.update()
+        if k == 6:
+            for s in (a, b):
+                s.setArray(L.ARRAY_VELOCITY, vel)
+        if k == 8:
+            q = a.params.copy()
+            q.gravity[0] = 1e-3
+            a.set_params(q)
+            b.set_params(q)
+        for x, y in zip(states(a), states(b)):
+            assert np.array_equal(x, y, equal_nan=True), (k, steps)
+        assert a.getElapsedTime() == b.getElapsedTime()
+
+
 def test_batch(device):
     inst = [scene(k, n) for k, n in (("poiseuille", 1000), ("peristalsis", 1100), ("poiseuille", 1500))]
     out = []
