@@ -85,6 +85,15 @@ __host__ __device__ inline bool row_masks_apply(const cmag_params& P) {
     return P.dim == 2 && P.system != CMAG_SYS_DAMBREAK && P.hash_order == CMAG_HASH_LINEAR &&
            2 * P.cellcount + 1 <= ROW_MASK_ROWS;
 }
+// Dam-break targets are shared between four lanes up to this many rows.
+// Two steps of a 3-D dam break by itself / of four at once on their own streams,
+// a lane to a target against four: 25,168 rows 395 / 104 us against 169 / 56,
+// 54,508: 412 / 115 against 260 / 95, 82,188: 399 / 126 against 261 / 120,
+// 117,260: 414 / 136 against 310 / 159 (four at once fill the chip either way,
+// and a shared target costs more work); 160,492: 466 / 161 against 389 / 223.
+// The stage launchers over a caller's arrays: 54,508 rows 214 against 137 us,
+// 82,188: 210 against 186, 117,260: 223 against 237.
+constexpr uint32_t SHARED_TARGETS = 3u << 15;
 // where a step's force pass integrates its targets (in place, at their particle
 // numbers); pos null: it only writes the accelerations
 struct StepArrays {
@@ -105,7 +114,7 @@ int launch_density_sub(const cmag_params& P, float* measures, const uint32_t* ke
                        uint32_t* masks = nullptr);
 int launch_force_sub(const cmag_params& P, float* acc, const float* posW, const float* velW,
                      const uint32_t* indexW, const uint32_t* keys, const uint32_t* cellFirst, const uint32_t* pre,
-                     uint32_t n, hipStream_t s, const uint32_t* masks = nullptr);
+                     uint32_t n, hipStream_t s, const uint32_t* masks = nullptr, const StepArrays& step = {});
 int launch_force(const cmag_params& P, float* acc, const float* measures, const float* sortedPos,
                  const float* sortedVel, const uint32_t* index, const uint32_t* cellStart,
                  const uint32_t* cellEnd, uint32_t n, hipStream_t s,

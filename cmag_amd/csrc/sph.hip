@@ -7,16 +7,6 @@
 
 namespace cmag {
 
-// Dam-break targets are shared between TARGET_LANES lanes up to this many rows.
-// Two steps of a 3-D dam break by itself / of four at once on their own streams,
-// a lane to a target against four: 25,168 rows 395 / 104 us against 169 / 56,
-// 54,508: 412 / 115 against 260 / 95, 82,188: 399 / 126 against 261 / 120,
-// 117,260: 414 / 136 against 310 / 159 (four at once fill the chip either way,
-// and a shared target costs more work); 160,492: 466 / 161 against 389 / 223.
-// The stage launchers over a caller's arrays: 54,508 rows 214 against 137 us,
-// 82,188: 210 against 186, 117,260: 223 against 237.
-constexpr uint32_t SHARED_TARGETS = 3u << 15;
-
 template <int SYS, int DIM, int HASH, typename Cells, int LANES = 1>
 __global__ __launch_bounds__(256) void density_kernel(const cmag_params P, float4* __restrict__ measures,
                                                        const float4* __restrict__ sortedPos, const Cells cells,
@@ -274,7 +264,7 @@ template <int DIM, int HASH, int CAP, int LANES>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CAP <= 8 && LANES == 1 ? 6 : 1, 8))) void force_sub_kernel(
     const cmag_params P, float4* __restrict__ acc, const float4* __restrict__ posW, const float4* __restrict__ velW,
     const uint32_t* __restrict__ indexW, const uint32_t* __restrict__ keys, const SubCells cells, uint32_t n,
-    const uint2* __restrict__ masks) {
+    const uint2* __restrict__ masks, const StepArrays step) {
     __shared__ uint32_t nbl[256 / 64][CAP][64];
     __shared__ LookupPlan lp;
     __shared__ LookupTables lt;
@@ -286,13 +276,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CAP <= 8 &&
     const LookupView v = lookup_view<DIM>(lp, lt, keys[i], key_masks<HASH>(P).x);
     force_body<CMAG_SYS_DAMBREAK, DIM, HASH, SubCells, CAP, LANES>(P, i, acc, nullptr, posW, velW, indexW, cells, n,
                                                                    nbl[threadIdx.x >> 6], &v, staged, masks, n,
-                                                                   nullptr, nullptr, {}, threadIdx.x % LANES);
+                                                                   nullptr, nullptr, step, threadIdx.x % LANES);
 }
 
 int launch_force_sub(const cmag_params& P, float* acc, const float* posW, const float* velW,
                      const uint32_t* indexW, const uint32_t* keys, const uint32_t* cellFirst, const uint32_t* pre,
-                     uint32_t n, hipStream_t s, const uint32_t* masks) {
+                     uint32_t n, hipStream_t s, const uint32_t* masks, const StepArrays& step) {
     if (n == 0) return CMAG_OK;
+    if (step.pos && n > SHARED_TARGETS)
+        return fail(CMAG_E_INVALID, "the sub-cell force pass integrates shared targets only");
     if (n >= (1u << NB_SHIFT_BITS)) return fail(CMAG_E_INVALID, "force passes take at most 2^27 particles");
     if (P.system != CMAG_SYS_DAMBREAK) return fail(CMAG_E_INVALID, "the sub-cell walk is DamBreak's");
     const SubCells cells{cellFirst, reinterpret_cast<const uint4*>(pre)};
@@ -301,7 +293,7 @@ int launch_force_sub(const cmag_params& P, float* acc, const float* posW, const 
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(div_up(n, 256 / LANES)), dim3(256), 0, s, P, reinterpret_cast<float4*>(acc),
                                reinterpret_cast<const float4*>(posW), reinterpret_cast<const float4*>(velW), indexW,
-                               keys, cells, n, reinterpret_cast<const uint2*>(masks));
+                               keys, cells, n, reinterpret_cast<const uint2*>(masks), step);
         };
         if (masks) go(force_sub_kernel<D, H, 8, LANES>);
         else go(force_sub_kernel<D, H, NB_CAP, LANES>);

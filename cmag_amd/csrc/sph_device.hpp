@@ -1520,8 +1520,11 @@ __device__ __forceinline__ void force_body(const cmag_params& P, uint32_t i, flo
     // holds them (4.1M particles in 256 channels: 810 -> 774 us a step; a
     // 17,500-particle channel: 28.4 -> 24.5 us).  The pass reads the sorted copies
     // only, so its targets' own rows may change under it.
-    if (!Cells::SUB && Cells::PADDED && step.pos)
-        integrate_row<SYS>(P, k, pi, vi.w, a, a, step.pos, step.vel, step.velLF, 0.0f, 0);
+    if (Cells::PADDED && (!Cells::SUB || LANES > 1) && step.pos) {
+        // packed rows hold -rho and the pressure term in the w of their copies
+        const float4 p = PACKED ? make_float4(pi.x, pi.y, pi.z, CMAG_DB_FLUID) : pi;
+        integrate_row<SYS>(P, k, p, PACKED ? step.velLF[k].w : vi.w, a, a, step.pos, step.vel, step.velLF, 0.0f, 0);
+    }
 }
 
 // ---- Peristalsis: pressure and viscous passes -------------------------------------

@@ -219,13 +219,14 @@ struct cmag_system {
     int enqueue_step() {
         CMAG_TRY(enqueue_front(true));
         CMAG_TRY(mark(CMAG_STAGE_FORCE));
-        // The channels' force pass integrates its targets; with stage timing on, the
-        // two stages run apart (the same operations, so the same results).  The
-        // sub-cell pass leaves them to a launch of their own: it waits for L1
-        // and its scattered stores cost what the launch does (1M dam break 0.691
-        // against 0.681 ms, 16M 7.39 against 7.42 ms).
+        // The channels' force pass integrates its targets, and the small dam
+        // breaks'; with stage timing on, the two stages run apart (the same
+        // operations, so the same results).  A large dam break leaves them to a
+        // launch of their own: its pass waits for L1, and the scattered stores
+        // cost what the launch does (1M rows 0.691 against 0.681 ms, 16M 7.39
+        // against 7.42 ms).
         StepArrays step;
-        if (!timing && !subwalk) {
+        if (!timing && (!subwalk || n <= SHARED_TARGETS)) {
             auto f4 = [](float* q) { return reinterpret_cast<float4*>(q); };
             step = StepArrays{f4(pos), f4(vel), f4(velLF), dState};
         }
@@ -234,7 +235,7 @@ struct cmag_system {
                                                cellStart, cellEnd, n, stream, cellFirst, pairs, rowMasks, step));
         } else if (subwalk) {
             CMAG_TRY(launch_force_sub(P, acc, posW, velW, indexW, hash, cellFirst, sort.pre, n, stream,
-                                      use_masks ? masks : nullptr));
+                                      use_masks ? masks : nullptr, step));
         } else {
             CMAG_TRY(launch_force(P, acc, measures, sortedPos, sortedVel, index, cellStart, cellEnd, n,
                                   stream, cellFirst, pairs, rowMasks, step));

@@ -1,5 +1,5 @@
-"""The channels' force pass integrates its targets; with stage timing on the two
-stages run as launches of their own.  The operations are the same, so the states
+"""The force pass of channels and small dam breaks integrates its targets; with
+stage timing on the two stages run as launches of their own.  The operations are the same, so the states
 are the same bit for bit."""
 import numpy as np
 import pytest
@@ -39,6 +39,25 @@ def test_system(device, kind, moving, n):
     for timing in (False, True):
         s = ParamSystem(p, pos.shape[0])
         for a, x in zip(ARRAYS, (pos, vel, vel)):
+            s.setArray(a, x)
+        s.enable_timing(timing)
+        for _ in range(3):
+            s.update()
+        out.append(states(s))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("cells", [3, 12])
+@pytest.mark.parametrize("order,xbits", [(L.HASH_LINEAR, 0), (L.HASH_MORTON, 3)])
+def test_small_dam_break(device, cells, order, xbits):
+    sc = S.dambreak3d(dx=0.4 / cells, hash_order=order, morton_xbits=xbits)
+    rng = np.random.default_rng(cells)
+    vel = rng.normal(scale=0.3, size=sc.pos.shape).astype(np.float32)  # w of every particle is carried along
+    out = []
+    for timing in (False, True):
+        s = ParamSystem(sc.params, sc.pos.shape[0])
+        for a, x in zip(ARRAYS, (sc.pos, vel, vel[::-1].copy())):
             s.setArray(a, x)
         s.enable_timing(timing)
         for _ in range(3):
