@@ -13,9 +13,9 @@
 //              330-343 for the moving walls), so the step needs no host input
 //   place,     every instance's particles into cell order: instance k's stay in
 //   reorder    [part0, part1), ordered as its own sort orders them
-//   density, force, integrate
-//              persistent kernels over a table of (instance, first particle)
-//              tiles; a workgroup runs one contiguous chunk of tiles and reads
+//   density, force (which integrates its targets; with stage timing on, a
+//              kernel of its own does): persistent kernels over a table of
+//              (instance, first particle) tiles; a workgroup runs one contiguous chunk of tiles and reads
 //              its instance's parameter block from device memory
 //
 // Every per-particle body is the one the single-system kernels run

@@ -253,7 +253,9 @@ int cmag_system_synchronize(cmag_system* s);
 /* stage timing (no reference counterpart): with timing on, update() records
  * HIP events between its stages on the object's stream; stage_times returns
  * the accumulated milliseconds and launch counts of each stage, in the order
- * hash, sort, reorder, density, force, integrate, and clears them. */
+ * hash, sort, reorder, density, force, integrate, and clears them.  Without
+ * timing the force pass of channels, batches and small dam breaks integrates
+ * its targets; with it the two stages are launches of their own (same results). */
 enum cmag_stage {
     CMAG_STAGE_HASH = 0, CMAG_STAGE_SORT = 1, CMAG_STAGE_REORDER = 2,
     CMAG_STAGE_DENSITY = 3, CMAG_STAGE_FORCE = 4, CMAG_STAGE_INTEGRATE = 5,
