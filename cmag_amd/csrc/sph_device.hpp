@@ -1254,14 +1254,19 @@ __device__ __forceinline__ void walk_row_masks(const cmag_params& P, uint32_t i,
                                                C&& cand, Q&& pairs) {
     const uint32_t* in = masks + i;
     int left = P.cellcount;  // rows until the target's own
+    // a grid of no more cells along y than the stencil reaches brings the
+    // target's own row back as other rows: then it is looked for in each (in
+    // every grid that cost a 200,003-particle channel 2 %: 62.4 -> 63.5 us)
+    const bool repeated = P.grid_size[1] <= (uint32_t)P.cellcount;
     walk_rows<2, HASH>(P, pi, gp, cells, [&](const Run& a, const Run& b, float py, float pz, bool whole) {
         const uint32_t total = a.len + b.len, off_b = b.s - a.len;
         uint32_t m = 0;
         if (whole) {
             m = *in;
             in += stride;
-            if (left-- == 0) {
-                const uint32_t da = i - a.s, t = da < a.len ? da : i - off_b;
+            if (left-- == 0 || repeated) {
+                const uint32_t da = i - a.s, db = i - b.s;
+                const uint32_t t = da < a.len ? da : db < b.len ? a.len + db : 32u;
                 m &= ~(t < 32u ? 1u << t : 0u);
             }
         }
