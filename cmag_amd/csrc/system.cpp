@@ -408,7 +408,9 @@ struct cmag_system {
     // adjoint of `steps` update()s from the current state, which is stepped
     // steps - 1 times on the way.  Each step's front leaves what the backward
     // half reads in a block of its own, so a step is made once: keeping the
-    // states instead took six copies a step and its front a second time
+    // states instead took six copies a step and its front a second time.  The
+    // last step's goes to the System's own arrays, which so belong together
+    // afterwards (hash, index, cell ranges, sorted rows and densities)
     int vjp_segment(uint32_t steps, float* gpos, float* gvel, float* gvelLF, double* gmu_acc, double* ggrav_acc) {
         if (P.system != CMAG_SYS_POISEUILLE)
             return fail(CMAG_E_INVALID, "vjp_segment: the adjoint covers the Poiseuille system");
@@ -419,12 +421,13 @@ struct cmag_system {
         auto part = [](size_t bytes) { return (bytes + 255) & ~(size_t)255; };
         const size_t rows = part(sizeof(float) * 4 * (size_t)n + 64), nums = part(sizeof(uint32_t) * ((size_t)n + 1));
         const size_t block = 3 * rows + nums + part(sizeof(uint32_t) * ((size_t)numCells + 1));
+        const size_t blocks = steps - 1;
         try {
-            kept.reserve(steps);
+            kept.reserve(blocks);
         } catch (...) {
             return fail(CMAG_E_INVALID, "vjp_segment: out of host memory");
         }
-        while (kept.size() < steps) {
+        while (kept.size() < blocks) {
             void* b = nullptr;
             CMAG_HIP_TRY(hipMalloc(&b, block));
             kept.push_back(b);
@@ -440,19 +443,17 @@ struct cmag_system {
         timing = false;
         const Kept own = current();
         int rc = CMAG_OK;
-        for (uint32_t t = 0; t < steps && rc == CMAG_OK; ++t) {
+        for (uint32_t t = 0; t + 1 < steps && rc == CMAG_OK; ++t) {
             use(slot(t));
-            if (t + 1 < steps) {
-                rc = enqueue_step();
-                if (rc == CMAG_OK) advance_clock();
-            } else {
-                rc = enqueue_front(false);
-            }
+            rc = enqueue_step();
+            if (rc == CMAG_OK) advance_clock();
         }
         use(own);
+        if (rc == CMAG_OK) rc = enqueue_front(false);
         timing = was_timing;
         CMAG_TRY(rc);
-        for (uint32_t t = steps; t-- > 0;) CMAG_TRY(enqueue_vjp(slot(t), gpos, gvel, gvelLF, gmu_acc, ggrav_acc));
+        CMAG_TRY(enqueue_vjp(own, gpos, gvel, gvelLF, gmu_acc, ggrav_acc));
+        for (uint32_t t = steps - 1; t-- > 0;) CMAG_TRY(enqueue_vjp(slot(t), gpos, gvel, gvelLF, gmu_acc, ggrav_acc));
         return CMAG_OK;
     }
 

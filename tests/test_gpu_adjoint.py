@@ -280,3 +280,42 @@ def test_vjp_does_not_depend_on_the_cell_order(device, xbits):
     for x, y in zip((a[0], a[1], a[2], a[4]), (b[0], b[1], b[2], b[4])):
         assert normwise(x[:, :2].astype(np.float64), y[:, :2].astype(np.float64)) <= 3e-6
     assert abs(a[3].sum() - b[3].sum()) <= 3e-6 * np.abs(a[3]).sum()
+
+
+@pytest.mark.parametrize("steps", [1, 2, 5])
+def test_a_segment_leaves_one_consistent_state(device, steps):
+    """after a segment the System's arrays are those of its last step's front:
+    hash, index, cell ranges, sorted rows and densities belong to the same
+    positions, as after steps - 1 updates and the adjoint of one more"""
+    import torch
+
+    from cmag_amd.systems import ParamSystem
+    sc = S.channel_poiseuille(2000, nu=2e-2, seed=11)
+    n = sc.pos.shape[0]
+    pos, vel = sc.pos.copy(), np.zeros_like(sc.pos)
+    # fast enough for particles to change cells between the steps
+    v = 0.4 * float(sc.params.cell_size[0]) / float(sc.params.delta_time)
+    vel[:sc.num_fluid, 0] = v * np.random.default_rng(2).uniform(0.5, 1.0, sc.num_fluid)
+    floats = (L.ARRAY_POSITION, L.ARRAY_VELOCITY, L.ARRAY_VELOCITYLEAPFROG, L.ARRAY_SORTEDPOS, L.ARRAY_SORTEDVEL,
+              L.ARRAY_MEASURES, L.ARRAY_ACCELERATION)
+    uints = (L.ARRAY_HASH, L.ARRAY_INDEX, L.ARRAY_CELLSTART)
+    out = []
+    for segment in (True, False):
+        s = ParamSystem.from_state(sc.params, pos, vel)
+        g = [torch.zeros((n, 4), dtype=torch.float32, device="cuda") for _ in range(3)]
+        torch.cuda.synchronize()
+        if segment:
+            s.vjp_segment(steps, *[x.data_ptr() for x in g])
+        else:
+            for _ in range(steps - 1):
+                s.update()
+            s.vjp_step(*[x.data_ptr() for x in g])
+        s.synchronize()
+        out.append([s.getArray(a) for a in floats] + [s.getUintArray(a) for a in uints])
+    got = dict(zip(floats + uints, out[0]))
+    index, start, hash_ = (got[a] for a in (L.ARRAY_INDEX, L.ARRAY_CELLSTART, L.ARRAY_HASH))
+    assert np.array_equal(got[L.ARRAY_SORTEDPOS], got[L.ARRAY_POSITION][index])
+    cells, first = np.unique(hash_, return_index=True)
+    assert np.array_equal(start[cells], first)
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
