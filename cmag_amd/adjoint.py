@@ -73,6 +73,17 @@ class ChannelRollout:
         for a, t in zip(self._ARRAYS, state):
             self.system.copy_to_device(a, t.data_ptr())
 
+    def _vjp(self, steps: int, *ptrs: int) -> None:
+        """vjp_segment; the steps' blocks are allocated outside torch, which may
+        hold the room for them in its cache"""
+        try:
+            self.system.vjp_segment(steps, *ptrs)
+        except L.CmagError as e:
+            if e.code != L.CMAG_E_SIZE:
+                raise
+            torch.cuda.empty_cache()
+            self.system.vjp_segment(steps, *ptrs)
+
     def _params(self, mu: float, gravity) -> None:
         P = self.params.copy()
         P.mu = float(mu)
@@ -138,7 +149,7 @@ class _Rollout(torch.autograd.Function):
             t0 = c * ce
             t1 = min(t0 + ce, run.steps)
             run._put(ctx.cps[c])
-            s.vjp_segment(t1 - t0, gpos.data_ptr(), gvel.data_ptr(), glf.data_ptr(), gmu.data_ptr(), ggrav.data_ptr())
+            run._vjp(t1 - t0, *[x.data_ptr() for x in (gpos, gvel, glf, gmu, ggrav)])
         s.synchronize()
         dtype, device, shape = ctx.mu_like
         dmu = gmu.sum().to(dtype=dtype, device=device).reshape(shape)

@@ -10,6 +10,7 @@
 #include <cstring>
 #include <initializer_list>
 #include <new>
+#include <string>
 #include <vector>
 
 #include "common.hpp"
@@ -405,6 +406,31 @@ struct cmag_system {
                                   gpos, gvelLF, stream);
     }
 
+    // at least `count` blocks, or none more than before: refused before anything
+    // is enqueued, so that a caller who can free memory may call again
+    int keep_blocks(size_t count, size_t bytes) {
+        const size_t had = kept.size();
+        if (count <= had) return CMAG_OK;
+        size_t room = 0, total = 0;
+        CMAG_HIP_TRY(hipMemGetInfo(&room, &total));
+        bool got = room / bytes >= count - had;
+        try {
+            if (got) kept.reserve(count);
+        } catch (...) {
+            got = false;
+        }
+        while (got && kept.size() < count) {
+            void* b = nullptr;
+            got = hipMalloc(&b, bytes) == hipSuccess;
+            if (got) kept.push_back(b);
+        }
+        if (got) return CMAG_OK;
+        (void)hipGetLastError();
+        for (; kept.size() > had; kept.pop_back()) (void)hipFree(kept.back());
+        return fail(CMAG_E_SIZE, "vjp_segment: too little memory for " + std::to_string(count) + " steps of " +
+                                     std::to_string(bytes) + " bytes");
+    }
+
     // adjoint of `steps` update()s from the current state, which is stepped
     // steps - 1 times on the way.  Each step's front leaves what the backward
     // half reads in a block of its own, so a step is made once: keeping the
@@ -416,22 +442,12 @@ struct cmag_system {
             return fail(CMAG_E_INVALID, "vjp_segment: the adjoint covers the Poiseuille system");
         if (n && (!gpos || !gvel || !gvelLF)) return fail(CMAG_E_INVALID, "vjp_segment: null adjoint");
         if (steps == 0) return CMAG_OK;
-        CMAG_TRY(alloc_vjp());
         // parts of a block on 256-byte boundaries; the walks read up to two rows past the sorted positions
         auto part = [](size_t bytes) { return (bytes + 255) & ~(size_t)255; };
         const size_t rows = part(sizeof(float) * 4 * (size_t)n + 64), nums = part(sizeof(uint32_t) * ((size_t)n + 1));
         const size_t block = 3 * rows + nums + part(sizeof(uint32_t) * ((size_t)numCells + 1));
-        const size_t blocks = steps - 1;
-        try {
-            kept.reserve(blocks);
-        } catch (...) {
-            return fail(CMAG_E_INVALID, "vjp_segment: out of host memory");
-        }
-        while (kept.size() < blocks) {
-            void* b = nullptr;
-            CMAG_HIP_TRY(hipMalloc(&b, block));
-            kept.push_back(b);
-        }
+        CMAG_TRY(keep_blocks(steps - 1, block));
+        CMAG_TRY(alloc_vjp());
         auto slot = [&](uint32_t t) {
             char* b = static_cast<char*>(kept[t]);
             auto f = [&](size_t at) { return reinterpret_cast<float*>(b + at); };

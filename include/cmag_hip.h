@@ -352,8 +352,8 @@ int cmag_system_vjp_step(cmag_system* s, float* gpos, float* gvel, float* gvelLF
  * steps - 1 times on the way: the adjoints of the last step's outputs in, of
  * the current state out.  Keeps 52 bytes per particle and 4 per cell of device
  * memory for each step but the last of the longest segment asked for, until the
- * system is destroyed; every array ends as steps - 1 update()s and a vjp_step
- * leave it */
+ * system is destroyed (CMAG_E_SIZE, with nothing changed, where there is too
+ * little); every array ends as steps - 1 update()s and a vjp_step leave it */
 int cmag_system_vjp_segment(cmag_system* s, uint32_t steps, float* gpos, float* gvel, float* gvelLF, double* gmu_acc,
                             double* ggrav_acc);
 /* device-to-device copy of rows [start, start+count) between a System array

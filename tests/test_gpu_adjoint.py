@@ -319,3 +319,52 @@ def test_a_segment_leaves_one_consistent_state(device, steps):
     assert np.array_equal(start[cells], first)
     for x, y in zip(*out):
         assert np.array_equal(x, y)
+
+
+def test_backward_finds_room_in_torchs_cache(device):
+    """memory that torch keeps for its own later use does not refuse a backward
+    pass: the segments' blocks (about 4 GB here) come from it"""
+    import torch
+
+    from cmag_amd.adjoint import ChannelRollout
+    sc = S.channel_poiseuille(17000, nu=1e-2, seed=3)
+    steps = 3000
+    run = ChannelRollout(sc.params, sc.pos, sc.vel, steps=steps, checkpoint_every=steps)
+    mu = torch.tensor(float(sc.params.mu), dtype=torch.float64, requires_grad=True)
+    g = torch.tensor([float(sc.params.gravity[a]) for a in range(3)], dtype=torch.float64, requires_grad=True)
+    pos, vel = run(mu, g)
+    loss = vel[:, 0].to(torch.float64).mean()
+    torch.cuda.synchronize()
+    hold = torch.empty(torch.cuda.mem_get_info()[0] - (2 << 30), dtype=torch.uint8, device="cuda")
+    del hold
+    assert torch.cuda.mem_get_info()[0] < 3 << 30
+    loss.backward()
+    torch.cuda.empty_cache()
+    assert float(g.grad[0]) > 0.0
+
+
+def test_a_segment_too_long_is_refused_whole(device):
+    """more steps than the memory holds: refused with nothing taken or changed"""
+    import torch
+
+    from cmag_amd.systems import ParamSystem
+    sc = S.channel_poiseuille(2000, nu=2e-2, seed=11)
+    n = sc.pos.shape[0]
+    s = ParamSystem.from_state(sc.params, sc.pos, sc.vel)
+    g = [torch.ones((n, 4), dtype=torch.float32, device="cuda") for _ in range(3)]
+    ptrs = [x.data_ptr() for x in g]
+    s.vjp_segment(1, *ptrs)
+    s.synchronize()
+    state, adj = s.getArray(L.ARRAY_POSITION), [x.clone() for x in g]
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    with pytest.raises(L.CmagError) as e:
+        s.vjp_segment(2**32 - 1, *ptrs)
+    assert e.value.code == L.CMAG_E_SIZE
+    assert torch.cuda.mem_get_info()[0] == free
+    assert np.array_equal(s.getArray(L.ARRAY_POSITION), state)
+    assert all(torch.equal(x, y) for x, y in zip(g, adj))
+    s.update()
+    s.vjp_segment(3, *ptrs)
+    s.synchronize()
+    assert all(torch.isfinite(x).all() for x in g)
