@@ -15,6 +15,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "step_graphs.hpp"
 #include "step_state.hpp"
 
 using namespace cmag;
@@ -73,10 +74,7 @@ struct cmag_system {
     StepState* dState = nullptr;
     bool state_dirty = true;
 
-    // one captured step, and many_steps of them
-    hipGraphExec_t graph = nullptr, many = nullptr;
-    bool graph_valid = false;
-    uint32_t many_steps = 0, last_run = 0;
+    StepGraphs<hipGraphExec_t> graphs;
 
     // per-stage event timing: ev[k] recorded before stage k, ev[NUM] after the last
     bool timing = false;
@@ -280,19 +278,17 @@ struct cmag_system {
     }
 
     void invalidate_graph() {
-        if (graph) (void)hipGraphExecDestroy(graph);
-        if (many) (void)hipGraphExecDestroy(many);
-        graph = many = nullptr;
-        graph_valid = false;
-        many_steps = last_run = 0;
+        if (graphs.one) (void)hipGraphExecDestroy(graphs.one);
+        if (graphs.many) (void)hipGraphExecDestroy(graphs.many);
+        graphs = {};
     }
 
     int capture_steps(uint32_t steps, hipGraphExec_t* out) {
         if (stream == nullptr) return fail(CMAG_E_STATE, "graph capture needs a non-default stream");
         hipGraph_t g = nullptr;
+        CMAG_HIP_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
         const bool was_timing = timing;
         timing = false;  // no event nodes inside the graph
-        CMAG_HIP_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
         int rc = CMAG_OK;
         for (uint32_t k = 0; k < steps && rc == CMAG_OK; ++k) rc = enqueue_step();
         timing = was_timing;
@@ -311,35 +307,6 @@ struct cmag_system {
         return CMAG_OK;
     }
 
-    int build_graph() {
-        invalidate_graph();
-        CMAG_TRY(capture_steps(1, &graph));
-        graph_valid = true;
-        return CMAG_OK;
-    }
-
-    // A graph launch costs the host and the gap to the next one what two or
-    // three of a step's six or seven kernels do, so steps are launched several
-    // at a time once a second run() in a row asks for as many: the first pass
-    // captures one step only, and counts that change never capture again (a
-    // larger graph replaces a smaller one, so MANY_STEPS - 1 times at most).
-    static constexpr uint32_t MANY_STEPS = 16;
-    int grow_graph(uint32_t steps) {
-        const uint32_t want = steps < MANY_STEPS ? steps : MANY_STEPS;
-        const bool again = want == last_run;
-        last_run = want;
-        if (!again || want < 2 || want <= many_steps) return CMAG_OK;
-        hipGraphExec_t g = nullptr;
-        CMAG_TRY(capture_steps(want, &g));
-        if (many) {
-            (void)hipStreamSynchronize(stream);  // it may be running
-            (void)hipGraphExecDestroy(many);
-        }
-        many = g;
-        many_steps = want;
-        return CMAG_OK;
-    }
-
     int run(uint32_t steps, bool use_graph) {
         if (!use_graph) {
             for (uint32_t k = 0; k < steps; ++k) CMAG_TRY(update());
@@ -348,12 +315,22 @@ struct cmag_system {
         CMAG_TRY(collect());
         CMAG_TRY(upload_state());
         CMAG_TRY(sort.ready(stream));
-        if (!graph_valid) CMAG_TRY(build_graph());
-        CMAG_TRY(grow_graph(steps));
+        CMAG_TRY(graphs.prepare(
+            steps,
+            [&](uint32_t k, hipGraphExec_t* out) {
+                const int rc = capture_steps(k, out);
+                if (rc != CMAG_OK) (void)hipGetLastError();
+                return rc;
+            },
+            [&](hipGraphExec_t g) {
+                (void)hipStreamSynchronize(stream);  // it may be running
+                (void)hipGraphExecDestroy(g);
+            }));
         for (uint32_t k = 0; k < steps;) {
-            const bool several = many && steps - k >= many_steps;
-            CMAG_HIP_TRY(hipGraphLaunch(several ? many : graph, stream));
-            for (uint32_t t = several ? many_steps : 1; t > 0; --t, ++k) advance_clock();
+            uint32_t several = 0;
+            const hipGraphExec_t g = graphs.next(steps - k, several);
+            CMAG_HIP_TRY(hipGraphLaunch(g, stream));
+            for (; several > 0; --several, ++k) advance_clock();
         }
         return CMAG_OK;
     }
