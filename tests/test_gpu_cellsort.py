@@ -11,7 +11,7 @@ from cmag_amd.systems import ParamSystem
 
 pytestmark = pytest.mark.gpu
 
-# edges of a wave, a workgroup, and a tile of the offset scan
+# edges of a wave and of a workgroup (the offset scan's tiles are cells: below)
 COUNTS = [1, 2, 63, 64, 65, 255, 257, 4095, 4097, 30011]
 
 
@@ -120,4 +120,83 @@ def test_batch_sort(device):
         b.synchronize()
         check_sorted(np.concatenate(key), u32(L.ARRAY_HASH, n), u32(L.ARRAY_INDEX, n), u32(L.ARRAY_CELLSTART, cells),
                      u32(L.ARRAY_CELLEND, cells))
+    b.close()
+
+
+def on_grid(p, sizes, n, seed, walls):
+    """p on a grid of these sizes, and n particles over all of it: half anywhere,
+    half in blocks of eight cells, among them the grid's first and last cells"""
+    cs = float(p.cell_size[0])
+    p.hash_order = L.HASH_LINEAR
+    for a, g in enumerate(sizes):
+        p.grid_size[a] = g
+        p.cell_size[a] = cs
+        p.world_origin[a] = 0.0
+        p.world_size[a] = g * cs
+    S.finalize(p)
+    rng = np.random.default_rng(seed)
+    g = np.array(sizes)
+    cell = rng.integers(0, g, (n, 3))
+    near = rng.integers(0, max(n // 64, 1), n // 2)
+    corner = rng.integers(0, g, (max(n // 64, 1), 3))
+    corner[0], corner[-1] = 0, g - 1
+    cell[: n // 2] = np.minimum(corner[near] + rng.integers(0, 2, (n // 2, 3)), g - 1)
+    cell[0], cell[-1] = 0, g - 1
+    pos = np.zeros((n, 4), np.float32)
+    pos[:, :3] = cs * (cell + rng.uniform(0.2, 0.8, (n, 3)))
+    pos[:, 3] = np.where(rng.uniform(size=n) < 0.3, 1.0, 4.0) if walls else 0.0
+    return p, pos
+
+
+# grids of two to eight 16,384-cell tiles whose workgroups sum the counts in
+# front of them, of 4,096-cell tiles with totals (from 2^18 cells), and of more
+# tiles than a workgroup sums (2^26 cells: the totals are scanned)
+@pytest.mark.parametrize("sizes", [(64, 32, 16), (64, 32, 64), (128, 64, 32), (1024, 256, 256)])
+@pytest.mark.parametrize("walk", [True, False])
+def test_system_sort_on_large_grids(device, sizes, walk):
+    n = 5000
+    p, pos = on_grid(S.dambreak3d(dx=0.05).params, sizes, n, sizes[2], True)
+    s = ParamSystem.from_state(p, pos, None)
+    s.set_subcell_walk(walk)
+    check_system(s, p, 1)
+    dens = np.zeros(n)
+    dens[s.getUintArray(L.ARRAY_INDEX)] = s.getArray(L.ARRAY_MEASURES)[:, 0]
+    # again from other cells: those that emptied hold no counts
+    s.setArray(L.ARRAY_POSITION, pos[::-1].copy())
+    check_system(s, p, 1)
+    back = np.zeros(n)
+    back[s.getUintArray(L.ARRAY_INDEX)] = s.getArray(L.ARRAY_MEASURES)[:, 0]
+    # the same neighbours in another order: at most 100 positive terms
+    assert np.max(np.abs(back[::-1] - dens) / dens) <= 50 * 6e-8
+    s.close()
+
+
+# cell totals that are no multiple of 16 in each of the offset kernel's forms
+@pytest.mark.parametrize("large", [(64, 32, 1), (128, 128, 1), (512, 256, 1)])
+def test_batch_sort_ends_in_a_partial_tile(device, large):
+    inst = []
+    for k, (sizes, n) in enumerate((((2, 4, 1), 30), (large, 3000))):
+        p, pos = on_grid(S.channel_poiseuille(1024, nu=1e-2, seed=1).params, sizes, n, k, False)
+        inst.append((p, pos, np.zeros_like(pos)))
+    b = Batch(inst)
+    n, cells = b.num_particles, b.num_cells
+    assert cells % 16 == 8
+    import torch
+
+    class View:
+        def __init__(self, ptr, k):
+            self.owner = b
+            self.__cuda_array_interface__ = {"shape": (k,), "typestr": "<i4", "data": (ptr, False), "version": 2}
+
+    def u32(arr, k):
+        return torch.as_tensor(View(b.device_ptr(arr), k), device="cuda").cpu().numpy().view(np.uint32)
+
+    key, cell0 = [], 0
+    for p, pos, _ in inst:
+        key.append(keys_of(p, pos) + np.uint32(cell0))
+        cell0 += S.num_cells(p)
+    b.update()
+    b.synchronize()
+    check_sorted(np.concatenate(key), u32(L.ARRAY_HASH, n), u32(L.ARRAY_INDEX, n), u32(L.ARRAY_CELLSTART, cells),
+                 u32(L.ARRAY_CELLEND, cells))
     b.close()

@@ -28,8 +28,9 @@ def passes(p, pos, order, xbits, vel=None):
     return m[:, :2], out[1]
 
 
-# blocks of 256 targets over one, two and more rows of cells, in clouds of 1 to
-# 100 particles a cell, at the border of the grid and inside it
+# blocks of 64 targets (up to 98,304 rows four lanes share one) over one, two and
+# more rows of cells, in clouds of 1 to 100 particles a cell, at the border of the
+# grid and inside it
 @pytest.mark.parametrize("n,rows,cells_x", [(64, 1, 3), (255, 2, 2), (257, 2, 4), (600, 3, 30), (3000, 4, 16),
                                              (2500, 5, 5)])
 @pytest.mark.parametrize("border", [False, True])
@@ -74,3 +75,43 @@ def test_row_masks_equal_the_tested_rows(device, build, crowd, cellcount):
     want = passes(p, pos, L.HASH_MORTON, 0, sc.vel)
     for got, ref in zip(passes(p, pos, L.HASH_LINEAR, 0, sc.vel), want):
         assert np.array_equal(got, ref, equal_nan=True)
+
+
+# the same for dam breaks whose targets have a lane each (more than 98,304
+# rows): clouds of `fill` particles a cell on average, from none to twice that,
+# walls among them, so that blocks span one, two and more rows of cells, candidate
+# rows fit the density pass's LDS stage or not, and runs hold 64 candidates or
+# more and less; at the border of the grid and inside it, with masks and without
+@pytest.mark.parametrize("n,fill,cells_x", [(98305, 8, 40), (100003, 22, 12), (98560, 22, 60), (120011, 45, 30),
+                                            (98305, 110, 9)])
+@pytest.mark.parametrize("border", [False, True])
+def test_one_lane_targets_in_irregular_clouds(device, n, fill, cells_x, border):
+    sc = S.dambreak3d(dx=0.02)
+    p = sc.params
+    at = np.zeros(3) if border else np.array([1, 1, 1])
+    rng = np.random.default_rng(n + fill)
+    rows = -(-n // (fill * cells_x))
+    ny = max(int(round(rows ** 0.5)), -(-rows // (int(p.grid_size[2]) - 2)))
+    nz = -(-rows // ny)
+    span = np.array([cells_x, ny, nz])
+    assert (at + span <= [int(g) for g in p.grid_size]).all()
+    cells = np.stack(np.meshgrid(*[np.arange(k) for k in span], indexing="ij"), -1).reshape(-1, 3)
+    weight = rng.uniform(0.0, 2.0, len(cells))
+    pick = cells[rng.choice(len(cells), n, p=weight / weight.sum())]
+    pos = np.zeros((n, 4), np.float32)
+    cs = np.array([float(c) for c in p.cell_size])
+    pos[:, :3] = [float(o) for o in p.world_origin] + cs * (at + pick + rng.uniform(0.01, 0.99, (n, 3)))
+    pos[:, 3] = np.where(rng.uniform(size=n) < 0.1, 1.0, 4.0)
+    want = passes(p, pos, L.HASH_LINEAR, 0)
+    for xbits in (0, 2, 4):
+        for got, ref in zip(passes(p, pos, L.HASH_MORTON, xbits), want):
+            assert np.array_equal(got, ref, equal_nan=True)
+    for order, xbits in ((L.HASH_LINEAR, 0), (L.HASH_MORTON, 4)):
+        q = type(p).from_buffer_copy(p)
+        q.hash_order, q.morton_xbits = order, xbits
+        S.finalize(q)
+        s = ParamSystem.from_state(q, pos, None)
+        s.set_inrange_masks(False)
+        s.update()
+        assert np.array_equal(s.getArray(L.ARRAY_ACCELERATION), want[1], equal_nan=True)
+        s.close()
