@@ -127,15 +127,17 @@ def measured_traffic(workload_key: str, kernel: str) -> float | None:
         return None
 
 
-# VALU issue peak: one wave64 VALU instruction per CU per cycle (four SIMDs of
-# 16 lanes, four cycles per wave64 instruction), 256 CUs at 2.4 GHz
-VALU_PEAK_WAVE_INSTS = 256 * 2.4e9
+# SIMD cycles a second: 256 CUs of four SIMDs at 2.4 GHz.  A wave64 instruction
+# takes two of them as an FP32 add, multiply or fma of vector registers and
+# constants, eight as a transcendental, and two to four as anything else (taken as
+# four; an FP32 one with a scalar register takes four too)
+VALU_PEAK_CYCLES = 256 * 4 * 2.4e9
 
 
 def valu_roofline(workload_key: str, per_stage: dict) -> list | None:
-    """Issue-rate roofline of the neighbour passes: the VALU instructions per
-    launch from the committed counter summary of this workload over the live
-    launch time, against the issue peak"""
+    """Issue roofline of the neighbour passes: the SIMD cycles their VALU
+    instructions take, from the committed counter summary of this workload, over
+    the live launch time, against the cycles there are"""
     f = ROOT / "profiles" / "valu.json"
     if not f.exists():
         return None
@@ -148,10 +150,10 @@ def valu_roofline(workload_key: str, per_stage: dict) -> list | None:
         k = rec.get(stage)
         if not k or stage not in per_stage or not per_stage[stage]["avg_ms"]:
             continue
-        achieved = k["valu_insts_per_launch"] / (per_stage[stage]["avg_ms"] * 1e-3)
+        achieved = k["issue_cycles_per_wave"] * k["waves"] / (per_stage[stage]["avg_ms"] * 1e-3)
         out.append({"bound": "valu", "kernel": stage, "achieved": round(achieved / 1e9, 1),
-                    "peak": round(VALU_PEAK_WAVE_INSTS / 1e9, 1), "unit": "G wave64 VALU instr/s",
-                    "frac": round(achieved / VALU_PEAK_WAVE_INSTS, 3),
+                    "peak": round(VALU_PEAK_CYCLES / 1e9, 1), "unit": "G SIMD issue cycles/s",
+                    "frac": round(achieved / VALU_PEAK_CYCLES, 3),
                     "valu_insts_per_wave": k["valu_insts_per_wave"],
                     "lane_utilization": k.get("valu_lane_utilization")})
     return out or None

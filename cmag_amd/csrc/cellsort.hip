@@ -24,7 +24,7 @@
 // costs 4 to 5 us whatever it does; a three-digit radix sort with the reorder
 // and the offset scan was 15 of them: a 200,000-particle channel's two steps
 // went from 136 to 90 us), memory above (16M dam break, 20.07M rows, 2^24 cells:
-// hash 166 us, offsets 90, place 95, reorder of both orders 587 us at 4.9 TB/s;
+// hash 192 us, offsets 17 + 53, place 91, reorder of both orders 588 us, 2.6 GB;
 // radix sort, reorder, offset scan and the separate walk-order copy 1,320 us).
 // Counts per tile by atomics in the hash kernel instead of their own launch
 // met on too few addresses: hash 460 us at 16M, 793 us at 1.6M.  The radix sort
@@ -42,8 +42,13 @@ namespace cmag {
 constexpr int OFF_ITEMS = 16;  // cells per thread: four 16-byte words, one occupancy half-word
 static_assert(WALK_MAX_PARTICLES == 1u << ENTRY_BUCKET_SHIFT, "entries hold the particle number below the bucket");
 // A grid of up to OFF_SMALL_TILES tiles of 1024 threads reads the counts before
-// its tile itself (at most 28 16-byte loads a thread: 8.4 us at 2^17 cells, 4.6 us
-// at 2^12, against two launches of 4.7 us)
+// its tile itself (at most 28 16-byte loads a thread): one launch of 4.5 us at
+// 2^12 cells, 7.3 at 2^14, 9.0 at 2^16 and 10.8 at 2^17, against two of 4.5 us at
+// each.  It saves eager steps a launch of the host's (17,500-particle channel,
+// 2^14 cells, one update 23.5 against 26.9 us; 2,240 particles, 10 captured steps
+// 117 against 120 us) and costs captured steps of large grids time (17,000
+// particles, 10 steps by themselves: 2^13 cells 416 against 419 us, 2^14 401 / 382,
+// 2^16 420 / 386, 2^17 437 / 386; the 200-step gradient on 2^17 cells 23.7 / 22.0 ms)
 constexpr int OFF_NT_SMALL = 1024, OFF_NT = 256;
 constexpr uint32_t OFF_SMALL_TILES = 8;
 // tile totals a workgroup of a larger grid sums itself (at most 32 a thread,

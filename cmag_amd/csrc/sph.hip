@@ -256,10 +256,12 @@ int launch_density_sub(const cmag_params& P, float* measures, const uint32_t* ke
 // global walk).  CAP: neighbour queue depth; with the in-range masks only
 // walked rows and blocks without staged lookups queue neighbours, and a
 // shallower queue leaves more LDS to the CU.  What bounds it: the rows gathered
-// for the pair terms (the data-return path of L1 is busy 88 % of the time, the
-// vector units 78 %), 32 B a neighbour.  16M dam break: 3.54 ms with registers
-// held so that six waves share a SIMD, 3.75 ms with seven (a spill inside the
-// pair loop), 3.56 ms with five.
+// for the pair terms (the data-return path of L1 is busy 88 % of the time, vector
+// issue about half of it), 32 B a neighbour.  Z-order cells, 16M dam break: 3.54 ms
+// with registers held so that six waves share a SIMD, 3.75 ms with seven (a spill
+// inside the pair loop), 3.56 ms with five.  Linear cells, a whole step of the 1M
+// one (1.6M rows): 679 us with six, though that spills, 702 with five and 744
+// with four, neither of which does.
 template <int DIM, int HASH, int CAP, int LANES>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CAP <= 8 && LANES == 1 ? 6 : 1, 8))) void force_sub_kernel(
     const cmag_params P, float4* __restrict__ acc, const float4* __restrict__ posW, const float4* __restrict__ velW,

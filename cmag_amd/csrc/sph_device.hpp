@@ -796,9 +796,10 @@ __device__ __forceinline__ void walk_lookup(const cmag_params& P, const float4& 
 // than MASK_BITS is walked as before.
 // Layout: two words, bit t of the first for candidate t < 32 of the run, bit t
 // of the second for candidate 32 + t.  The scan takes the run's candidates in
-// pairs, the first 32 into one word, the rest into the other: a compare and an
-// add with carry a candidate.  (One 64-bit word shifted by two bits a pair took
-// four and a half, of which v_lshlrev_b64 and the selects most.)
+// pairs, the first 32 into one word, the rest into the other: a subtraction and
+// a funnel shift a candidate, and one more a pair (shift_in_less below).  (One
+// 64-bit word shifted by two bits a pair took four and a half instructions a
+// candidate, of which v_lshlrev_b64 and the selects most.)
 constexpr int MASK_BITS = 64;
 constexpr int MASK_ROWS = 9;
 
