@@ -388,9 +388,11 @@ struct cmag_system {
     int keep_blocks(size_t count, size_t bytes) {
         const size_t had = kept.size();
         if (count <= had) return CMAG_OK;
+        // what the card could never hold is not tried; the rest is, whatever the
+        // runtime reports as free
         size_t room = 0, total = 0;
         CMAG_HIP_TRY(hipMemGetInfo(&room, &total));
-        bool got = room / bytes >= count - had;
+        bool got = total / bytes >= count - had;
         try {
             if (got) kept.reserve(count);
         } catch (...) {
